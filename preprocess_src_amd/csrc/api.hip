@@ -644,7 +644,7 @@ lbmibm_status lbmibm_create(const lbmibm_params *p, const lbmibm_cells *cells, l
         ctx->nty = (ctx->ny + TILE_Y - 1) / TILE_Y;
         ctx->ntz = (ctx->nz + TILE_Z - 1) / TILE_Z;
         ctx->ntiles = ctx->ntx * ctx->nty * ctx->ntz;
-        ctx->nblk_bin = (nv + 255) / 256;
+        ctx->nblk_bin = (nv + BIN_WG - 1) / BIN_WG;
         if (ctx->nx > 30000 || ctx->ny > 29990 || ctx->nz > 30000) return fail(LBMIBM_ERR_ARG);  // short4 bins
         CK(dev_alloc(ctx, (void **)&ctx->node0, (size_t)nv * sizeof(short4)));
         CK(dev_alloc(ctx, &ctx->srec, (size_t)nv * 6 * szT));

@@ -69,24 +69,61 @@ __device__ __forceinline__ int home_tile(const BinGeom &g, double x, double y, d
     return xw / TILE_X + g.ntx * (yh / TILE_Y + g.nty * (zw / TILE_Z));
 }
 
-// Slot for a lane in counters[key], lanes with equal keys aggregated into one
-// atomic per wave.  All lanes of the wave must call it.
-__device__ __forceinline__ int wave_aggregated_add(int *counters, int key, bool active) {
-    const int lane = threadIdx.x & 63;
-    unsigned long long pending = __ballot(active);
-    int result = 0;
-    while (pending) {
-        const int leader = __ffsll((long long)pending) - 1;
-        const int lkey = __shfl(key, leader);
-        const unsigned long long grp = __ballot(active && key == lkey) & pending;
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&counters[lkey], __popcll(grp));
-        base = __shfl(base, leader);
-        if ((grp >> lane) & 1ull) result = base + __popcll(grp & ((1ull << lane) - 1ull));
-        pending &= ~grp;
+// Additions to per-tile counters in device memory, combined per work group: a
+// table in LDS holds the tiles that the group's vertices meet, and each tile
+// then costs one device atomic per work group.  Vertices are numbered along a
+// Morton curve, so 1024 of them meet 10 to 30 tiles, and the counters of
+// neighbouring tiles share cache lines: what these kernels wait for is the
+// line's atomics one after another, which one atomic per wave and tile made
+// about 10 times as many.  Any order and any number of tiles is accepted (the
+// table has twice as many entries as a group has vertices).  On 64 cells of
+// 2562 vertices, per launch before and after: k_vol_center 22.0 -> 7.4 us,
+// k_bin_scatter 22.2 -> 6.4 us, k_bin_count 23.0 -> 5.4 us.
+constexpr int BIN_WG = 1024;  // vertices per work group of the binning kernels
+struct TileTable {
+    static constexpr int SIZE = 2048;
+    static_assert(SIZE >= 2 * BIN_WG && SIZE >= 2 * VOL_CH, "an entry for every vertex of a group");
+    int key[SIZE], cnt[SIZE];
+    // all threads of the group, then a barrier
+    __device__ __forceinline__ void clear() {
+        for (int i = threadIdx.x; i < SIZE; i += blockDim.x) {
+            key[i] = -1;
+            cnt[i] = 0;
+        }
     }
-    return result;
-}
+    // Whole waves: counts each active lane's tile; the table entry in `slot`,
+    // the lane's rank among the group's vertices of that tile as the result.
+    __device__ __forceinline__ int add(int tile, bool active, int &slot) {
+        const int lane = threadIdx.x & 63;
+        unsigned long long pending = __ballot(active), mine = 0ull;
+        while (pending) {  // lanes of equal tiles, from registers alone
+            const int lead = __builtin_amdgcn_readlane(tile, __ffsll((long long)pending) - 1);
+            const bool in = active && tile == lead;
+            const unsigned long long grp = __ballot(in);
+            if (in) mine = grp;
+            pending &= ~grp;
+        }
+        const int leader = mine ? __ffsll((long long)mine) - 1 : lane;
+        int s = 0, r = 0;
+        if (active && lane == leader) {
+            s = (int)(((unsigned)tile * 2654435761u) >> 21);  // 11 bits
+            for (;;) {
+                const int was = atomicCAS(&key[s], -1, tile);
+                if (was == -1 || was == tile) break;
+                s = (s + 1) & (SIZE - 1);
+            }
+            r = atomicAdd(&cnt[s], __popcll(mine));
+        }
+        slot = __shfl(s, leader);
+        return __shfl(r, leader) + __popcll(mine & ((1ull << lane) - 1ull));
+    }
+    // After a barrier, all threads: adds the counts to the device counters;
+    // cnt then holds the group's first position in each tile (after a barrier).
+    __device__ __forceinline__ void flush(int *__restrict__ counters) {
+        for (int i = threadIdx.x; i < SIZE; i += blockDim.x)
+            if (cnt[i] > 0) cnt[i] = atomicAdd(&counters[key[i]], cnt[i]);
+    }
+};
 
 }  // namespace lbmibm
 

@@ -15,7 +15,7 @@
 //
 // Both directions work on lattice tiles of 16x8x8 nodes.  After each change
 // of the positions the vertices are binned by the tile of their first stencil
-// node (counting sort with wave-aggregated counters).
+// node (counting sort, counters combined per work group).
 //   - Spreading: one work group per tile takes the vertices of its own bin
 //     and of its 7 lower neighbours, keeps those whose stencil meets the tile
 //     (per-wave queue), and accumulates their contributions into the tile in
@@ -177,10 +177,13 @@ __device__ __forceinline__ int source_tiles(int t, int o, int n, int tile, bool 
 // ---- binning ---------------------------------------------------------------
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_bin_count(const double *__restrict__ xs, const T *__restrict__ cf, int nv,
-                                                   BinGeom bg, int *__restrict__ home,
-                                                   int *__restrict__ tile_count, float *__restrict__ blk_fmax) {
-    __shared__ float shm[4];
+__global__ __launch_bounds__(BIN_WG) void k_bin_count(const double *__restrict__ xs, const T *__restrict__ cf, int nv,
+                                                      BinGeom bg, int *__restrict__ home,
+                                                      int *__restrict__ tile_count, float *__restrict__ blk_fmax) {
+    __shared__ float shm[BIN_WG / 64];
+    __shared__ TileTable tab;
+    tab.clear();
+    __syncthreads();
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     const bool on = v < nv;
     int t = 0;
@@ -191,13 +194,18 @@ __global__ __launch_bounds__(256) void k_bin_count(const double *__restrict__ xs
         fm = fmaxf(fabsf((float)cf[v]), fmaxf(fabsf((float)cf[nv + v]), fabsf((float)cf[2 * (size_t)nv + v])));
         fm *= 1.0001f;  // margin for the float rounding of |f|
     }
-    (void)wave_aggregated_add(tile_count, t, on);
+    int slot;
+    (void)tab.add(t, on, slot);
     // per-block max |f| (one store per block; k_tile_scan reduces them)
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) fm = fmaxf(fm, __shfl_xor(fm, o));
     if ((threadIdx.x & 63) == 0) shm[threadIdx.x >> 6] = fm;
     __syncthreads();
-    if (threadIdx.x == 0) blk_fmax[blockIdx.x] = fmaxf(fmaxf(shm[0], shm[1]), fmaxf(shm[2], shm[3]));
+    tab.flush(tile_count);
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < BIN_WG / 64; k++) fm = fmaxf(fm, shm[k]);
+        blk_fmax[blockIdx.x] = fm;
+    }
 }
 
 // Heavy-first order of the tiles: a counting sort on a 256-level key of the
@@ -313,17 +321,24 @@ template <typename T> struct SpreadRec {
 };
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_bin_scatter(const double *__restrict__ xs, const T *__restrict__ cf,
+__global__ __launch_bounds__(BIN_WG) void k_bin_scatter(const double *__restrict__ xs, const T *__restrict__ cf,
                                                      const int *__restrict__ home, int nv, IbmGeom g,
                                                      const int *__restrict__ tile_off, int *__restrict__ tile_cur,
                                                      int *__restrict__ home_list, short4 *__restrict__ node0,
                                                      SpreadRec<T> *__restrict__ rec) {
+    __shared__ TileTable tab;
+    tab.clear();
+    __syncthreads();
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     const bool on = v < nv;
     const int t = on ? home[v] : 0;
-    const int r = wave_aggregated_add(tile_cur, t, on);
+    int slot;
+    const int r = tab.add(t, on, slot);
+    __syncthreads();
+    tab.flush(tile_cur);
+    __syncthreads();
     if (on) {
-        const int pos = tile_off[t] + r;
+        const int pos = tile_off[t] + tab.cnt[slot] + r;
         home_list[pos] = v;
         int x1, y1, z1;
         SpreadRec<T> sr;
@@ -1391,7 +1406,7 @@ lbmibm_status tile_offsets(lbmibm_ctx *ctx, hipStream_t stream, int nblk_fmax) {
 // The scatter of the binning: home list, first stencil nodes and spreading
 // records (fractions, current forces) in bin order.
 template <typename T> lbmibm_status bin_scatter(lbmibm_ctx *ctx, hipStream_t stream) {
-    hipLaunchKernelGGL(k_bin_scatter<T>, dim3(ctx->nblk_bin), dim3(256), 0, stream, (const double *)ctx->xs,
+    hipLaunchKernelGGL(k_bin_scatter<T>, dim3(ctx->nblk_bin), dim3(BIN_WG), 0, stream, (const double *)ctx->xs,
                        (const T *)spread_force(ctx), ctx->home, ctx->nv, geom_of(ctx), ctx->tile_off, ctx->tile_cur,
                        ctx->home_list, ctx->node0, (SpreadRec<T> *)ctx->srec);
     LBMIBM_LAUNCHED(ctx, "k_bin_scatter");
@@ -1407,7 +1422,7 @@ template <typename T> lbmibm_status bin_impl(lbmibm_ctx *ctx) {
     hipLaunchKernelGGL(k_zero_int, dim3((ctx->ntiles + 255) / 256), dim3(256), 0, stream, ctx->tile_count,
                        ctx->ntiles);
     LBMIBM_LAUNCHED(ctx, "k_zero_int");
-    hipLaunchKernelGGL(k_bin_count<T>, dim3(ctx->nblk_bin), dim3(256), 0, stream, (const double *)ctx->xs,
+    hipLaunchKernelGGL(k_bin_count<T>, dim3(ctx->nblk_bin), dim3(BIN_WG), 0, stream, (const double *)ctx->xs,
                        (const T *)spread_force(ctx), nv, bin_geom(ctx), ctx->home, ctx->tile_count, ctx->blk_fmax);
     LBMIBM_LAUNCHED(ctx, "k_bin_count");
     lbmibm_status s = tile_offsets(ctx, stream, ctx->nblk_bin);
@@ -1462,7 +1477,7 @@ template <typename T> lbmibm_status spread_impl(lbmibm_ctx *ctx) {
     } else {  // same positions, new forces: refresh the force part of the records
         hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, ctx->stream, (int *)ctx->absmax, 1);
         LBMIBM_LAUNCHED(ctx, "k_zero_int");
-        hipLaunchKernelGGL(k_bin_forces<T>, dim3(ctx->nblk_bin), dim3(256), 0, ctx->stream, ctx->home_list,
+        hipLaunchKernelGGL(k_bin_forces<T>, dim3((ctx->nv + 255) / 256), dim3(256), 0, ctx->stream, ctx->home_list,
                            (const T *)spread_force(ctx), ctx->nv, (SpreadRec<T> *)ctx->srec, ctx->absmax);
         LBMIBM_LAUNCHED(ctx, "k_bin_forces");
     }

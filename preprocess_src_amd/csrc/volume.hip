@@ -235,41 +235,43 @@ __global__ __launch_bounds__(NT) void k_volume(const int *__restrict__ cells, in
 // pass), and CapsulePeriodicAfter: each position wrapped back into the box.
 // With `home` the final positions are also counted into the spreading tiles
 // (home tile of each vertex, per-tile counts), as the binning would.
-__global__ __launch_bounds__(256) void k_vol_center(const int4 *__restrict__ chunks, double *__restrict__ xs, int nv,
+__global__ __launch_bounds__(VOL_CH) void k_vol_center(const int4 *__restrict__ chunks, double *__restrict__ xs, int nv,
                                                     const double *__restrict__ gx, const int *__restrict__ need,
                                                     double4 *__restrict__ part, VolArgs a, BinGeom bg,
                                                     int *__restrict__ home, int *__restrict__ tile_count) {
     __shared__ double sh[128];
+    __shared__ TileTable tab;
     WgReduce red{sh, 0};
+    if (home) tab.clear();
+    __syncthreads();
     const int4 ch = chunks[blockIdx.x];
     const bool unwrap = need[ch.x] == 0;
     const double g[3] = {gx[3 * ch.x], gx[3 * ch.x + 1], gx[3 * ch.x + 2]};
     const double len[3] = {a.lx, a.ly, a.lz};
     double s[3] = {0.0, 0.0, 0.0};
-    // a uniform trip count: the tile counters aggregate over whole waves
-    for (int base = 0; base < ch.z; base += 256) {
-        const int j = ch.y + base + (int)threadIdx.x;
-        const bool on = base + (int)threadIdx.x < ch.z;
-        double fin[3] = {0.0, 0.0, 0.0};
-        if (on) {
-            for (int d = 0; d < 3; d++) {
-                double *P = xs + d * (size_t)nv + j;
-                const double x0 = *P;
-                const bool per = d != 1 || a.py;
-                const double x = unwrap && per ? unwrap1(x0, g[d], len[d]) : x0;
-                s[d] += x;
-                const double w = per ? rewrap1(x, len[d]) : x;
-                if (w != x0) *P = w;
-                fin[d] = w;
-            }
-        }
-        if (home) {
-            const int t = on ? home_tile(bg, fin[0], fin[1], fin[2]) : 0;
-            if (on) home[j] = t;
-            (void)wave_aggregated_add(tile_count, t, on);
+    const int j = ch.y + (int)threadIdx.x;
+    const bool on = (int)threadIdx.x < ch.z;
+    double fin[3] = {0.0, 0.0, 0.0};
+    if (on) {
+        for (int d = 0; d < 3; d++) {
+            double *P = xs + d * (size_t)nv + j;
+            const double x0 = *P;
+            const bool per = d != 1 || a.py;
+            const double x = unwrap && per ? unwrap1(x0, g[d], len[d]) : x0;
+            s[d] = x;
+            const double w = per ? rewrap1(x, len[d]) : x;
+            if (w != x0) *P = w;
+            fin[d] = w;
         }
     }
-    red.sum<3>(s);
+    if (home) {
+        const int t = on ? home_tile(bg, fin[0], fin[1], fin[2]) : 0;
+        if (on) home[j] = t;
+        int slot;
+        (void)tab.add(t, on, slot);
+    }
+    red.sum<3>(s);  // its barrier also orders the table
+    if (home) tab.flush(tile_count);
     if (threadIdx.x == 0) part[blockIdx.x] = make_double4(s[0], s[1], s[2], 0.0);
 }
 
@@ -343,7 +345,7 @@ lbmibm_status run_impl(lbmibm_ctx *ctx, int mode, hipStream_t stream) {
         const BinGeom bg{ctx->nx, ctx->ny, ctx->nz, ctx->nxp, ctx->nyp, ctx->nzp, ctx->p.periodic_y == 0,
                          ctx->ntx, ctx->nty, ctx->p.dx};
         LBMIBM_KT(ctx, stream, "k_vol_center",
-                  hipLaunchKernelGGL(k_vol_center, dim3(ctx->vol_nvc), dim3(256), 0, stream, ctx->vol_vchunks,
+                  hipLaunchKernelGGL(k_vol_center, dim3(ctx->vol_nvc), dim3(VOL_CH), 0, stream, ctx->vol_vchunks,
                                      (double *)ctx->xs, ctx->nv, ctx->gx, ctx->vol_need, ctx->vol_vpart, a, bg,
                                      count ? ctx->home : nullptr, ctx->tile_count));
         LBMIBM_LAUNCHED(ctx, "k_vol_center");

@@ -1,0 +1,60 @@
+"""Kernel paths at the sizes where they can go wrong (tile and work-group
+edges, remainders, smallest and largest inputs), against the oracle or a plain
+FP64 evaluation."""
+import numpy as np
+import pytest
+
+from tests.pairs import gpu_of, oracle_of, rel
+
+pytestmark = pytest.mark.gpu
+
+
+def _scattered(lx, ly, lz, nc, level, seed):
+    """nc cells whose vertices lie anywhere in the box, in random order: every
+    work group of the binning meets most of the tiles."""
+    from preprocess_src_amd import mesh
+    c = np.zeros((nc, 3))
+    cells = mesh.assemble([level] * nc, c, np.repeat(np.eye(3)[None], nc, 0), 3.0)
+    rng = np.random.default_rng(seed)
+    n = cells["x"].size
+    pos = [rng.uniform(-0.5, 0.5, n) * (v - 1e-6) for v in (lx, ly, lz)]
+    return cells, pos
+
+
+def _spread_both(lx, ly, lz, prec, cells, pos, forces, **kw):
+    """Lattice force of the oracle and of the library for the given positions
+    and nodal forces (COMP nodes)."""
+    o = oracle_of(lx, ly, lz, cells=cells, **kw)
+    g = gpu_of(lx, ly, lz, prec, cells=cells, **kw)
+    for k, v in zip("xyz", pos):
+        o.cells[k][:] = v
+    g.set_cells_state(x=pos[0], y=pos[1], z=pos[2])
+    for k, v in zip(("cfx", "cfy", "cfz"), forces):
+        o.cells[k][:] = v
+    g.set_cells_state(fx=forces[0], fy=forces[1], fz=forces[2])
+    o.ibm_st1()
+    g.ibm_st1()
+    comp = o.bc == 0
+    F = [f[comp] for f in g.lattice_force()]
+    g.close()
+    return F, [f[comp] for f in (o.fx, o.fy, o.fz)]
+
+
+# FP64: sums of at most a few hundred terms, 1e-11 of max |F| as the other
+# spreading tests; FP32: the weights' FP32 rounding, 1e-5
+SPREAD_TOL = {"f64": 1e-11, "f32": 1e-5}
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("nc", [1, 6, 7, 13])  # 162, 972, 1134, 2106 vertices: the binning's work groups hold 1024
+def test_binning_of_vertices_in_random_order(nc, prec, form, monkeypatch):
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", str(form))
+    lx, ly, lz = 64, 40, 64
+    print(f"[binning] nc={nc} prec={prec} form={form}", flush=True)
+    cells, pos = _scattered(lx, ly, lz, nc, 2, seed=5 + nc)
+    rng = np.random.default_rng(3)
+    forces = [1e-3 * rng.standard_normal(pos[0].size) for _ in range(3)]
+    F, ref = _spread_both(lx, ly, lz, prec, cells, pos, forces)
+    for a, b in zip(F, ref):
+        assert rel(a, b) < SPREAD_TOL[prec]
