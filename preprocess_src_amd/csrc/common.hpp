@@ -36,7 +36,7 @@ struct DevStatus {
 // Lattice tiles of the immersed-boundary kernels.
 constexpr int VOL_SMALL = 3072;
 constexpr int VOL_CH = 1024;  // elements / vertices per volume-correction chunk
-constexpr int TILE_X = 16, TILE_Y = 8, TILE_Z = 8;
+constexpr int TILE_X = 8, TILE_Y = 8, TILE_Z = 8;
 constexpr int ASM_CH = 256;  // vertices per chunk of the fused membrane assembly (k_assemble)
 
 // Lattice geometry of the vertex binning: unpadded and padded sizes, walls
@@ -214,7 +214,10 @@ struct lbmibm_ctx {
     int bicg_var[3] = {0, 0, 0};  // shape variant of the on-chip classes, form of class 2 (autotuned)
     int interp_form = 0;          // 0: tiles staged in LDS, 1: one thread per vertex, rows from memory (autotuned)
     int spread_form = 0;          // 0: source bins per tile, 1: home boxes + gather (autotuned)
-    void *sbox = nullptr;         // [ntiles][3][SB_N] staging boxes of spread form 1
+    void *sbox = nullptr;         // [ntiles + sb_maxextra][3][SB_N] staging boxes of spread form 1
+    int *tile_ex = nullptr;       // [ntiles] first extra chunk of each tile (spread form 1)
+    int2 *sb_extra = nullptr;     // [sb_maxextra] tile and chunk of the extra work groups, (-1, 0) unused
+    int sb_maxextra = 0;
     int *sb_cand = nullptr;       // [(nx+ny+nz)*4] box entries per coordinate (spread form 1)
     int big_lds = 0;              // dynamic LDS of the class-2 forms that use LDS (the whole CU)
     int *onchip_cells = nullptr;  // cells of classes 0 and 1

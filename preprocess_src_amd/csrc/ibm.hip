@@ -13,7 +13,9 @@
 // Vertex positions and stencil selection are FP64 in every precision mode;
 // weights, lattice fields (u, F) and nodal forces use the arithmetic type T.
 //
-// Both directions work on lattice tiles of 16x8x8 nodes.  After each change
+// Both directions work on lattice tiles of 8x8x8 nodes (16x8x8 left a third of
+// the CUs idle on a few dozen cells, and its boxes let one or two work groups
+// share a CU where these let three).  After each change
 // of the positions the vertices are binned by the tile of their first stencil
 // node (counting sort, counters combined per work group).
 //   - Spreading: one work group per tile takes the vertices of its own bin
@@ -59,7 +61,7 @@ __device__ __forceinline__ int pmod(int i, int n) {
 // sin and cos of (pi/2) t for t in [0, 1).  FP32: Taylor series of both to
 // degree 13 / 12 in x = (pi/2) t (truncation below 1e-9 on [0, pi/2), so the
 // result is within a few ulp of the correctly rounded value), evaluated by
-// Horner in x^2 with no range reduction.  FP64: the library sincos.
+// Horner in x^2 with no range reduction.
 __device__ __forceinline__ void sincos_quarter(float t, float *s, float *c) {
     const float x = 1.57079632679489662f * t, x2 = x * x;
     float ps = -1.0f / 6227020800.0f;
@@ -78,7 +80,33 @@ __device__ __forceinline__ void sincos_quarter(float t, float *s, float *c) {
     pc = pc * x2 - 0.5f;
     *c = 1.0f + x2 * pc;
 }
-__device__ __forceinline__ void sincos_quarter(double t, double *s, double *c) { sincos(M_PI / 2 * t, s, c); }
+// FP64: the Taylor series of both to degree 17 / 16 of x = (pi/2) min(t, 1 - t)
+// in [0, pi/4] (1 - t is exact for t >= 1/2; the first terms left out are below
+// 1e-18), sine and cosine exchanged for t > 1/2.  No range reduction, and half
+// the registers of the library's sincos.
+__device__ __forceinline__ void sincos_quarter(double t, double *s, double *c) {
+    const bool upper = t > 0.5;
+    const double x = 1.57079632679489661923 * (upper ? 1.0 - t : t), x2 = x * x;
+    double ps = 1.0 / 355687428096000.0;  // 1/17!
+    ps = fma(ps, x2, -1.0 / 1307674368000.0);
+    ps = fma(ps, x2, 1.0 / 6227020800.0);
+    ps = fma(ps, x2, -1.0 / 39916800.0);
+    ps = fma(ps, x2, 1.0 / 362880.0);
+    ps = fma(ps, x2, -1.0 / 5040.0);
+    ps = fma(ps, x2, 1.0 / 120.0);
+    ps = fma(ps, x2, -1.0 / 6.0);
+    double pc = 1.0 / 20922789888000.0;  // 1/16!
+    pc = fma(pc, x2, -1.0 / 87178291200.0);
+    pc = fma(pc, x2, 1.0 / 479001600.0);
+    pc = fma(pc, x2, -1.0 / 3628800.0);
+    pc = fma(pc, x2, 1.0 / 40320.0);
+    pc = fma(pc, x2, -1.0 / 720.0);
+    pc = fma(pc, x2, 1.0 / 24.0);
+    pc = fma(pc, x2, -0.5);
+    const double sn = fma(x * x2, ps, x), cs = fma(x2, pc, 1.0);
+    *s = upper ? cs : sn;
+    *c = upper ? sn : cs;
+}
 
 // Weights 1 + cos(pi |x_node - xtr| / (2h)) of the 4 nodes from
 // floor(xtr/h)-1 (ibm.cu:103-121).  With t = frac(xtr/h) the distances are
@@ -239,43 +267,62 @@ __device__ void heavy_first_order(const int *load, int n, int *hist, int *order)
     __syncthreads();
 }
 
+// Vertices per work group of k_spread_box, and the work groups of a tile.
+constexpr int SB_CHUNK = 800;
+__host__ __device__ __forceinline__ int spread_chunks(int cnt) { return (cnt + SB_CHUNK - 1) / SB_CHUNK; }
+
+// Exclusive scans over the tiles, in one work group, 1024 tiles per round: the
+// bins' offsets, and the extra chunks of the tiles that k_spread_box shares
+// out (listed in `extra`, (-1, 0) behind the last); and the maximum of the
+// per-block force maxima.  Both scans ride in one 64-bit wave scan, one barrier a round.
 __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile_count, int *__restrict__ tile_off,
                                                     int *__restrict__ tile_cur, int ntiles,
                                                     const float *__restrict__ blk_fmax, int nblk,
-                                                    unsigned *__restrict__ absmax) {
-    // exclusive scan over tiles in one work group, 1024 entries per round,
-    // and the maximum of the per-block force maxima
-    __shared__ int sh[1024];
-    __shared__ float shm[1024];
-    __shared__ int carry;
+                                                    unsigned *__restrict__ absmax, int *__restrict__ tile_ex,
+                                                    int2 *__restrict__ extra, int maxextra) {
+    __shared__ unsigned long long wtot[2][16];
+    __shared__ float wmax[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float fm = 0.0f;
     for (int i = threadIdx.x; i < nblk; i += 1024) fm = fmaxf(fm, blk_fmax[i]);
-    shm[threadIdx.x] = fm;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-        if (threadIdx.x < o) shm[threadIdx.x] = fmaxf(shm[threadIdx.x], shm[threadIdx.x + o]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *absmax = __float_as_uint(shm[0]);
-    for (int base = 0; base < ntiles; base += 1024) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) fm = fmaxf(fm, __shfl_xor(fm, o));
+    if (lane == 0) wmax[wave] = fm;
+    unsigned long long carry = 0ull;  // vertices in the low half, extra chunks in the high half
+    int parity = 0;
+    for (int base = 0; base < ntiles; base += 1024, parity ^= 1) {
         const int i = base + threadIdx.x;
-        const int v = i < ntiles ? tile_count[i] : 0;
-        sh[threadIdx.x] = v;
+        const int cnt = i < ntiles ? tile_count[i] : 0, ex = max(spread_chunks(cnt) - 1, 0);
+        const unsigned long long own = (unsigned)cnt | ((unsigned long long)ex << 32);
+        unsigned long long incl = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long t = __shfl_up(incl, o);
+            if (lane >= o) incl += t;
+        }
+        if (lane == 63) wtot[parity][wave] = incl;
         __syncthreads();
-        for (int o = 1; o < 1024; o <<= 1) {
-            const int t = threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
-            __syncthreads();
-            sh[threadIdx.x] += t;
-            __syncthreads();
+        unsigned long long b = carry + incl - own;
+#pragma unroll
+        for (int w = 0; w < 16; w++) {
+            const unsigned long long t = wtot[parity][w];
+            if (w < wave) b += t;
+            carry += t;
         }
         if (i < ntiles) {
-            tile_off[i] = carry + sh[threadIdx.x] - v;
+            tile_off[i] = (int)(unsigned)b;
             tile_cur[i] = 0;
+            const int e0 = (int)(b >> 32);
+            tile_ex[i] = e0;
+            for (int c = 0; c < ex; c++)
+                if (e0 + c < maxextra) extra[e0 + c] = make_int2(i, c + 1);
         }
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += sh[1023];
-        __syncthreads();
+    }
+    for (int e = (int)(carry >> 32) + (int)threadIdx.x; e < maxextra; e += 1024) extra[e] = make_int2(-1, 0);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) fm = fmaxf(fm, wmax[w]);
+        *absmax = __float_as_uint(fm);
     }
 }
 
@@ -386,9 +433,14 @@ __global__ void k_zero_int(int *__restrict__ p, int n) {
     if (i < n) p[i] = 0;
 }
 
+// a[k] for a runtime k by selects (a runtime index would put a in scratch)
+template <typename T> __device__ __forceinline__ T sel4(const T (&a)[4], int k) {
+    return k == 0 ? a[0] : k == 1 ? a[1] : k == 2 ? a[2] : a[3];
+}
+
 // ---- spreading ---------------------------------------------------------------
 
-// LDS accumulator layout of a 16x8x8 tile with row strides 20 and 176: the
+// LDS accumulator layout of a tile, rows padded to strides 20 and 176: the
 // 64 (kx,ky,kz) offsets of one stencil fall on 32 distinct 8-byte bank slots.
 constexpr int ACC_SX = 20, ACC_SXY = 176, ACC_N = ACC_SXY * TILE_Z;
 
@@ -419,8 +471,18 @@ template <> struct FixedPoint<float> {
             atomicAdd(&acc[d * stride + li], (unsigned long long)__double_as_longlong(t));
         }
     }
+    // the fixed-point bits of v * scale, as add() forms them
+    __device__ __forceinline__ static unsigned long long fixed(double v, double scale) {
+        return (unsigned long long)__double_as_longlong(fma(v, scale, 6755399441055744.0));
+    }
     __device__ __forceinline__ static long long value(unsigned long long a) {
         return (long long)(a << 16) >> 16;  // sign-extend the low 48 bits
+    }
+    // value(a) * inv, inv a power of two: value(a) + bits(1.5 2^52) are the
+    // bits of value(a) + 1.5 2^52, and the subtraction is exact
+    __device__ __forceinline__ static double real(unsigned long long a, double inv) {
+        const double t = __longlong_as_double(value(a) + 0x4338000000000000ll);
+        return fma(t, inv, -6755399441055744.0 * inv);
     }
 };
 template <> struct FixedPoint<double> {
@@ -433,7 +495,11 @@ template <> struct FixedPoint<double> {
 #pragma unroll
         for (int d = 0; d < 3; d++) atomicAdd(&acc[d * stride + li], (unsigned long long)llrint(w * f[d] * scale));
     }
+    __device__ __forceinline__ static unsigned long long fixed(double v, double scale) {
+        return (unsigned long long)llrint(v * scale);
+    }
     __device__ __forceinline__ static long long value(unsigned long long a) { return (long long)a; }
+    __device__ __forceinline__ static double real(unsigned long long a, double inv) { return (double)value(a) * inv; }
 };
 
 template <typename T>
@@ -572,54 +638,185 @@ __global__ __launch_bounds__(256) void k_spread_tiles(const SpreadRec<T> *__rest
 }
 
 // Spreading, form 1.  One work group per tile takes its home vertices only
-// and adds each one's whole 4x4x4 stencil into an LDS box of the tile plus
-// the 3 nodes above it on each axis (its stencils cannot leave that box), in
-// the fixed point of form 0, with no per-node masks; the box is then written
-// to a staging array, and k_spread_gather sums for each lattice node the box
-// entries that map to it.  Form 0 visits a vertex once per tile its stencil
-// touches (2.2 tiles on average with 16x8x8 tiles), each visit walking the 64
-// nodes under masks.  Lane l of wave w takes column NW l + w of the bin read
-// as WG columns, so that the lanes of a wave hold vertices far apart.
+// and adds their whole 4x4x4 stencils into an LDS box of the tile plus the 3
+// nodes above it on each axis (its stencils cannot leave that box); the box is
+// then written to a staging array, and k_spread_gather sums for each lattice
+// node the box entries that map to it.
+//
+// Vertices whose stencils start at the same node ("a cell") add to the same
+// 64 nodes, F[(ky,kz), (kx,d)] = sum_v (wy_ky wz_kz)(v) (wx_kx f_d)(v): a 16 x 12
+// product over the cell's vertices, which the FP64 matrix instruction takes
+// four vertices at a time.  The work group sorts its vertices by cell in LDS
+// (within a cell by vertex id, so that the sums do not depend on the order in
+// which the binning placed them), a wave multiplies one cell after another,
+// and each cell's 192 sums then go into the box as 64-bit fixed point with
+// integer LDS atomics.  That rate of the atomics is what bounded the form that
+// issued them per vertex (about 12 cycles per wave and CU): a mesh of 2562
+// vertices on a radius of 4 has 13 vertices per cell, the uneven suspension of
+// 1024 cells 4.8.  Per launch, before and after: 64 cells of 2562 vertices
+// (FP32) 90 -> 31 us, that suspension 250 -> 194 us, 384 such cells in FP64
+// 144 -> 120 us; with 8x8x8 tiles, 16x8x8 before.  What bounds it now is the
+// latency of its phases (loads, scan, sort, products) at the three work groups
+// that the box's LDS admits per CU.
+// The weights are formed in T, their products and sums in FP64.
 constexpr int SB_X = TILE_X + 3, SB_Y = TILE_Y + 3, SB_Z = TILE_Z + 3, SB_N = SB_X * SB_Y * SB_Z;
 constexpr int SPREAD_BOX_WG = 512;
 constexpr int SB_MAXC = 4;  // box entries per lattice coordinate and axis (k_spread_gather)
+constexpr int SB_KEYS = TILE_X * SB_Y * TILE_Z;  // cells of a tile; y from -3 (below the wall in the first tile row)
+// A tile of more than SB_CHUNK vertices is shared out by its cells between
+// several work groups, each with a box of its own (the tile's own one and
+// extra ones, which k_spread_combine adds to it): 64 cells of radius 4 fill 159 of
+// 1024 tiles with up to 2490 vertices, and the launch would end with the fullest.
+// SPAN: sorted vertices per wave and batch; with these two work groups fit a
+// CU's LDS.
+constexpr int SB_VPT = 2, SB_CAP = SB_VPT * SPREAD_BOX_WG;
+template <typename T> constexpr int SB_SPAN = sizeof(T) == 4 ? 32 : 16;
+static_assert(SB_CAP > SB_CHUNK, "the sort takes a chunk and a spread about it");
+typedef double double_x4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
-__global__ __launch_bounds__(SPREAD_BOX_WG) void k_spread_box(const SpreadRec<T> *__restrict__ rec,
+__global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_spread_box(const SpreadRec<T> *__restrict__ rec,
                                                               const short4 *__restrict__ node0,
+                                                              const int *__restrict__ home_list,
                                                               const int *__restrict__ tile_count,
                                                               const int *__restrict__ tile_off, T *__restrict__ S,
-                                                              IbmGeom g, TileGeom tg,
-                                                              const int *__restrict__ order) {
+                                                              IbmGeom g, TileGeom tg, const int *__restrict__ order,
+                                                              const int2 *__restrict__ extra, int maxextra) {
+    constexpr int WG_ = SPREAD_BOX_WG, NW = WG_ / 64, SPAN = SB_SPAN<T>, BATCH = NW * SPAN;
+    constexpr int KPT = (SB_KEYS + WG_) / WG_;  // keys per thread of the scan, and the total
+    // REC values per sorted vertex: sin and cos of the x, y and z fractions, the
+    // force and a 0 (for the result columns that no component has); the record
+    // behind the last one is all 0: what a block's missing vertices read
+    constexpr int REC = 10;
+    union Work {
+        int id[SB_CAP + 4];  // the selected vertices, then vertex ids by unordered position
+        T b[REC * (BATCH + 1)];
+    };
     __shared__ unsigned long long acc[3 * SB_N];
-    __shared__ float wmax[SPREAD_BOX_WG / 64];
-    const int tile = order[blockIdx.x];
+    __shared__ Work wk;
+    __shared__ int start[SB_KEYS + 1];  // counts of the keys, then their first sorted positions
+    __shared__ unsigned short okey[SB_CAP];
+    __shared__ int wsum[NW], nsel;
+    __shared__ float wmax[NW];
+    // the extra chunks of full tiles first, then every tile's first chunk
+    int tile, chunk = 0, slot;
+    if ((int)blockIdx.x < maxextra) {
+        const int2 ex = extra[blockIdx.x];
+        if (ex.x < 0) return;  // not so many chunks
+        tile = ex.x;
+        chunk = ex.y;
+        slot = tg.ntiles + blockIdx.x;
+    } else {
+        tile = slot = order[blockIdx.x - maxextra];
+    }
     const int cnt = tile_count[tile], off = tile_off[tile];
     if (cnt == 0) return;  // whole work group leaves together; the gather skips empty tiles
+    const int nch = spread_chunks(cnt);
     const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
     const int ox = tx * TILE_X, oy = ty * TILE_Y, oz = tz * TILE_Z;
-    for (int k = threadIdx.x; k < 3 * SB_N; k += blockDim.x) acc[k] = 0ull;
-    constexpr int NW = SPREAD_BOX_WG / 64;
-    const int R = (cnt + SPREAD_BOX_WG - 1) / SPREAD_BOX_WG;
-    const int col = NW * (threadIdx.x & 63) + (threadIdx.x >> 6);
-    // a box node takes at most one term per home vertex, each at most
-    // |f|max / (8 dx^3) with |f|max over the tile's own vertices (a maximum,
-    // so independent of the order of the records): the power of two keeps
-    // the sums below 2^kBits
-    float fm = 0.0f;
-    for (int r = 0; r < R; r++) {
-        const int i = col * R + r;
-        if (i >= cnt) break;
-        const SpreadRec<T> sr = rec[off + i];
-        fm = fmaxf(fm, fmaxf(fabsf((float)sr.f[0]), fmaxf(fabsf((float)sr.f[1]), fabsf((float)sr.f[2]))));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // the cell of a vertex's first stencil node (x, z wrapped at binning; y
+    // raw: with walls it may lie below the lattice in the first tile row), -1
+    // when this tile is not a valid home or the cell is another chunk's
+    auto key_of = [&](short4 n0) {
+        int y1 = n0.y - 3;
+        if (!g.walls) wrap_index(y1, g.ny);
+        const int bx = n0.x - ox, by = y1 - oy + 3, bz = n0.z - oz;
+        if (bx < 0 || bx >= TILE_X || bz < 0 || bz >= TILE_Z || by < 0 || by >= SB_Y) return -1;
+        if (nch > 1 && (bx + 5 * by + 3 * bz) % nch != chunk) return -1;
+        return bx + TILE_X * (by + SB_Y * bz);
+    };
+    for (int k = tid; k < 3 * SB_N; k += WG_) acc[k] = 0ull;
+    for (int k = tid; k <= SB_KEYS; k += WG_) start[k] = 0;
+    if (tid == 0) nsel = 0;
+    __syncthreads();
+    int n = cnt;
+    if (nch > 1) {
+#pragma unroll 2
+        for (int i0 = 0; i0 < cnt; i0 += WG_) {  // whole waves: one counter update per wave
+            const int i = i0 + tid;
+            const bool take = i < cnt && key_of(node0[off + min(i, cnt - 1)]) >= 0;
+            const unsigned long long m = __ballot(take);
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&nsel, __popcll(m));
+            at = __builtin_amdgcn_readfirstlane(at) + __popcll(m & ((1ull << lane) - 1ull));
+            if (take && at < SB_CAP) wk.id[at] = i;
+        }
+        __syncthreads();
+        n = nsel;
     }
+    const bool sorted = n <= SB_CAP;
+    // this thread's vertices, all loads first
+    int key[SB_VPT], id[SB_VPT], r[SB_VPT];
+    SpreadRec<T> sr[SB_VPT];
+    float fm = 0.0f;
+    if (sorted) {
+        int i[SB_VPT];
+        short4 n0[SB_VPT];
+#pragma unroll
+        for (int j = 0; j < SB_VPT; j++) {
+            const int at = tid + j * WG_;
+            i[j] = off + (at < n ? (nch > 1 ? wk.id[at] : at) : 0);
+        }
+#pragma unroll
+        for (int j = 0; j < SB_VPT; j++) {
+            key[j] = -1;
+            if (tid + j * WG_ < n) {
+                n0[j] = node0[i[j]];
+                id[j] = home_list[i[j]];
+                sr[j] = rec[i[j]];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < SB_VPT; j++)
+            if (tid + j * WG_ < n) {
+                key[j] = key_of(n0[j]);
+                r[j] = key[j] >= 0 ? atomicAdd(&start[key[j]], 1) : 0;
+                fm = fmaxf(fm, fmaxf(fabsf((float)sr[j].f[0]), fmaxf(fabsf((float)sr[j].f[1]), fabsf((float)sr[j].f[2]))));
+            }
+    } else {
+        for (int i = tid; i < cnt; i += WG_) {
+            const SpreadRec<T> s = rec[off + i];
+            fm = fmaxf(fm, fmaxf(fabsf((float)s.f[0]), fmaxf(fabsf((float)s.f[1]), fabsf((float)s.f[2]))));
+        }
+    }
+    // a box node takes at most one term per vertex, each at most |f|max /
+    // (8 dx^3) with |f|max over the chunk's own vertices (a maximum, so
+    // independent of the order of the records): the power of two keeps the
+    // sums below 2^kBits
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) fm = fmaxf(fm, __shfl_xor(fm, o));
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = fm;
+    if (lane == 0) wmax[wave] = fm;
     __syncthreads();
-    fm = wmax[0];
+    // exclusive scan of the key counts, KPT consecutive keys per thread
+    {
+        int own[KPT], before = 0;
 #pragma unroll
-    for (int w = 1; w < NW; w++) fm = fmaxf(fm, wmax[w]);
+        for (int k = 0; k < KPT; k++) {
+            own[k] = KPT * tid + k < SB_KEYS ? start[KPT * tid + k] : 0;
+            before += own[k];
+        }
+        int incl = before;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(incl, o);
+            if (lane >= o) incl += t;
+        }
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        int base = incl - before;
+        fm = wmax[0];
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            if (w < wave) base += wsum[w];
+            fm = fmaxf(fm, wmax[w]);
+        }
+#pragma unroll
+        for (int k = 0; k < KPT; k++) {
+            if (KPT * tid + k <= SB_KEYS) start[KPT * tid + k] = base;
+            base += own[k];
+        }
+    }
     // the float rounding of a double |f| may round down
     const double fmax = (double)fm * (1.0 + 0x1p-20);
     double scale = 1.0;
@@ -627,43 +824,181 @@ __global__ __launch_bounds__(SPREAD_BOX_WG) void k_spread_box(const SpreadRec<T>
         const double bound = (double)cnt * fmax / (8.0 * g.dx * g.dx * g.dx);
         scale = ldexp(1.0, FixedPoint<T>::kBits - 1 - ilogb(bound));
     }
-    const T w64 = (T)(1.0 / (64.0 * g.dx * g.dx * g.dx));
-    for (int r = 0; r < R; r++) {
-        const int i = col * R + r;
-        if (i >= cnt) break;
-        const short4 n0 = node0[off + i];
-        const SpreadRec<T> sr = rec[off + i];
-        // box coordinates of the first stencil node (x, z wrapped at binning;
-        // y raw: with walls it may lie below the lattice in the first tile row)
-        const int bx = n0.x - ox, bz = n0.z - oz;
-        int y1 = n0.y - 3;
-        if (!g.walls) wrap_index(y1, g.ny);
-        const int by = y1 - oy;
-        if (bx < 0 || bx >= TILE_X || bz < 0 || bz >= TILE_Z || by < -3 || by >= TILE_Y) continue;  // not a valid home
-        T wx[4], wy[4], wz[4];
-        stencil_weights<T>(sr.t[0], wx);
-        stencil_weights<T>(sr.t[1], wy);
-        stencil_weights<T>(sr.t[2], wz);
-        const FixedPoint<T> fp(sr.f[0], sr.f[1], sr.f[2], scale);
+    const double w64 = scale / (64.0 * g.dx * g.dx * g.dx);
+    __syncthreads();
+    if (sorted) {
+        // unordered positions, then ordered by vertex id within each cell
 #pragma unroll
-        for (int kz = 0; kz < 4; kz++) {
+        for (int j = 0; j < SB_VPT; j++)
+            if (key[j] >= 0) wk.id[start[key[j]] + r[j]] = id[j];
+        __syncthreads();
 #pragma unroll
-            for (int ky = 0; ky < 4; ky++) {
-                if (by + ky < 0) continue;  // below the wall
-                const T wyz = wy[ky] * wz[kz] * w64;
-                const int row = bx + SB_X * ((by + ky) + SB_Y * (bz + kz));
+        for (int j = 0; j < SB_VPT; j++) {
+            if (key[j] < 0) continue;
+            const int a = start[key[j]], b = start[key[j] + 1];
+            int at = a;
+            for (int t = a; t < b; t += 4) {  // four reads at a time
+                const int i0 = wk.id[t], i1 = wk.id[t + 1], i2 = wk.id[t + 2], i3 = wk.id[t + 3];
+                at += i0 < id[j];
+                at += t + 1 < b && i1 < id[j];
+                at += t + 2 < b && i2 < id[j];
+                at += t + 3 < b && i3 < id[j];
+            }
+            r[j] = at;
+            okey[at] = (unsigned short)key[j];
+        }
+        n = start[SB_KEYS];
+        // operand lane j = lane & 15 of vertex lane >> 4: wy_(j&3) wz_(j>>2) and
+        // wx_(j&3) f_(j>>2); result lane: kx = lane & 3, d = (lane >> 2) & 3,
+        // ky = lane >> 4, register i: kz = i
+        const int jx = lane & 3, jz = (lane >> 2) & 3;
+        const T sgx = jx == 0 || jx == 3 ? T(-1) : T(1), sgz = jz == 0 || jz == 3 ? T(-1) : T(1);
+        const int vrec = REC * (lane >> 4);
+        unsigned long long *const out = acc + jz * SB_N + jx + SB_X * ((lane >> 4) - 3);
+        const bool edge = g.walls && ty == 0;
+        __syncthreads();
+        // batches of equal size, spans of equal size per wave
+        const int nb = (n + BATCH - 1) / BATCH, span = nb ? ((n + nb - 1) / nb + NW - 1) / NW : 0;
+        for (int s0 = 0; s0 < n; s0 += NW * span) {
 #pragma unroll
-                for (int kx = 0; kx < 4; kx++) fp.add(acc, row + kx, wx[kx] * wyz, SB_N);
+            for (int j = 0; j < SB_VPT; j++) {
+                if (key[j] < 0 || r[j] < s0 || r[j] >= s0 + NW * span) continue;
+                T *o = wk.b + REC * (r[j] - s0);
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    T sn, cs;
+                    sincos_quarter(sr[j].t[d], &sn, &cs);
+                    o[2 * d] = sn;
+                    o[2 * d + 1] = cs;
+                    o[6 + d] = sr[j].f[d];
+                }
+                o[9] = T(0);
+            }
+            if (tid < REC) wk.b[REC * NW * span + tid] = T(0);
+            __syncthreads();
+            const int sA = s0 + wave * span;
+            const int m = __builtin_amdgcn_readfirstlane(min(span, n - sA));
+            if (m > 0) {
+                // the span's blocks of up to four vertices of one cell, listed
+                // one per lane: first slot, end of the cell's slots, key
+                const int kk = lane < m ? (int)okey[sA + lane] : -1;
+                const int prev = __shfl_up(kk, 1);
+                const unsigned long long starts = __ballot(lane < m && (lane == 0 || kk != prev));
+                const unsigned long long upto = (2ull << lane) - 1ull, later = starts & ~upto;
+                const int first = 63 - __clzll((long long)(starts & upto));  // slot 0 is a start
+                const int last = later ? __ffsll((long long)later) - 1 : m;
+                const bool blk = lane < m && ((lane - first) & 3) == 0;
+                const unsigned long long blocks = __ballot(blk);
+                const int nblk = __popcll(blocks);
+                const unsigned long long below = blk ? blocks : ~blocks;
+                // the cell's place in the box: x + SB_X (y + 3) + SB_X SB_Y z, y from -3
+                const int box = kk % TILE_X + SB_X * (kk / TILE_X % SB_Y + SB_Y * (kk / (TILE_X * SB_Y)));
+                // every lane takes part, those without a block behind the list
+                const int list = __builtin_amdgcn_ds_permute(
+                    4 * ((blk ? 0 : nblk) + __popcll(below & (upto >> 1))), lane | (last << 6) | (box << 12));
+                auto operands = [&](int d, double &A, double &B) {
+                    const int p = d & 63, e = (d >> 6) & 63;
+                    const int at = (lane >> 4) < e - p ? REC * (wave * span + p) + vrec : REC * NW * span;
+                    const T *qx = wk.b + at + (jx & 1), *qz = wk.b + at + 4 + (jz & 1);
+                    const T wx = fma(sgx, qx[0], T(1)), wy = fma(sgx, qx[2], T(1)), wz = fma(sgz, qz[0], T(1));
+                    A = (double)wy * (double)wz;
+                    B = (double)wx * (double)wk.b[at + 6 + jz];
+                };
+                // a cell's sums into the box: result column d = 3 is none
+                auto flush = [&](int d, const double_x4 &c) {
+                    const int at = d >> 12;
+                    // below the wall only in the first tile row (the box has no such rows)
+                    const bool low = edge && at % (SB_X * SB_Y) / SB_X + (lane >> 4) < 3;
+                    unsigned long long *o = out + at;
+                    if (jz < 3 && !low) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) atomicAdd(o + i * SB_X * SB_Y, FixedPoint<T>::fixed(c[i], w64));
+                    }
+                };
+                // two halves of the list at once: their chains of loads,
+                // product and addition do not wait for each other
+                const int h = (nblk + 1) >> 1;
+                const double_x4 zero = {0.0, 0.0, 0.0, 0.0};
+                double_x4 c0 = zero, c1 = zero;
+                double A0, B0, A1, B1;
+                int d0 = __builtin_amdgcn_readlane(list, 0), d1 = __builtin_amdgcn_readlane(list, min(h, nblk - 1));
+                operands(d0, A0, B0);
+                operands(d1, A1, B1);
+                bool new0 = true, new1 = true;
+                for (int i = 0; i < h; i++) {
+                    if (new0) c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(A0, B0, zero, 0, 0, 0);
+                    else c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(A0, B0, c0, 0, 0, 0);
+                    if (new1) c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(A1, B1, zero, 0, 0, 0);
+                    else c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(A1, B1, c1, 0, 0, 0);
+                    const int e0 = d0, e1 = d1;
+                    if (i + 1 < h) {  // the next blocks' operands while these are multiplied
+                        d0 = __builtin_amdgcn_readlane(list, i + 1);
+                        d1 = __builtin_amdgcn_readlane(list, min(h + i + 1, nblk - 1));
+                        operands(d0, A0, B0);
+                        operands(d1, A1, B1);
+                    }
+                    new0 = i + 1 == h || (e0 & 63) + 4 >= ((e0 >> 6) & 63);
+                    new1 = h + i + 1 >= nblk || (e1 & 63) + 4 >= ((e1 >> 6) & 63);
+                    if (new0) flush(e0, c0);
+                    if (new1 && h + i < nblk) flush(e1, c1);
+                }
+            }
+            __syncthreads();
+        }
+    } else {
+        // more vertices than the sort holds (thousands in a single lattice
+        // cell): their terms one by one
+        const T w1 = (T)(1.0 / (64.0 * g.dx * g.dx * g.dx));
+        for (int i = tid; i < cnt; i += WG_) {
+            const int kc = key_of(node0[off + i]);
+            if (kc < 0) continue;
+            const SpreadRec<T> s = rec[off + i];
+            T wx[4], wy[4], wz[4];
+            stencil_weights<T>(s.t[0], wx);
+            stencil_weights<T>(s.t[1], wy);
+            stencil_weights<T>(s.t[2], wz);
+            const FixedPoint<T> fp(s.f[0], s.f[1], s.f[2], scale);
+            const int bx = kc % TILE_X, by = (kc / TILE_X) % SB_Y - 3, bz = kc / (TILE_X * SB_Y);
+#pragma unroll 1
+            for (int c = 0; c < 64; c++) {
+                const int kx = c & 3, ky = (c >> 2) & 3, kz = c >> 4;
+                if (by + ky < 0) continue;
+                fp.add(acc, bx + kx + SB_X * ((by + ky) + SB_Y * (bz + kz)),
+                       sel4(wx, kx) * (sel4(wy, ky) * sel4(wz, kz) * w1), SB_N);
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
     const double inv_scale = 1.0 / scale;
-    T *St = S + (size_t)tile * 3 * SB_N;
-    for (int k = threadIdx.x; k < SB_N; k += blockDim.x)
+    T *St = S + (size_t)slot * 3 * SB_N;
+    for (int k0 = tid; k0 < 3 * SB_N; k0 += 4 * WG_) {  // four reads, then four stores
+        unsigned long long a[4];
 #pragma unroll
-        for (int d = 0; d < 3; d++)
-            St[d * SB_N + k] = (T)((double)FixedPoint<T>::value(acc[d * SB_N + k]) * inv_scale);
+        for (int j = 0; j < 4; j++) a[j] = acc[min(k0 + j * WG_, 3 * SB_N - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k0 + j * WG_ < 3 * SB_N) St[k0 + j * WG_] = (T)FixedPoint<T>::real(a[j], inv_scale);
+    }
+}
+
+// Adds the extra boxes of each tile that was shared out to the tile's own box,
+// chunk by chunk: work group e takes the tile whose first extra chunk is e, the
+// others leave at once (5 us on 64 cells, 15 us on the 1024-cell suspension).
+// The gather adding them itself took 64 instead of 44 us on that suspension:
+// the loop over chunks keeps its loads from being issued together.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_spread_combine(T *__restrict__ S, const int2 *__restrict__ extra,
+                                                         const int *__restrict__ tile_count, int ntiles) {
+    const int2 ex = extra[blockIdx.x];
+    if (ex.x < 0 || ex.y != 1) return;
+    const int nx = spread_chunks(tile_count[ex.x]) - 1;
+    T *own = S + (size_t)ex.x * 3 * SB_N;
+    const T *more = S + (size_t)(ntiles + blockIdx.x) * 3 * SB_N;
+    for (int k = threadIdx.x; k < 3 * SB_N; k += 1024) {
+        T a = own[k];
+        for (int c = 0; c < nx; c++) a += more[(size_t)c * 3 * SB_N + k];
+        own[k] = a;
+    }
 }
 
 // Sums, per lattice node, the box entries of k_spread_box that map to it, in
@@ -1011,11 +1346,6 @@ __device__ __forceinline__ void stencil_d(double xtr, double h, int &first, W w[
 }
 
 // Stencil of a position as stencil3 (spacing dx) with weight derivatives.
-// a[k] for a runtime k by selects (a runtime index would put a in scratch)
-template <typename T> __device__ __forceinline__ T sel4(const T (&a)[4], int k) {
-    return k == 0 ? a[0] : k == 1 ? a[1] : k == 2 ? a[2] : a[3];
-}
-
 template <typename W> struct StencilD {
     int x1, y1, z1;
     W wx[4], wy[4], wz[4], dx[4], dy[4], dz[4];
@@ -1395,7 +1725,8 @@ lbmibm_status tile_offsets(lbmibm_ctx *ctx, hipStream_t stream, int nblk_fmax) {
     const IbmGeom g = geom_of(ctx);
     TileGeom tg{ctx->ntx, ctx->nty, ctx->ntz, ctx->ntiles};
     hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->tile_off, ctx->tile_cur,
-                       ctx->ntiles, ctx->blk_fmax, nblk_fmax, ctx->absmax);
+                       ctx->ntiles, ctx->blk_fmax, nblk_fmax, ctx->absmax, ctx->tile_ex, ctx->sb_extra,
+                       ctx->sb_maxextra);
     LBMIBM_LAUNCHED(ctx, "k_tile_scan");
     hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->ntiles, g, tg,
                        ctx->tile_cand, ctx->order_spread, ctx->order_interp, ctx->order_calls);
@@ -1440,10 +1771,17 @@ template <typename T> lbmibm_status spread_launch(lbmibm_ctx *ctx, int form) {
     const IbmGeom g = geom_of(ctx);
     if (form == 1) {
         LBMIBM_KT(ctx, ctx->stream, "k_spread_box",
-                  hipLaunchKernelGGL(k_spread_box<T>, dim3(ctx->ntiles), dim3(SPREAD_BOX_WG), 0, ctx->stream,
-                                     (const SpreadRec<T> *)ctx->srec, ctx->node0, ctx->tile_count, ctx->tile_off,
-                                     (T *)ctx->sbox, g, tg, ctx->order_interp));
+                  hipLaunchKernelGGL(k_spread_box<T>, dim3(ctx->sb_maxextra + ctx->ntiles), dim3(SPREAD_BOX_WG), 0,
+                                     ctx->stream,
+                                     (const SpreadRec<T> *)ctx->srec, ctx->node0, ctx->home_list, ctx->tile_count,
+                                     ctx->tile_off, (T *)ctx->sbox, g, tg, ctx->order_interp, ctx->sb_extra,
+                                     ctx->sb_maxextra));
         LBMIBM_LAUNCHED(ctx, "k_spread_box");
+        if (ctx->sb_maxextra > 0) {
+            hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra), dim3(1024), 0,
+                               ctx->stream, (T *)ctx->sbox, ctx->sb_extra, ctx->tile_count, ctx->ntiles);
+            LBMIBM_LAUNCHED(ctx, "k_spread_combine");
+        }
         LBMIBM_KT(ctx, ctx->stream, "k_spread_gather",
                   hipLaunchKernelGGL(k_spread_gather<T>, dim3((unsigned)xcd_grid((int)((ctx->N + 255) / 256))), dim3(256), 0,
                                      ctx->stream, (const T *)ctx->sbox, ctx->tile_count, ctx->sb_cand,
@@ -1617,6 +1955,11 @@ lbmibm_status ibm_interp_adjoint(lbmibm_ctx *ctx) {
 }
 
 lbmibm_status ibm_setup(lbmibm_ctx *ctx) {
+    // extra chunks: at most nv / SB_CHUNK over all tiles
+    ctx->sb_maxextra = ctx->nv / SB_CHUNK;
+    lbmibm_status s = dev_alloc(ctx, (void **)&ctx->tile_ex, (size_t)ctx->ntiles * sizeof(int));
+    if (s == LBMIBM_OK) s = dev_alloc(ctx, (void **)&ctx->sb_extra, (size_t)ctx->sb_maxextra * sizeof(int2));
+    if (s != LBMIBM_OK) return s;
     const int lds64 = (int)(3 * (size_t)RN * sizeof(double));
     const int lds32 = (int)(3 * (size_t)RN * sizeof(float));
     LBMIBM_HIP(ctx, hipFuncSetAttribute((const void *)k_interp_tiles<double>,
@@ -1687,7 +2030,7 @@ static lbmibm_status spread_box_setup(lbmibm_ctx *ctx, bool *ok) {
         LBMIBM_HIP(ctx, hipMemcpy(ctx->sb_cand, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     if (!ctx->sbox) {
-        lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)ctx->ntiles * 3 * SB_N * ctx->szT);
+        lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)(ctx->ntiles + ctx->sb_maxextra) * 3 * SB_N * ctx->szT);
         if (s != LBMIBM_OK) return s;
     }
     *ok = true;

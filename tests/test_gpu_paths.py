@@ -58,3 +58,61 @@ def test_binning_of_vertices_in_random_order(nc, prec, form, monkeypatch):
     F, ref = _spread_both(lx, ly, lz, prec, cells, pos, forces)
     for a, b in zip(F, ref):
         assert rel(a, b) < SPREAD_TOL[prec]
+
+
+def _crowded(lx, ly, lz, levels, seed, lo, hi):
+    """Cells whose vertices lie anywhere between the corners lo and hi (in
+    lattice nodes of the fluid frame), in random order."""
+    from preprocess_src_amd import mesh
+    nc = len(levels)
+    cells = mesh.assemble(levels, np.zeros((nc, 3)), np.repeat(np.eye(3)[None], nc, 0), 3.0)
+    rng = np.random.default_rng(seed)
+    n = cells["x"].size
+    # node i of an axis of m nodes sits at i - (m - 1) / 2
+    return cells, [rng.uniform(a, b, n) - (m - 1) / 2.0 for a, b, m in zip(lo, hi, (lx, ly, lz))]
+
+
+# corners of the first stencil nodes (a vertex between nodes i and i + 1 starts
+# its stencil at i - 1): within one tile of 16 x 8 x 8 below the sort's capacity,
+# above it (several passes), in one lattice cell below and above it, and more
+# vertices than 16-bit indices hold; across the lower wall
+CROWDS = [([3, 3], (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)), ([4, 4], (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)),
+          ([3], (5.1, 12.1, 12.1), (5.9, 12.9, 12.9)), ([4], (5.1, 12.1, 12.1), (5.9, 12.9, 12.9)),
+          ([5, 3], (5.1, 12.1, 12.1), (6.9, 12.9, 12.9)), ([5] * 7, (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)),
+          ([4, 4], (2.0, -0.5, 9.0), (16.9, 1.0, 16.9))]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("k", range(len(CROWDS)))
+def test_spread_of_crowded_tiles(k, prec, monkeypatch):
+    """Home boxes summed per lattice cell: tiles and cells around the
+    capacities of the sort; forces over several decades."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
+    levels, lo, hi = CROWDS[k]
+    lx, ly, lz = 48, 40, 40
+    print(f"[crowd] {k} {prec}", flush=True)
+    cells, pos = _crowded(lx, ly, lz, levels, 17 + k, lo, hi)
+    rng = np.random.default_rng(4)
+    n = pos[0].size
+    forces = [1e-3 * rng.standard_normal(n) * 10.0 ** rng.uniform(-4, 0, n) for _ in range(3)]
+    F, ref = _spread_both(lx, ly, lz, prec, cells, pos, forces)
+    for a, b in zip(F, ref):
+        assert rel(a, b) < SPREAD_TOL[prec]
+
+
+def test_spread_of_crowded_tiles_does_not_depend_on_the_order():
+    """Repeated binning places the vertices of a tile in another order; the
+    lattice force keeps its bits."""
+    lx, ly, lz = 48, 40, 40
+    cells, pos = _crowded(lx, ly, lz, [4, 4, 3], 3, (2.0, 2.0, 2.0), (40.0, 34.0, 34.0))
+    rng = np.random.default_rng(4)
+    forces = [1e-3 * rng.standard_normal(pos[0].size) for _ in range(3)]
+    g = gpu_of(lx, ly, lz, "f32", cells=cells)
+    out = []
+    for _ in range(6):
+        g.set_cells_state(x=pos[0], y=pos[1], z=pos[2], fx=forces[0], fy=forces[1], fz=forces[2])
+        g.ibm_st1()
+        out.append(np.concatenate(g.lattice_force()))
+    g.close()
+    for a in out[1:]:
+        assert np.array_equal(a, out[0])
