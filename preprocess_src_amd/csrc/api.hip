@@ -640,7 +640,9 @@ lbmibm_status lbmibm_create(const lbmibm_params *p, const lbmibm_cells *cells, l
         std::vector<double> ones(nc, 1.0);
         CK(up_T(&ctx->gscale, ones.data(), nc));
         // lattice tiles and vertex bins of the immersed-boundary kernels
-        ctx->ntx = (ctx->nx + TILE_X - 1) / TILE_X;
+        ctx->pointwise = ctx->prec != LBMIBM_F64 && p->vof_period > 0;
+        ctx->tile_x = ctx->pointwise ? TILE_XW : TILE_X;
+        ctx->ntx = (ctx->nx + ctx->tile_x - 1) / ctx->tile_x;
         ctx->nty = (ctx->ny + TILE_Y - 1) / TILE_Y;
         ctx->ntz = (ctx->nz + TILE_Z - 1) / TILE_Z;
         ctx->ntiles = ctx->ntx * ctx->nty * ctx->ntz;

@@ -37,12 +37,13 @@ struct DevStatus {
 constexpr int VOL_SMALL = 3072;
 constexpr int VOL_CH = 1024;  // elements / vertices per volume-correction chunk
 constexpr int TILE_X = 8, TILE_Y = 8, TILE_Z = 8;
+constexpr int TILE_XW = 16;  // tile width in x where the spreading sums point by point (lbmibm_ctx::pointwise)
 constexpr int ASM_CH = 256;  // vertices per chunk of the fused membrane assembly (k_assemble)
 
 // Lattice geometry of the vertex binning: unpadded and padded sizes, walls
 // beyond the y range or periodic y, spacing and tiles per axis.
 struct BinGeom {
-    int nx, ny, nz, nxp, nyp, nzp, walls, ntx, nty;
+    int nx, ny, nz, nxp, nyp, nzp, walls, ntx, nty, tx;  // tx: nodes of a tile in x
     double dx;
 };
 
@@ -66,7 +67,7 @@ __device__ __forceinline__ int home_tile(const BinGeom &g, double x, double y, d
     xw = min(max(xw, 0), g.nx - 1);
     zw = min(max(zw, 0), g.nz - 1);
     yh = min(max(yh, 0), g.ny - 1);
-    return xw / TILE_X + g.ntx * (yh / TILE_Y + g.nty * (zw / TILE_Z));
+    return xw / g.tx + g.ntx * (yh / TILE_Y + g.nty * (zw / TILE_Z));
 }
 
 // Additions to per-tile counters in device memory, combined per work group: a
@@ -77,7 +78,7 @@ __device__ __forceinline__ int home_tile(const BinGeom &g, double x, double y, d
 // line's atomics one after another, which one atomic per wave and tile made
 // about 10 times as many.  Any order and any number of tiles is accepted (the
 // table has twice as many entries as a group has vertices).  On 64 cells of
-// 2562 vertices, per launch before and after: k_vol_center 22.0 -> 7.4 us,
+// 2562 vertices, per launch before and after: k_vol_center 22.0 -> 9.4 us,
 // k_bin_scatter 22.2 -> 6.4 us, k_bin_count 23.0 -> 5.4 us.
 constexpr int BIN_WG = 1024;  // vertices per work group of the binning kernels
 struct TileTable {
@@ -249,6 +250,13 @@ struct lbmibm_ctx {
     // immersed boundary: vertices binned by the lattice tile of their first
     // stencil node (rebuilt whenever the positions change)
     int ntx = 0, nty = 0, ntz = 0, ntiles = 0, nblk_bin = 0;
+    // FP32 values under a volume-of-fluid indicator, which is FP64: the
+    // indicator's sweeps switch on the last bits of the velocity (a different
+    // rounding of the spread force alone moves vf by 2e-6), so these runs
+    // keep FP32 products summed point by point, over tiles of TILE_XW nodes,
+    // and with them the results they always had.
+    bool pointwise = false;
+    int tile_x = lbmibm::TILE_X;  // nodes of a tile in x
     short4 *node0 = nullptr;                 // [Nv] first stencil node (x,z wrapped, y+3), bin order
     void *srec = nullptr;                    // [Nv] stencil fractions and force (6 T), bin order
     int *home = nullptr, *home_list = nullptr;  // [Nv]

@@ -45,6 +45,7 @@ struct IbmGeom {
 
 struct TileGeom {
     int ntx, nty, ntz, ntiles;
+    int tx;  // nodes of a tile in x
 };
 
 __device__ __forceinline__ bool wrap_index(int &i, int n) {
@@ -61,24 +62,25 @@ __device__ __forceinline__ int pmod(int i, int n) {
 // sin and cos of (pi/2) t for t in [0, 1).  FP32: Taylor series of both to
 // degree 13 / 12 in x = (pi/2) t (truncation below 1e-9 on [0, pi/2), so the
 // result is within a few ulp of the correctly rounded value), evaluated by
-// Horner in x^2 with no range reduction.
+// Horner in x^2 with no range reduction; explicit multiply-adds, so that the
+// bits do not depend on where the compiler moves the terms.
 __device__ __forceinline__ void sincos_quarter(float t, float *s, float *c) {
     const float x = 1.57079632679489662f * t, x2 = x * x;
     float ps = -1.0f / 6227020800.0f;
-    ps = ps * x2 + 1.0f / 39916800.0f;
-    ps = ps * x2 - 1.0f / 362880.0f;
-    ps = ps * x2 + 1.0f / 5040.0f;
-    ps = ps * x2 - 1.0f / 120.0f;
-    ps = ps * x2 + 1.0f / 6.0f;
+    ps = fmaf(ps, x2, 1.0f / 39916800.0f);
+    ps = fmaf(ps, x2, -1.0f / 362880.0f);
+    ps = fmaf(ps, x2, 1.0f / 5040.0f);
+    ps = fmaf(ps, x2, -1.0f / 120.0f);
+    ps = fmaf(ps, x2, 1.0f / 6.0f);
     // sin x = x (1 - x^2 (1/6 - x^2 (1/120 - ...)))
-    *s = x - x * x2 * ps;
+    *s = fmaf(-x * x2, ps, x);
     float pc = 1.0f / 479001600.0f;
-    pc = pc * x2 - 1.0f / 3628800.0f;
-    pc = pc * x2 + 1.0f / 40320.0f;
-    pc = pc * x2 - 1.0f / 720.0f;
-    pc = pc * x2 + 1.0f / 24.0f;
-    pc = pc * x2 - 0.5f;
-    *c = 1.0f + x2 * pc;
+    pc = fmaf(pc, x2, -1.0f / 3628800.0f);
+    pc = fmaf(pc, x2, 1.0f / 40320.0f);
+    pc = fmaf(pc, x2, -1.0f / 720.0f);
+    pc = fmaf(pc, x2, 1.0f / 24.0f);
+    pc = fmaf(pc, x2, -0.5f);
+    *c = fmaf(x2, pc, 1.0f);
 }
 // FP64: the Taylor series of both to degree 17 / 16 of x = (pi/2) min(t, 1 - t)
 // in [0, pi/4] (1 - t is exact for t >= 1/2; the first terms left out are below
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(1024) void k_tile_order(const int *__restrict__ til
     for (int t = threadIdx.x; t < ntiles; t += 1024) {
         const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
         int sxs[4], sys[4], szs[4];
-        const int nsx = source_tiles(tx, tx * TILE_X, g.nx, TILE_X, true, sxs);
+        const int nsx = source_tiles(tx, tx * tg.tx, g.nx, tg.tx, true, sxs);
         const int nsy = source_tiles(ty, ty * TILE_Y, g.ny, TILE_Y, !g.walls, sys);
         const int nsz = source_tiles(tz, tz * TILE_Z, g.nz, TILE_Z, true, szs);
         int c = 0;
@@ -556,12 +558,12 @@ __global__ __launch_bounds__(256) void k_spread_tiles(const SpreadRec<T> *__rest
     __shared__ int queue[4][128];
     const int tile = order[blockIdx.x];
     const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
-    const int ox = tx * TILE_X, oy = ty * TILE_Y, oz = tz * TILE_Z;
-    const int lx = min(TILE_X, g.nx - ox), ly = min(TILE_Y, g.ny - oy), lz = min(TILE_Z, g.nz - oz);
+    const int ox = tx * tg.tx, oy = ty * TILE_Y, oz = tz * TILE_Z;
+    const int lx = min(tg.tx, g.nx - ox), ly = min(TILE_Y, g.ny - oy), lz = min(TILE_Z, g.nz - oz);
     for (int k = threadIdx.x; k < 3 * ACC_N; k += blockDim.x) acc[k] = 0ull;
     // source bins: tiles holding first stencil nodes that reach this tile
     int sxs[4], sys[4], szs[4];
-    const int nsx = source_tiles(tx, ox, g.nx, TILE_X, true, sxs);
+    const int nsx = source_tiles(tx, ox, g.nx, tg.tx, true, sxs);
     const int nsy = source_tiles(ty, oy, g.ny, TILE_Y, !g.walls, sys);
     const int nsz = source_tiles(tz, oz, g.nz, TILE_Z, true, szs);
     // fixed-point scale: at most `total` vertices reach one node, each with a
@@ -626,8 +628,8 @@ __global__ __launch_bounds__(256) void k_spread_tiles(const SpreadRec<T> *__rest
     __syncthreads();
     const double inv_scale = 1.0 / scale;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
-    for (int k = threadIdx.x; k < TILE_X * TILE_Y * TILE_Z; k += blockDim.x) {
-        const int la = k % TILE_X, lb = (k / TILE_X) % TILE_Y, lc = k / (TILE_X * TILE_Y);
+    for (int k = threadIdx.x; k < tg.tx * TILE_Y * TILE_Z; k += blockDim.x) {
+        const int la = k % tg.tx, lb = (k / tg.tx) % TILE_Y, lc = k / (tg.tx * TILE_Y);
         if (la >= lx || lb >= ly || lc >= lz) continue;
         const size_t nidx = (size_t)(ox + la) + (size_t)g.nx * ((size_t)(oy + lb) + (size_t)g.ny * (oz + lc));
         const int li = la + ACC_SX * lb + ACC_SXY * lc;
@@ -1001,15 +1003,91 @@ __global__ __launch_bounds__(1024) void k_spread_combine(T *__restrict__ S, cons
     }
 }
 
+// Spreading, form 1, point by point (lbmibm_ctx::pointwise): every vertex adds
+// its 64 products, formed in FP32, to the box of its tile, at the rate of the
+// LDS atomics.  Such runs hardly notice it: 15 of the 800 us of a step on
+// 77x46x51 nodes, which the indicator's sweeps bound.  Lane l of wave w takes column
+// NW l + w of the bin read as WG columns, so that the lanes of a wave hold
+// vertices far apart.
+constexpr int SP_X = TILE_XW + 3, SP_N = SP_X * SB_Y * SB_Z;
+__global__ __launch_bounds__(SPREAD_BOX_WG) void k_spread_points(const SpreadRec<float> *__restrict__ rec,
+                                                                 const short4 *__restrict__ node0,
+                                                                 const int *__restrict__ tile_count,
+                                                                 const int *__restrict__ tile_off,
+                                                                 float *__restrict__ S, IbmGeom g, TileGeom tg,
+                                                                 const int *__restrict__ order) {
+    __shared__ unsigned long long acc[3 * SP_N];
+    __shared__ float wmax[SPREAD_BOX_WG / 64];
+    const int tile = order[blockIdx.x];
+    const int cnt = tile_count[tile], off = tile_off[tile];
+    if (cnt == 0) return;  // whole work group leaves together; the gather skips empty tiles
+    const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
+    const int ox = tx * TILE_XW, oy = ty * TILE_Y, oz = tz * TILE_Z;
+    for (int k = threadIdx.x; k < 3 * SP_N; k += SPREAD_BOX_WG) acc[k] = 0ull;
+    constexpr int NW = SPREAD_BOX_WG / 64;
+    const int R = (cnt + SPREAD_BOX_WG - 1) / SPREAD_BOX_WG;
+    const int first = (NW * (threadIdx.x & 63) + (threadIdx.x >> 6)) * R, last = min(first + R, cnt);
+    float fm = 0.0f;
+    for (int i = first; i < last; i++) {
+        const SpreadRec<float> sr = rec[off + i];
+        fm = fmaxf(fm, fmaxf(fabsf(sr.f[0]), fmaxf(fabsf(sr.f[1]), fabsf(sr.f[2]))));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) fm = fmaxf(fm, __shfl_xor(fm, o));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = fm;
+    __syncthreads();
+    fm = wmax[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) fm = fmaxf(fm, wmax[w]);
+    const double fmax = (double)fm * (1.0 + 0x1p-20);  // scale as in k_spread_box
+    double scale = 1.0;
+    if (fmax > 0.0) {
+        const double bound = (double)cnt * fmax / (8.0 * g.dx * g.dx * g.dx);
+        scale = ldexp(1.0, FixedPoint<float>::kBits - 1 - ilogb(bound));
+    }
+    const float w64 = (float)(1.0 / (64.0 * g.dx * g.dx * g.dx));
+    for (int i = first; i < last; i++) {
+        const short4 n0 = node0[off + i];
+        const SpreadRec<float> sr = rec[off + i];
+        const int bx = n0.x - ox, bz = n0.z - oz;
+        int y1 = n0.y - 3;
+        if (!g.walls) wrap_index(y1, g.ny);
+        const int by = y1 - oy;
+        if (bx < 0 || bx >= TILE_XW || bz < 0 || bz >= TILE_Z || by < -3 || by >= TILE_Y) continue;  // not a valid home
+        float wx[4], wy[4], wz[4];
+        stencil_weights<float>(sr.t[0], wx);
+        stencil_weights<float>(sr.t[1], wy);
+        stencil_weights<float>(sr.t[2], wz);
+        const FixedPoint<float> fp(sr.f[0], sr.f[1], sr.f[2], scale);
+#pragma unroll
+        for (int kz = 0; kz < 4; kz++) {
+#pragma unroll
+            for (int ky = 0; ky < 4; ky++) {
+                if (by + ky < 0) continue;  // below the wall
+                const float wyz = wy[ky] * wz[kz] * w64;
+                const int row = bx + SP_X * ((by + ky) + SB_Y * (bz + kz));
+#pragma unroll
+                for (int kx = 0; kx < 4; kx++) fp.add(acc, row + kx, wx[kx] * wyz, SP_N);
+            }
+        }
+    }
+    __syncthreads();
+    const double inv_scale = 1.0 / scale;
+    float *St = S + (size_t)tile * 3 * SP_N;
+    for (int k = threadIdx.x; k < 3 * SP_N; k += SPREAD_BOX_WG)
+        St[k] = (float)FixedPoint<float>::real(acc[k], inv_scale);
+}
+
 // Sums, per lattice node, the box entries of k_spread_box that map to it, in
 // a fixed order (deterministic).  cx/cy/cz list for each coordinate of an axis
 // up to SB_MAXC entries (tile index along the axis) * 32 + box coordinate,
 // padded with -1 (built once on the host).
-template <typename T>
+template <typename T, int TX>
 __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, const int *__restrict__ tile_count,
                                                        const int *__restrict__ cx, const int *__restrict__ cy,
                                                        const int *__restrict__ cz, T *__restrict__ F, IbmGeom g,
                                                        TileGeom tg) {
+    constexpr int BX = TX + 3, BN = BX * SB_Y * SB_Z;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
     // each XCD gathers one contiguous eighth of the lattice: the box rows
     // of neighbouring y rows share cache lines, which are then fetched into
@@ -1038,7 +1116,7 @@ __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, 
         for (int iy = 0; iy < SB_MAXC; iy++) {
             if (ey[iy] < 0) break;
             const int tyz = tg.ntx * ((ey[iy] >> 5) + tg.nty * (ez[iz] >> 5));
-            const int byz = SB_X * ((ey[iy] & 31) + SB_Y * (ez[iz] & 31));
+            const int byz = BX * ((ey[iy] & 31) + SB_Y * (ez[iz] & 31));
             int cnt[SB_MAXC];
 #pragma unroll
             for (int ix = 0; ix < SB_MAXC; ix++) cnt[ix] = ex[ix] >= 0 ? tile_count[(ex[ix] >> 5) + tyz] : 0;
@@ -1047,10 +1125,10 @@ __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, 
             for (int ix = 0; ix < SB_MAXC; ix++) {
                 v0[ix] = v1[ix] = v2[ix] = T(0);
                 if (cnt[ix] > 0) {
-                    const size_t b = (size_t)((ex[ix] >> 5) + tyz) * 3 * SB_N + (ex[ix] & 31) + byz;
+                    const size_t b = (size_t)((ex[ix] >> 5) + tyz) * 3 * BN + (ex[ix] & 31) + byz;
                     v0[ix] = S[b];
-                    v1[ix] = S[b + SB_N];
-                    v2[ix] = S[b + 2 * SB_N];
+                    v1[ix] = S[b + BN];
+                    v2[ix] = S[b + 2 * BN];
                 }
             }
 #pragma unroll
@@ -1065,13 +1143,36 @@ __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, 
 
 // ---- interpolation + advection ------------------------------------------------
 
+// The part of a tile's bin that work group b takes: the tiles that
+// k_spread_box shares out are shared out here too, their vertices in equal
+// parts, the extra parts first.  False (for the whole group) without any.
+__device__ __forceinline__ bool tile_part(int b, const int *__restrict__ order, const int2 *__restrict__ extra,
+                                          int maxextra, const int *__restrict__ tile_count,
+                                          const int *__restrict__ tile_off, int &tile, int &cnt, int &off) {
+    int chunk = 0;
+    if (b < maxextra) {
+        const int2 ex = extra[b];
+        if (ex.x < 0) return false;
+        tile = ex.x;
+        chunk = ex.y;
+    } else {
+        tile = order[b - maxextra];
+    }
+    const int all = tile_count[tile];
+    if (all == 0) return false;
+    const int nch = spread_chunks(all), first = (int)((long long)all * chunk / nch);
+    cnt = (int)((long long)all * (chunk + 1) / nch) - first;
+    off = tile_off[tile] + first;
+    return true;
+}
+
 // Velocity box staged per tile: the tile plus 1 node below and 4 above on
 // every axis.  The first stencil node of a home vertex lies in the tile, an
 // RK stage moves it by less than one node in practice (|u| M dt << dx), and
 // the stencil spans 4 nodes; stages that leave the box read global memory.
 constexpr int RX = TILE_X + 5, RY = TILE_Y + 5, RZ = TILE_Z + 5, RN = RX * RY * RZ;
 constexpr int RLO = 1;  // nodes of the box below the tile
-constexpr int INTERP_WG = 512;  // work-group size of k_interp_tiles
+constexpr int INTERP_WG = 256;  // work-group size of k_interp_tiles (a tile of the suspension holds 300 vertices)
 
 // Out-of-line and not unrolled: it is the rare path, and inlining it into
 // every RK stage would multiply the kernel's code size.
@@ -1106,41 +1207,6 @@ __device__ __forceinline__ void interp_global(const T *__restrict__ U, size_t N,
     }
 }
 
-// Interpolation from the staged box when the stencil lies inside it.
-template <typename T>
-__device__ __forceinline__ void interp_tile(const T *__restrict__ U, size_t N, const T *__restrict__ Us,
-                                            const IbmGeom &g, int bx, int by, int bz, double x, double y, double z,
-                                            bool unit, T &ur, T &vr, T &wr) {
-    int x1, y1, z1;
-    T wx[4], wy[4], wz[4];
-    stencil3<T>(g, x, y, z, unit, x1, y1, z1, wx, wy, wz);
-    int rx = x1 - bx, rz = z1 - bz, ry = y1 - by;
-    if (rx < 0) rx += g.nx; else if (rx >= g.nx) rx -= g.nx;
-    if (rz < 0) rz += g.nz; else if (rz >= g.nz) rz -= g.nz;
-    if (!g.walls) { if (ry < 0) ry += g.ny; else if (ry >= g.ny) ry -= g.ny; }
-    if (rx < 0 || rx + 3 >= RX || ry < 0 || ry + 3 >= RY || rz < 0 || rz + 3 >= RZ) {
-        interp_global<T>(U, N, g, x, y, z, unit, ur, vr, wr);
-        return;
-    }
-    ur = vr = wr = T(0);
-#pragma unroll
-    for (int kz = 0; kz < 4; kz++) {
-        const T wz64 = wz[kz] * T(1.0 / 64.0);
-#pragma unroll
-        for (int ky = 0; ky < 4; ky++) {
-            const T wyz = wy[ky] * wz64;
-            const int row = rx + RX * ((ry + ky) + RY * (rz + kz));
-#pragma unroll
-            for (int kx = 0; kx < 4; kx++) {
-                const T dlt = wx[kx] * wyz;
-                ur += dlt * Us[row + kx];
-                vr += dlt * Us[RN + row + kx];
-                wr += dlt * Us[2 * RN + row + kx];
-            }
-        }
-    }
-}
-
 struct AdvectArgs {
     double dt, M;
     double lx, ly, lz;
@@ -1154,74 +1220,161 @@ template <typename T> struct Row4 {
     T v[4];
 } __attribute__((aligned(sizeof(T))));
 
-// Interpolation straight from the velocity field: one wide load per stencil
-// row and component, the same products and summation order as interp_tile.
-// A row that wraps in x is read node by node.
-template <typename T>
-__device__ __forceinline__ void interp_rows(const T *__restrict__ U, size_t N, const IbmGeom &g, double x,
-                                            double y, double z, bool unit, T &ur, T &vr, T &wr) {
-    int x1, y1, z1;
-    T wx[4], wy[4], wz[4];
-    stencil3<T>(g, x, y, z, unit, x1, y1, z1, wx, wy, wz);
-    const bool whole = x1 >= 0 && x1 + 3 < g.nx;
-    int ixw[4];
-    bool okx[4];
+// The interpolated velocity inside one lattice cell.  With t = frac(X/h) the
+// four weights of an axis are 1 - s, 1 + c, 1 + s, 1 - c (s, c = sin, cos of
+// pi t / 2), so a row contributes (u0+u1+u2+u3) + s (u2-u0) + c (u1-u3), and the
+// 64 stencil nodes reduce to 27 coefficients per component of the products of
+// (1, s, c) along the axes.  They depend on the cell alone: the RK stages move a
+// vertex by a small part of a cell, so one reading of the 192 node values
+// serves all four stages almost always, and a stage takes 78 FMAs instead of
+// 272.  What bounded both forms was the VALU (2700 instructions per vertex, now
+// 2100) and the reads (768 LDS values per vertex, or 48 rows per stage).  Per
+// launch before and after, the form that each size takes: 64 cells of 2562
+// vertices (FP32) 65 -> 29.6 us, 32 such cells 46 -> 27, 384 uneven cells in
+// FP64 245 -> 147, the 1024-cell suspension (FP32) 212 -> 214: there the VALU
+// is busy for two thirds of the launch either way, and reading the velocity
+// from one XCD's L2 (872 -> 244 MB fetched, tile rows kept on one XCD) gained
+// nothing against the heavy-first order.
+template <typename T> struct CellField {
+    int x1, y1, z1;  // first stencil node of the cell (unpadded)
+    T a[3][27];      // [component][z][y][x], over (1, s, c) each
+    // fetch(kx-row of 4 values, ky, kz, component)
+    template <typename Fetch> __device__ __forceinline__ void load(Fetch fetch) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        ixw[k] = x1 + k;
-        okx[k] = wrap_index(ixw[k], g.nx);
-    }
-    ur = vr = wr = T(0);
+        for (int d = 0; d < 3; d++) {
+            T *o = a[d];
 #pragma unroll
-    for (int kz = 0; kz < 4; kz++) {
-        int iz = z1 + kz;
-        if (!wrap_index(iz, g.nz)) continue;
-        const T wz64 = wz[kz] * T(1.0 / 64.0);
+            for (int kz = 0; kz < 4; kz++) {
+                T r[4][3];
 #pragma unroll
-        for (int ky = 0; ky < 4; ky++) {
-            int iy = y1 + ky;
-            if (g.walls) {
-                if (iy < 0 || iy >= g.ny) continue;
-            } else if (!wrap_index(iy, g.ny)) continue;
-            const T wyz = wy[ky] * wz64;
-            const size_t rowb = (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz);
-            T ru[4], rv[4], rw[4];
-            if (whole) {
-                const Row4<T> a = *(const Row4<T> *)(U + rowb + x1);
-                const Row4<T> b = *(const Row4<T> *)(U + N + rowb + x1);
-                const Row4<T> c = *(const Row4<T> *)(U + 2 * N + rowb + x1);
-#pragma unroll
-                for (int kx = 0; kx < 4; kx++) { ru[kx] = a.v[kx]; rv[kx] = b.v[kx]; rw[kx] = c.v[kx]; }
-            } else {
-#pragma unroll
-                for (int kx = 0; kx < 4; kx++) {
-                    const size_t n = rowb + (okx[kx] ? ixw[kx] : 0);
-                    ru[kx] = okx[kx] ? U[n] : T(0);
-                    rv[kx] = okx[kx] ? U[N + n] : T(0);
-                    rw[kx] = okx[kx] ? U[2 * N + n] : T(0);
+                for (int ky = 0; ky < 4; ky++) {
+                    T u[4];
+                    fetch(u, ky, kz, d);
+                    r[ky][0] = (u[0] + u[2]) + (u[1] + u[3]);
+                    r[ky][1] = u[2] - u[0];
+                    r[ky][2] = u[1] - u[3];
                 }
-            }
 #pragma unroll
-            for (int kx = 0; kx < 4; kx++) {
-                const T dlt = wx[kx] * wyz;
-                ur += dlt * ru[kx];
-                vr += dlt * rv[kx];
-                wr += dlt * rw[kx];
+                for (int m = 0; m < 3; m++) {
+                    const T y[3] = {(r[0][m] + r[2][m]) + (r[1][m] + r[3][m]), r[2][m] - r[0][m], r[1][m] - r[3][m]};
+#pragma unroll
+                    for (int l = 0; l < 3; l++) {
+                        const int k = 3 * l + m;
+                        if (kz == 0) { o[k] = y[l]; o[9 + k] = -y[l]; }
+                        if (kz == 1) { o[k] += y[l]; o[18 + k] = y[l]; }
+                        if (kz == 2) { o[k] += y[l]; o[9 + k] += y[l]; }
+                        if (kz == 3) { o[k] += y[l]; o[18 + k] -= y[l]; }
+                    }
+                }
+                // one slice's loads at a time: all 192 in flight would take
+                // the registers of two more waves
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+    }
+    __device__ __forceinline__ void at(const T sn[3], const T cs[3], T &ur, T &vr, T &wr) const {
+        T v[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            T z[3];
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                T y[3];
+#pragma unroll
+                for (int l = 0; l < 3; l++) {
+                    const T *q = a[d] + 9 * k + 3 * l;
+                    y[l] = fma(cs[0], q[2], fma(sn[0], q[1], q[0]));
+                }
+                z[k] = fma(cs[1], y[2], fma(sn[1], y[1], y[0]));
+            }
+            v[d] = fma(cs[2], z[2], fma(sn[2], z[1], z[0])) * T(1.0 / 64.0);
+        }
+        ur = v[0]; vr = v[1]; wr = v[2];
+    }
+    // sum_d k_d times the gradient of component d; kf = pi / (2 h) turns the
+    // derivatives (0, c, -s) of (1, s, c) into those along the position
+    __device__ __forceinline__ void grad(const T k[3], const T sn[3], const T cs[3], T kf, T out[3]) const {
+        T V[3], DX[3], DY[3];
+#pragma unroll
+        for (int z = 0; z < 3; z++) {
+            T vx[3], dx[3];
+#pragma unroll
+            for (int l = 0; l < 3; l++) {
+                T b[3];
+#pragma unroll
+                for (int m = 0; m < 3; m++) {
+                    const int q = 9 * z + 3 * l + m;
+                    b[m] = fma(k[2], a[2][q], fma(k[1], a[1][q], k[0] * a[0][q]));
+                }
+                vx[l] = fma(cs[0], b[2], fma(sn[0], b[1], b[0]));
+                dx[l] = fma(cs[0], b[1], -(sn[0] * b[2]));
+            }
+            V[z] = fma(cs[1], vx[2], fma(sn[1], vx[1], vx[0]));
+            DX[z] = fma(cs[1], dx[2], fma(sn[1], dx[1], dx[0]));
+            DY[z] = fma(cs[1], vx[1], -(sn[1] * vx[2]));
+        }
+        const T q = kf * T(1.0 / 64.0);
+        out[0] = q * fma(cs[2], DX[2], fma(sn[2], DX[1], DX[0]));
+        out[1] = q * fma(cs[2], DY[2], fma(sn[2], DY[1], DY[0]));
+        out[2] = q * fma(cs[2], V[1], -(sn[2] * V[2]));
+    }
+    // load() from a field [3][N] in memory; every active lane of the wave calls it
+    __device__ __forceinline__ void load_field(const T *__restrict__ U, size_t N, const IbmGeom &g, const int f[3]) {
+        x1 = f[0]; y1 = f[1]; z1 = f[2];
+        const bool whole = __all(f[0] >= 0 && f[0] + 3 < g.nx);
+        int ixw[4];
+        bool okx[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            ixw[k] = f[0] + k;
+            okx[k] = wrap_index(ixw[k], g.nx);
+        }
+        load([&](T *o, int ky, int kz, int d) {
+            int iy = f[1] + ky, iz = f[2] + kz;
+            const bool ok = wrap_index(iz, g.nz) && (g.walls ? (iy >= 0 && iy < g.ny) : wrap_index(iy, g.ny));
+            // a row outside the lattice holds 0
+            const size_t row = ok ? d * N + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz) : 0;
+            if (whole) {  // one (unaligned) wide load
+                const Row4<T> r = *(const Row4<T> *)(U + row + f[0]);
+#pragma unroll
+                for (int kx = 0; kx < 4; kx++) o[kx] = ok ? r.v[kx] : T(0);
+            } else {  // a row of the wave wraps in x
+#pragma unroll
+                for (int kx = 0; kx < 4; kx++) o[kx] = ok && okx[kx] ? U[row + (okx[kx] ? ixw[kx] : 0)] : T(0);
+            }
+        });
+    }
+    // whether a lane of the wave is in another cell than the one loaded
+    __device__ __forceinline__ bool left(const int f[3]) const { return __any(f[0] != x1 || f[1] != y1 || f[2] != z1); }
+};
+
+// First stencil node (unpadded, unwrapped) and sine and cosine of the
+// fractions of a position (as stencil3).
+template <typename W>
+__device__ __forceinline__ void cell_of(const IbmGeom &g, double x, double y, double z, bool unit, int f[3], W sn[3],
+                                        W cs[3]) {
+    const double X[3] = {x, y, z};
+    const int np[3] = {g.nxp, g.nyp, g.nzp};
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        // RK2 / Euler branches use unit spacing (ibm.cu:524-551, 581-608)
+        const double q = unit ? X[d] + (double)(np[d] - 1) / 2.0 : over_h(X[d] + (double)(np[d] - 1) * g.dx / 2.0, g.dx);
+        const double fl = floor(q);
+        f[d] = (int)fl - 3;
+        sincos_quarter((W)(q - fl), &sn[d], &cs[d]);
     }
 }
 
 // The RK stages of vertex j (ibm.cu:430-517, 524-551, 581-608) with the
-// interpolation ip(x, y, z, unit, u, v, w), then the periodic wrap of the new
-// position (ibm.cu:616-632) and its stores.  xin and xo may be the same array
-// (each vertex is read before it is written, by the same thread).
+// interpolation ip(stage, x, y, z, unit, u, v, w), then the periodic wrap of the new
+// position (ibm.cu:616-632) and its stores.  (xn, yn, zn) is the vertex's
+// position; xo may be the array that it was read from (each vertex is read
+// before it is written, by the same thread).
 template <typename T, typename Interp>
-__device__ __forceinline__ void advect_vertex(int j, const double *xin, double *xo, T *__restrict__ uvw,
+__device__ __forceinline__ void advect_vertex(int j, double xn, double yn, double zn, double *xo, T *__restrict__ uvw,
                                               double *__restrict__ xd, int nv, const AdvectArgs &a, Interp ip) {
     const double M = a.M, dt = a.dt;
     const bool unit = a.rk != 4;
-    const double xn = xin[j], yn = xin[nv + j], zn = xin[2 * (size_t)nv + j];
     // stage s is taken at X + k_{s-1} (M dt/2, M dt/2, M dt) for RK4 and
     // X + k_1 M for RK2, each offset evaluated as (k M) dt / 2 in that order;
     // the stage sum is (k1 + 2 k2 + 2 k3 + k4)/6, (k1 + k2)/2, k1.  One loop
@@ -1238,7 +1391,7 @@ __device__ __forceinline__ void advect_vertex(int j, const double *xin, double *
                 if (s < 3) { ox /= 2.0; oy /= 2.0; oz /= 2.0; }
             }
         }
-        ip(xn + ox, yn + oy, zn + oz, unit, ku, kv, kw);
+        ip(s, xn + ox, yn + oy, zn + oz, unit, ku, kv, kw);
         const T wt = (a.rk == 4 && (s == 1 || s == 2)) ? T(2) : T(1);
         su += wt * ku; sv += wt * kv; sw += wt * kw;
     }
@@ -1261,40 +1414,105 @@ __device__ __forceinline__ void advect_vertex(int j, const double *xin, double *
 // Interpolation form 0: one work group per tile stages the tile's velocity
 // plus halo in LDS once and runs its home vertices from there.
 template <typename T>
-__global__ __launch_bounds__(INTERP_WG) void k_interp_tiles(const T *__restrict__ U, const double *xin, double *xo,
+__global__ __launch_bounds__(INTERP_WG, sizeof(T) == 4 ? 3 : 2) void k_interp_tiles(const T *__restrict__ U, const double *xin, double *xo,
                                                       T *__restrict__ uvw, double *__restrict__ xd,
                                                       const int *__restrict__ tile_count,
                                                       const int *__restrict__ tile_off,
                                                       const int *__restrict__ home_list, int nv, IbmGeom g,
-                                                      TileGeom tg, AdvectArgs a, const int *__restrict__ order) {
+                                                      TileGeom tg, AdvectArgs a, const int *__restrict__ order,
+                                                      const int2 *__restrict__ extra, int maxextra) {
     extern __shared__ double dyn[];
     T *Us = (T *)dyn;  // [3][RZ][RY][RX]
-    const int tile = order[blockIdx.x];
-    const int cnt = tile_count[tile], off = tile_off[tile];
-    if (cnt == 0) return;  // whole work group leaves together
+    int tile, cnt, off;
+    if (!tile_part((int)blockIdx.x, order, extra, maxextra, tile_count, tile_off, tile, cnt, off)) return;
     const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
     const int bx = tx * TILE_X - RLO, by = ty * TILE_Y - RLO, bz = tz * TILE_Z - RLO;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
-    for (int k = threadIdx.x; k < RN; k += blockDim.x) {
-        const int rx = k % RX, ry = (k / RX) % RY, rz = k / (RX * RY);
-        // the box may span an axis more than once on small lattices
-        const int ix = pmod(bx + rx, g.nx), iz = pmod(bz + rz, g.nz);
-        int iy = by + ry;
-        bool ok = true;
-        if (g.walls) ok = iy >= 0 && iy < g.ny;
-        else iy = pmod(iy, g.ny);
-        T u = T(0), v = T(0), w = T(0);
-        if (ok) {
-            const size_t n = (size_t)ix + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz);
-            u = U[n]; v = U[N + n]; w = U[2 * N + n];
+    // the first vertex's position, read while the box is staged
+    int id = 0;
+    double x[3] = {0.0, 0.0, 0.0};
+    if ((int)threadIdx.x < cnt) {
+        id = home_list[off + threadIdx.x];
+#pragma unroll
+        for (int d = 0; d < 3; d++) x[d] = xin[d * (size_t)nv + id];
+    }
+    // 16 lanes per box row of 13 nodes, four rows at a time so that their
+    // loads are in flight together
+    static_assert(RX <= 16, "a row per 16 lanes");
+    const bool small = min(min(g.nx, g.nz), g.walls ? RY : g.ny) < RX;  // the box may span an axis more than once
+    const int rx = threadIdx.x & 15;
+    int ix = bx + rx;
+    if (small) ix = pmod(ix, g.nx);
+    else wrap_index(ix, g.nx);
+    constexpr int ROWS = INTERP_WG / 16, AHEAD = 4;
+    for (int row0 = threadIdx.x >> 4; row0 < RY * RZ; row0 += AHEAD * ROWS) {
+        T v[AHEAD][3];
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            const int row = row0 + j * ROWS;
+            int iy = by + row % RY, iz = bz + row / RY;
+            bool ok = row < RY * RZ && rx < RX;
+            if (small) iz = pmod(iz, g.nz);
+            else wrap_index(iz, g.nz);
+            if (g.walls) ok = ok && iy >= 0 && iy < g.ny;
+            else if (small) iy = pmod(iy, g.ny);
+            else wrap_index(iy, g.ny);
+            const size_t n = ok ? (size_t)ix + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz) : 0;
+#pragma unroll
+            for (int d = 0; d < 3; d++) v[j][d] = ok ? U[d * N + n] : T(0);
         }
-        Us[k] = u; Us[RN + k] = v; Us[2 * RN + k] = w;
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            const int row = row0 + j * ROWS;
+            if (row < RY * RZ && rx < RX)
+#pragma unroll
+                for (int d = 0; d < 3; d++) Us[d * RN + rx + RX * row] = v[j][d];
+        }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < cnt; i += blockDim.x) {
-        advect_vertex<T>(home_list[off + i], xin, xo, uvw, xd, nv, a,
-                         [&](double x, double y, double z, bool unit, T &u, T &v, T &w) {
-                             interp_tile<T>(U, N, Us, g, bx, by, bz, x, y, z, unit, u, v, w);
+    for (int i = threadIdx.x; i < cnt; i += INTERP_WG) {
+        // FP32: the next vertex's position while this one moves (FP64 has no
+        // registers for it)
+        const bool ahead = sizeof(T) == 4;
+        if (!ahead && i >= INTERP_WG) {
+            id = home_list[off + i];
+#pragma unroll
+            for (int d = 0; d < 3; d++) x[d] = xin[d * (size_t)nv + id];
+        }
+        const int j = id;
+        const double xn = x[0], yn = x[1], zn = x[2];
+        if (ahead && i + INTERP_WG < cnt) {
+            id = home_list[off + i + INTERP_WG];
+#pragma unroll
+            for (int d = 0; d < 3; d++) x[d] = xin[d * (size_t)nv + id];
+        }
+        CellField<T> cf;
+        bool out = false;
+        advect_vertex<T>(j, xn, yn, zn, xo, uvw, xd, nv, a,
+                         [&](int stage, double x, double y, double z, bool unit, T &u, T &v, T &w) {
+                             int f[3];
+                             T sn[3], cs[3];
+                             cell_of<T>(g, x, y, z, unit, f, sn, cs);
+                             // the whole wave reads again when one of its lanes left its cell
+                             // (a lane's own branch would keep both sets of coefficients)
+                             if (__any(stage == 0 || f[0] != cf.x1 || f[1] != cf.y1 || f[2] != cf.z1)) {
+                                 cf.x1 = f[0]; cf.y1 = f[1]; cf.z1 = f[2];
+                                 int rx = f[0] - bx, ry = f[1] - by, rz = f[2] - bz;
+                                 if (rx < 0) rx += g.nx; else if (rx >= g.nx) rx -= g.nx;
+                                 if (rz < 0) rz += g.nz; else if (rz >= g.nz) rz -= g.nz;
+                                 if (!g.walls) { if (ry < 0) ry += g.ny; else if (ry >= g.ny) ry -= g.ny; }
+                                 out = rx < 0 || rx + 3 >= RX || ry < 0 || ry + 3 >= RY || rz < 0 || rz + 3 >= RZ;
+                                 const T *row = Us + (out ? 0 : rx + RX * (ry + RY * rz));
+                                 cf.load([&](T *o, int ky, int kz, int d) {
+#pragma unroll
+                                     for (int kx = 0; kx < 4; kx++) o[kx] = row[d * RN + RX * (ky + RY * kz) + kx];
+                                 });
+                             }
+                             if (out) {  // not in the box: from memory
+                                 interp_global<T>(U, N, g, x, y, z, unit, u, v, w);
+                                 return;
+                             }
+                             cf.at(sn, cs, u, v, w);
                          });
     }
 }
@@ -1309,10 +1527,83 @@ __global__ __launch_bounds__(256) void k_interp_vert(const T *__restrict__ U, co
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nv) return;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
-    advect_vertex<T>(home_list[i], xin, xo, uvw, xd, nv, a,
-                     [&](double x, double y, double z, bool unit, T &u, T &v, T &w) {
-                         interp_rows<T>(U, N, g, x, y, z, unit, u, v, w);
+    const int j = home_list[i];
+    CellField<T> cf;
+    advect_vertex<T>(j, xin[j], xin[nv + j], xin[2 * (size_t)nv + j], xo, uvw, xd, nv, a,
+                     [&](int stage, double x, double y, double z, bool unit, T &u, T &v, T &w) {
+                         int f[3];
+                         T sn[3], cs[3];
+                         cell_of<T>(g, x, y, z, unit, f, sn, cs);
+                         if (stage == 0 || cf.left(f)) cf.load_field(U, N, g, f);
+                         cf.at(sn, cs, u, v, w);
                      });
+}
+
+// Interpolation point by point (lbmibm_ctx::pointwise): FP32 products summed in
+// the order of the stencil.  The rows of a z plane are read before they are
+// used; work groups of one wave spread the few vertices of such runs over the chip.
+__global__ __launch_bounds__(64) void k_interp_points(const float *__restrict__ U, const double *xin, double *xo,
+                                                      float *__restrict__ uvw, double *__restrict__ xd,
+                                                      const int *__restrict__ home_list, int nv, IbmGeom g,
+                                                      AdvectArgs a) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= nv) return;
+    const size_t N = (size_t)g.nx * g.ny * g.nz;
+    const int j = home_list[i];
+    advect_vertex<float>(
+        j, xin[j], xin[nv + j], xin[2 * (size_t)nv + j], xo, uvw, xd, nv, a,
+        [&](int, double x, double y, double z, bool unit, float &ur, float &vr, float &wr) {
+            int x1, y1, z1;
+            float wx[4], wy[4], wz[4];
+            stencil3<float>(g, x, y, z, unit, x1, y1, z1, wx, wy, wz);
+            const bool whole = x1 >= 0 && x1 + 3 < g.nx;
+            int ix[4];
+            bool okx[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                ix[k] = x1 + k;
+                okx[k] = wrap_index(ix[k], g.nx);
+            }
+            ur = vr = wr = 0.0f;
+#pragma unroll
+            for (int kz = 0; kz < 4; kz++) {
+                int iz = z1 + kz;
+                const bool okz = wrap_index(iz, g.nz);
+                float r[4][3][4];
+                bool ok[4];
+#pragma unroll
+                for (int ky = 0; ky < 4; ky++) {
+                    int iy = y1 + ky;
+                    ok[ky] = okz && (g.walls ? iy >= 0 && iy < g.ny : wrap_index(iy, g.ny));
+                    const size_t row = ok[ky] ? (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz) : 0;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        const float *u = U + d * N + row;
+                        if (whole) {  // one (unaligned) wide load
+                            const Row4<float> q = *(const Row4<float> *)(u + x1);
+#pragma unroll
+                            for (int kx = 0; kx < 4; kx++) r[ky][d][kx] = q.v[kx];
+                        } else {
+#pragma unroll
+                            for (int kx = 0; kx < 4; kx++) r[ky][d][kx] = okx[kx] ? u[ix[kx]] : 0.0f;
+                        }
+                    }
+                }
+                const float wz64 = wz[kz] * (1.0f / 64.0f);
+#pragma unroll
+                for (int ky = 0; ky < 4; ky++) {
+                    if (!ok[ky]) continue;
+                    const float wyz = wy[ky] * wz64;
+#pragma unroll
+                    for (int kx = 0; kx < 4; kx++) {
+                        const float dlt = wx[kx] * wyz;
+                        ur = fmaf(dlt, r[ky][0][kx], ur);
+                        vr = fmaf(dlt, r[ky][1][kx], vr);
+                        wr = fmaf(dlt, r[ky][2][kx], wr);
+                    }
+                }
+            }
+        });
 }
 
 // ---- adjoints (vector-Jacobian products) ------------------------------------
@@ -1326,94 +1617,6 @@ __global__ __launch_bounds__(256) void k_interp_vert(const T *__restrict__ U, co
 // position terms the same way, and adds the velocity adjoint to the nodes
 // per tile in LDS (k_advect_adj_scatter).
 
-template <typename W>
-__device__ __forceinline__ void stencil_d(double xtr, double h, int &first, W w[4], W dw[4]) {
-    const double q = over_h(xtr, h);
-    const double fl = floor(q);
-    first = (int)fl - 1;
-    const W t = (W)(q - fl);
-    W sn, cs;
-    sincos_quarter(t, &sn, &cs);
-    w[0] = W(1) - sn;
-    w[1] = W(1) + cs;
-    w[2] = W(1) + sn;
-    w[3] = W(1) - cs;
-    const W k = (W)(M_PI / (2.0 * h));
-    dw[0] = -k * cs;
-    dw[1] = -k * sn;
-    dw[2] = k * cs;
-    dw[3] = k * sn;
-}
-
-// Stencil of a position as stencil3 (spacing dx) with weight derivatives.
-template <typename W> struct StencilD {
-    int x1, y1, z1;
-    W wx[4], wy[4], wz[4], dx[4], dy[4], dz[4];
-    __device__ __forceinline__ StencilD(const IbmGeom &g, double x, double y, double z) {
-        stencil_d<W>(x + (double)(g.nxp - 1) * g.dx / 2.0, g.dx, x1, wx, dx);
-        stencil_d<W>(y + (double)(g.nyp - 1) * g.dx / 2.0, g.dx, y1, wy, dy);
-        stencil_d<W>(z + (double)(g.nzp - 1) * g.dx / 2.0, g.dx, z1, wz, dz);
-        x1 -= 2;
-        y1 -= 2;
-        z1 -= 2;
-    }
-    // visits every stencil node inside the lattice: f(node index, weight
-    // product, its gradient with respect to the position, stencil offsets)
-    template <typename Fn> __device__ __forceinline__ void each(const IbmGeom &g, Fn f) const {
-#pragma unroll
-        for (int kz = 0; kz < 4; kz++) {
-            int iz = z1 + kz;
-            if (!wrap_index(iz, g.nz)) continue;
-#pragma unroll
-            for (int ky = 0; ky < 4; ky++) {
-                int iy = y1 + ky;
-                if (g.walls) {
-                    if (iy < 0 || iy >= g.ny) continue;
-                } else if (!wrap_index(iy, g.ny)) continue;
-#pragma unroll
-                for (int kx = 0; kx < 4; kx++) {
-                    int ix = x1 + kx;
-                    if (!wrap_index(ix, g.nx)) continue;
-                    const size_t n = (size_t)ix + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz);
-                    const W w = wx[kx] * wy[ky] * wz[kz];
-                    const W gx = dx[kx] * wy[ky] * wz[kz], gy = wx[kx] * dy[ky] * wz[kz], gz = wx[kx] * wy[ky] * dz[kz];
-                    f(n, w, gx, gy, gz, kx, ky, kz);
-                }
-            }
-        }
-    }
-    // the 16 nodes of z-slice kz only (same products as each)
-    template <typename Fn> __device__ __forceinline__ void slice(const IbmGeom &g, int kz, Fn f) const {
-        int iz = z1 + kz;
-        if (!wrap_index(iz, g.nz)) return;
-        const W wzk = sel4(wz, kz), dzk = sel4(dz, kz);
-#pragma unroll
-        for (int ky = 0; ky < 4; ky++) {
-            int iy = y1 + ky;
-            if (g.walls) {
-                if (iy < 0 || iy >= g.ny) continue;
-            } else if (!wrap_index(iy, g.ny)) continue;
-#pragma unroll
-            for (int kx = 0; kx < 4; kx++) {
-                int ix = x1 + kx;
-                if (!wrap_index(ix, g.nx)) continue;
-                const size_t n = (size_t)ix + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz);
-                const W w = wx[kx] * wy[ky] * wzk;
-                const W gx = dx[kx] * wy[ky] * wzk, gy = wx[kx] * dy[ky] * wzk, gz = wx[kx] * wy[ky] * dzk;
-                f(n, w, gx, gy, gz);
-            }
-        }
-    }
-};
-
-// Sum over the 4 lanes of an aligned quad; every lane gets the same bits
-// ((a + b) + (c + d) in each, addition being commutative).
-template <typename T> __device__ __forceinline__ T quad_sum(T v) {
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
-    return v;
-}
-
 // Adjoint of ibm_st1 at the current positions and nodal forces: given Fa (the
 // adjoint of the lattice force), cfa = sum D Fa is the adjoint of the nodal
 // force and xa += sum (Fa . f) grad D that of the position, D = phi^3/dx^3.
@@ -1424,20 +1627,20 @@ __global__ __launch_bounds__(256) void k_spread_adj(const double *__restrict__ x
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nv) return;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
-    const StencilD<T> st(g, xs[j], xs[nv + j], xs[2 * (size_t)nv + j]);
-    const T f0 = cf[j], f1 = cf[nv + j], f2 = cf[2 * (size_t)nv + j];
-    const T w64 = (T)(1.0 / (64.0 * g.dx * g.dx * g.dx));
-    T b0 = T(0), b1 = T(0), b2 = T(0), x0 = T(0), x1 = T(0), x2 = T(0);
-    st.each(g, [&](size_t n, T w, T gx, T gy, T gz, int, int, int) {
-        const T a0 = Fa[n], a1 = Fa[N + n], a2 = Fa[2 * N + n];
-        b0 += w * a0; b1 += w * a1; b2 += w * a2;
-        const T s = a0 * f0 + a1 * f1 + a2 * f2;
-        x0 += s * gx; x1 += s * gy; x2 += s * gz;
-    });
-    cfa[j] = b0 * w64; cfa[nv + j] = b1 * w64; cfa[2 * (size_t)nv + j] = b2 * w64;
-    xa[j] += (double)(x0 * w64);
-    xa[nv + j] += (double)(x1 * w64);
-    xa[2 * (size_t)nv + j] += (double)(x2 * w64);
+    const T f0[3] = {cf[j], cf[nv + j], cf[2 * (size_t)nv + j]};
+    CellField<T> field;
+    int f[3];
+    T sn[3], cs[3], b[3], x[3];
+    cell_of<T>(g, xs[j], xs[nv + j], xs[2 * (size_t)nv + j], false, f, sn, cs);
+    field.load_field(Fa, N, g, f);
+    field.at(sn, cs, b[0], b[1], b[2]);
+    field.grad(f0, sn, cs, (T)(M_PI / (2.0 * g.dx)), x);
+    const T w = (T)(1.0 / (g.dx * g.dx * g.dx));  // both carry the 1/64
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        cfa[(size_t)d * nv + j] = b[d] * w;
+        xa[(size_t)d * nv + j] += (double)(x[d] * w);
+    }
 }
 
 // Adjoint of ibm_st2 with RK4 at the current positions and velocity field:
@@ -1447,7 +1650,7 @@ __global__ __launch_bounds__(256) void k_spread_adj(const double *__restrict__ x
 // ua += phi^3(X_s) kb_s and X_s-bar = sum (u . kb_s) grad phi^3, which feeds
 // the stage before it (ibm.cu:430-517: X2 = X + h/2 k1, X3 = X + h/2 k2,
 // X4 = X + h k3, X' = X + h (k1 + 2 k2 + 2 k3 + k4)/6, h = M dt).
-// Two kernels.  k_advect_adj_vert, four lanes per vertex in bin order, does
+// Two kernels.  k_advect_adj_vert, one lane per vertex in bin order, does
 // the gathers (the stage positions, X-bar) and writes each stage's position
 // and kb_s to a record; k_advect_adj_scatter, one work group per tile over
 // its home vertices, adds the velocity adjoint of the records.
@@ -1457,84 +1660,65 @@ template <typename T> struct AdvRec {
     T k[3];       // kb_s
 };
 
-// Four lanes per vertex (bin order): lane z of the quad sums the z-th slice
-// of every stencil, and quad_sum completes the sums in all four lanes, so
-// the four follow the same stage chain.  One lane per vertex left most of the
-// machine idle on the small cell counts the gradient is taken on.
+// One lane per vertex (bin order), the velocity and its gradient from the
+// coefficients of its cell (CellField), which the four stages nearly always
+// share.  Four lanes per vertex with a z-slice each, which read the 64 nodes
+// for every stage's velocity and again for its gradient, took 108 us on 32
+// cells of 2562 vertices; this takes 57.
 template <typename T>
 __global__ __launch_bounds__(256) void k_advect_adj_vert(const double *__restrict__ xs, const T *__restrict__ U,
                                                          double *__restrict__ xa, const int *__restrict__ home_list,
                                                          int nv, IbmGeom g, double h, AdvRec<T> *__restrict__ rec,
                                                          unsigned *__restrict__ kbmax) {
     __shared__ float shm[4];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = t >> 2, sub = t & 3;  // vertex in bin order, stencil z-slice
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;  // vertex in bin order
     float km = 0.0f;
-    if (i < nv) {  // the same for the four lanes of a quad
+    if (i < nv) {
         const int j = home_list[i];
         const size_t N = (size_t)g.nx * g.ny * g.nz;
-        const T q64 = T(1.0 / 64.0);
         const double X[3] = {xs[j], xs[nv + j], xs[2 * (size_t)nv + j]};
-        auto interp = [&](const double p[3], double k[3]) {
-            const StencilD<T> st(g, p[0], p[1], p[2]);
-            T u0 = T(0), u1 = T(0), u2 = T(0);
-            st.slice(g, sub, [&](size_t n, T w, T, T, T) {
-                u0 += w * U[n]; u1 += w * U[N + n]; u2 += w * U[2 * N + n];
-            });
-            k[0] = (double)(quad_sum(u0) * q64);
-            k[1] = (double)(quad_sum(u1) * q64);
-            k[2] = (double)(quad_sum(u2) * q64);
-        };
-        double P[4][3], k[3];
+        CellField<T> cf;
+        int f[3];
+        T sn[3], cs[3];
+        double P[4][3], back[4] = {0.0, h / 2.0, h / 2.0, h};  // X_s = X + back[s] k_{s-1}
 #pragma unroll
         for (int d = 0; d < 3; d++) P[0][d] = X[d];
-        interp(P[0], k);
 #pragma unroll
-        for (int d = 0; d < 3; d++) P[1][d] = X[d] + k[d] * h / 2.0;
-        interp(P[1], k);
+        for (int s = 0; s < 3; s++) {
+            cell_of<T>(g, P[s][0], P[s][1], P[s][2], false, f, sn, cs);
+            if (s == 0 || cf.left(f)) cf.load_field(U, N, g, f);
+            T k[3];
+            cf.at(sn, cs, k[0], k[1], k[2]);
 #pragma unroll
-        for (int d = 0; d < 3; d++) P[2][d] = X[d] + k[d] * h / 2.0;
-        interp(P[2], k);
-#pragma unroll
-        for (int d = 0; d < 3; d++) P[3][d] = X[d] + k[d] * h;
+            for (int d = 0; d < 3; d++) P[s + 1][d] = X[d] + (s < 2 ? (double)k[d] * h / 2.0 : (double)k[d] * h);
+        }
         const double xb[3] = {xa[j], xa[nv + j], xa[2 * (size_t)nv + j]};
-        double acc[3] = {xb[0], xb[1], xb[2]};
-        double kb[4][3];
+        double acc[3] = {xb[0], xb[1], xb[2]}, next[3] = {0.0, 0.0, 0.0};
         const double cw[4] = {h / 6.0, h / 3.0, h / 3.0, h / 6.0};
+        const T kf = (T)(M_PI / (2.0 * g.dx));
 #pragma unroll
-        for (int s = 0; s < 4; s++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) kb[s][d] = cw[s] * xb[d];
-        const double back[4] = {0.0, h / 2.0, h / 2.0, h};  // X_s = X + back[s] k_{s-1}
-#pragma unroll
-        for (int s = 3; s >= 0; s--) {  // kb_s is final here (stage s+1 came first)
-            const T k0 = (T)kb[s][0], k1 = (T)kb[s][1], k2 = (T)kb[s][2];
-            if (sub == s) {  // the quad's lanes write one record each
-                AdvRec<T> r;
-                r.p[0] = P[s][0]; r.p[1] = P[s][1]; r.p[2] = P[s][2];
-                r.k[0] = k0; r.k[1] = k1; r.k[2] = k2;
-                rec[4 * (size_t)i + s] = r;
-            }
-            km += fmaxf(fabsf((float)k0), fmaxf(fabsf((float)k1), fabsf((float)k2)));
-            const StencilD<T> st(g, P[s][0], P[s][1], P[s][2]);
-            T g0 = T(0), g1 = T(0), g2 = T(0);
-            st.slice(g, sub, [&](size_t n, T, T gx, T gy, T gz) {
-                const T sdot = U[n] * k0 + U[N + n] * k1 + U[2 * N + n] * k2;
-                g0 += sdot * gx; g1 += sdot * gy; g2 += sdot * gz;
-            });
-            const double xs_[3] = {(double)(quad_sum(g0) * q64), (double)(quad_sum(g1) * q64),
-                                   (double)(quad_sum(g2) * q64)};
+        for (int s = 3; s >= 0; s--) {  // kb_s = cw[s] xb + back[s + 1] X_{s+1}-bar
+            AdvRec<T> r;
 #pragma unroll
             for (int d = 0; d < 3; d++) {
-                acc[d] += xs_[d];
-                if (s > 0) kb[s - 1][d] += back[s] * xs_[d];
+                r.p[d] = P[s][d];
+                r.k[d] = (T)(cw[s] * xb[d] + next[d]);
+            }
+            rec[4 * (size_t)i + s] = r;
+            km += fmaxf(fabsf((float)r.k[0]), fmaxf(fabsf((float)r.k[1]), fabsf((float)r.k[2])));
+            cell_of<T>(g, P[s][0], P[s][1], P[s][2], false, f, sn, cs);
+            if (cf.left(f)) cf.load_field(U, N, g, f);
+            T gr[3];
+            cf.grad(r.k, sn, cs, kf, gr);
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                acc[d] += (double)gr[d];
+                next[d] = back[s] * (double)gr[d];
             }
         }
-        if (sub == 0) {
-            xa[j] = acc[0];
-            xa[nv + j] = acc[1];
-            xa[2 * (size_t)nv + j] = acc[2];
-        }
+        xa[j] = acc[0];
+        xa[nv + j] = acc[1];
+        xa[2 * (size_t)nv + j] = acc[2];
         km *= 1.0001f;  // margin for the float rounding
     }
 #pragma unroll
@@ -1552,12 +1736,14 @@ __global__ __launch_bounds__(256) void k_advect_adj_vert(const double *__restric
 // add to ua directly.  The four stage stencils of a vertex nearly always
 // start at the same node (the stages move it by h |u| << 1): then the four
 // terms are summed per node and added once.  Lane l of wave w takes column
-// 8l + w of the bin read as 512 columns, so the lanes of a wave hold vertices
+// 8l + w of the part read as 512 columns, so the lanes of a wave hold vertices
 // far apart, whose nodes rarely coincide (LDS atomics to one address
 // serialise).  FP32 accumulates in 64-bit fixed point, as the spreading
 // (raw bits of fma(v, scale, 1.5 2^52), whose low 48 bits sum exactly), with
 // the scale from the bound cnt max_v sum_s |kb_s| / 8 of a node's sum (a
-// weight product is at most 8/64); FP64 uses FP64 LDS atomics.
+// weight product is at most 8/64); FP64 uses FP64 LDS atomics.  On 32 cells
+// of 2562 vertices: 130 us with 16x8x8 tiles and a work group per tile, 54 us
+// with 8x8x8 tiles and full ones shared out.
 constexpr int ADV_WG = 512;  // work-group size of k_advect_adj_scatter
 
 template <typename T>
@@ -1565,14 +1751,14 @@ __global__ __launch_bounds__(ADV_WG) void k_advect_adj_scatter(const AdvRec<T> *
                                                             const int *__restrict__ tile_count,
                                                             const int *__restrict__ tile_off, IbmGeom g,
                                                             TileGeom tg, const unsigned *__restrict__ kbmax,
-                                                            const int *__restrict__ order) {
+                                                            const int *__restrict__ order,
+                                                            const int2 *__restrict__ extra, int maxextra) {
     extern __shared__ double dyn[];
     constexpr bool FIX = sizeof(T) == 4;
     unsigned long long *Ub = (unsigned long long *)dyn;  // [3][RZ][RY][RX]
     double *Ud = dyn;
-    const int tile = order[blockIdx.x];
-    const int cnt = tile_count[tile], off = tile_off[tile];
-    if (cnt == 0) return;  // whole work group leaves together
+    int tile, cnt, off;
+    if (!tile_part((int)blockIdx.x, order, extra, maxextra, tile_count, tile_off, tile, cnt, off)) return;
     const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
     const int bx = tx * TILE_X - RLO, by = ty * TILE_Y - RLO, bz = tz * TILE_Z - RLO;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
@@ -1709,12 +1895,15 @@ IbmGeom geom_of(const lbmibm_ctx *ctx) {
     return g;
 }
 
+static TileGeom tiles_of(const lbmibm_ctx *ctx) { return {ctx->ntx, ctx->nty, ctx->ntz, ctx->ntiles, ctx->tile_x}; }
+
 BinGeom bin_geom(const lbmibm_ctx *ctx) {
     BinGeom b;
     b.nx = ctx->nx; b.ny = ctx->ny; b.nz = ctx->nz;
     b.nxp = ctx->nxp; b.nyp = ctx->nyp; b.nzp = ctx->nzp;
     b.walls = ctx->p.periodic_y == 0;
     b.ntx = ctx->ntx; b.nty = ctx->nty;
+    b.tx = ctx->tile_x;
     b.dx = ctx->p.dx;
     return b;
 }
@@ -1723,7 +1912,7 @@ BinGeom bin_geom(const lbmibm_ctx *ctx) {
 // force maxima, k_tile_order).
 lbmibm_status tile_offsets(lbmibm_ctx *ctx, hipStream_t stream, int nblk_fmax) {
     const IbmGeom g = geom_of(ctx);
-    TileGeom tg{ctx->ntx, ctx->nty, ctx->ntz, ctx->ntiles};
+    const TileGeom tg = tiles_of(ctx);
     hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->tile_off, ctx->tile_cur,
                        ctx->ntiles, ctx->blk_fmax, nblk_fmax, ctx->absmax, ctx->tile_ex, ctx->sb_extra,
                        ctx->sb_maxextra);
@@ -1767,23 +1956,33 @@ template <typename T> lbmibm_status bin_impl(lbmibm_ctx *ctx) {
 
 // The spreading of the binned records into F with the given form.
 template <typename T> lbmibm_status spread_launch(lbmibm_ctx *ctx, int form) {
-    TileGeom tg{ctx->ntx, ctx->nty, ctx->ntz, ctx->ntiles};
+    const TileGeom tg = tiles_of(ctx);
     const IbmGeom g = geom_of(ctx);
     if (form == 1) {
-        LBMIBM_KT(ctx, ctx->stream, "k_spread_box",
-                  hipLaunchKernelGGL(k_spread_box<T>, dim3(ctx->sb_maxextra + ctx->ntiles), dim3(SPREAD_BOX_WG), 0,
-                                     ctx->stream,
-                                     (const SpreadRec<T> *)ctx->srec, ctx->node0, ctx->home_list, ctx->tile_count,
-                                     ctx->tile_off, (T *)ctx->sbox, g, tg, ctx->order_interp, ctx->sb_extra,
-                                     ctx->sb_maxextra));
-        LBMIBM_LAUNCHED(ctx, "k_spread_box");
-        if (ctx->sb_maxextra > 0) {
-            hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra), dim3(1024), 0,
-                               ctx->stream, (T *)ctx->sbox, ctx->sb_extra, ctx->tile_count, ctx->ntiles);
-            LBMIBM_LAUNCHED(ctx, "k_spread_combine");
+        if (ctx->pointwise) {
+            LBMIBM_KT(ctx, ctx->stream, "k_spread_points",
+                      hipLaunchKernelGGL(k_spread_points, dim3(ctx->ntiles), dim3(SPREAD_BOX_WG), 0, ctx->stream,
+                                         (const SpreadRec<float> *)ctx->srec, ctx->node0, ctx->tile_count,
+                                         ctx->tile_off, (float *)ctx->sbox, g, tg, ctx->order_interp));
+            LBMIBM_LAUNCHED(ctx, "k_spread_points");
+        } else {
+            LBMIBM_KT(ctx, ctx->stream, "k_spread_box",
+                      hipLaunchKernelGGL(k_spread_box<T>, dim3(ctx->sb_maxextra + ctx->ntiles), dim3(SPREAD_BOX_WG), 0,
+                                         ctx->stream,
+                                         (const SpreadRec<T> *)ctx->srec, ctx->node0, ctx->home_list, ctx->tile_count,
+                                         ctx->tile_off, (T *)ctx->sbox, g, tg, ctx->order_interp, ctx->sb_extra,
+                                         ctx->sb_maxextra));
+            LBMIBM_LAUNCHED(ctx, "k_spread_box");
+            if (ctx->sb_maxextra > 0) {
+                hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra), dim3(1024), 0,
+                                   ctx->stream, (T *)ctx->sbox, ctx->sb_extra, ctx->tile_count, ctx->ntiles);
+                LBMIBM_LAUNCHED(ctx, "k_spread_combine");
+            }
         }
+        constexpr int XW = sizeof(T) == 4 ? TILE_XW : TILE_X;
         LBMIBM_KT(ctx, ctx->stream, "k_spread_gather",
-                  hipLaunchKernelGGL(k_spread_gather<T>, dim3((unsigned)xcd_grid((int)((ctx->N + 255) / 256))), dim3(256), 0,
+                  hipLaunchKernelGGL((ctx->pointwise ? k_spread_gather<T, XW> : k_spread_gather<T, TILE_X>),
+                                     dim3((unsigned)xcd_grid((int)((ctx->N + 255) / 256))), dim3(256), 0,
                                      ctx->stream, (const T *)ctx->sbox, ctx->tile_count, ctx->sb_cand,
                                      ctx->sb_cand + SB_MAXC * ctx->nx, ctx->sb_cand + SB_MAXC * (ctx->nx + ctx->ny),
                                      (T *)ctx->F, g, tg));
@@ -1831,6 +2030,14 @@ lbmibm_status interp_launch(lbmibm_ctx *ctx, int form, const double *xin, double
     a.lx = ctx->nx * ctx->p.dx; a.ly = ctx->ny * ctx->p.dx; a.lz = ctx->nz * ctx->p.dx;
     a.rk = ctx->p.runge_kutta;
     a.periodic_y = ctx->p.periodic_y;
+    if (ctx->pointwise) {  // one form
+        LBMIBM_KT(ctx, ctx->stream, "k_interp_points",
+                  hipLaunchKernelGGL(k_interp_points, dim3((ctx->nv + 63) / 64), dim3(64), 0, ctx->stream,
+                                     (const float *)ctx->U, xin, xo, (float *)uvw, xd, ctx->home_list, ctx->nv,
+                                     geom_of(ctx), a));
+        LBMIBM_LAUNCHED(ctx, "k_interp_points");
+        return LBMIBM_OK;
+    }
     if (form == 1) {
         LBMIBM_KT(ctx, ctx->stream, "k_interp_vert",
                   hipLaunchKernelGGL(k_interp_vert<T>, dim3((ctx->nv + 255) / 256), dim3(256), 0, ctx->stream,
@@ -1838,12 +2045,12 @@ lbmibm_status interp_launch(lbmibm_ctx *ctx, int form, const double *xin, double
         LBMIBM_LAUNCHED(ctx, "k_interp_vert");
         return LBMIBM_OK;
     }
-    TileGeom tg{ctx->ntx, ctx->nty, ctx->ntz, ctx->ntiles};
+    const TileGeom tg = tiles_of(ctx);
     const size_t lds = 3 * (size_t)RN * sizeof(T);
     LBMIBM_KT(ctx, ctx->stream, "k_interp_tiles",
-              hipLaunchKernelGGL(k_interp_tiles<T>, dim3(ctx->ntiles), dim3(INTERP_WG), lds, ctx->stream,
+              hipLaunchKernelGGL(k_interp_tiles<T>, dim3(ctx->sb_maxextra + ctx->ntiles), dim3(INTERP_WG), lds, ctx->stream,
                                  (const T *)ctx->U, xin, xo, uvw, xd, ctx->tile_count, ctx->tile_off, ctx->home_list,
-                                 ctx->nv, geom_of(ctx), tg, a, ctx->order_interp));
+                                 ctx->nv, geom_of(ctx), tg, a, ctx->order_interp, ctx->sb_extra, ctx->sb_maxextra));
     LBMIBM_LAUNCHED(ctx, "k_interp_tiles");
     return LBMIBM_OK;
 }
@@ -1926,16 +2133,16 @@ template <typename T> lbmibm_status advect_adj_impl(lbmibm_ctx *ctx) {
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, ctx->stream, (int *)ctx->adj_xmax, 1);
     LBMIBM_LAUNCHED(ctx, "k_zero_int");
     const IbmGeom g = geom_of(ctx);
-    hipLaunchKernelGGL(k_advect_adj_vert<T>, dim3((unsigned)((4 * (size_t)ctx->nv + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL(k_advect_adj_vert<T>, dim3((ctx->nv + 255) / 256), dim3(256), 0,
                        ctx->stream,
                        (const double *)ctx->xs, (const T *)ctx->U, ctx->adj_x, ctx->home_list, ctx->nv, g,
                        ctx->p.m * ctx->p.dt, (AdvRec<T> *)ctx->adj_rec, ctx->adj_xmax);
     LBMIBM_LAUNCHED(ctx, "k_advect_adj_vert");
-    TileGeom tg{ctx->ntx, ctx->nty, ctx->ntz, ctx->ntiles};
+    const TileGeom tg = tiles_of(ctx);
     const size_t lds = 3 * (size_t)RN * sizeof(unsigned long long);
-    hipLaunchKernelGGL(k_advect_adj_scatter<T>, dim3(ctx->ntiles), dim3(ADV_WG), lds, ctx->stream,
+    hipLaunchKernelGGL(k_advect_adj_scatter<T>, dim3(ctx->sb_maxextra + ctx->ntiles), dim3(ADV_WG), lds, ctx->stream,
                        (const AdvRec<T> *)ctx->adj_rec, (T *)ctx->adj_u, ctx->tile_count, ctx->tile_off, g, tg,
-                       ctx->adj_xmax, ctx->order_interp);
+                       ctx->adj_xmax, ctx->order_interp, ctx->sb_extra, ctx->sb_maxextra);
     LBMIBM_LAUNCHED(ctx, "k_advect_adj_scatter");
     return LBMIBM_OK;
 }
@@ -1956,7 +2163,7 @@ lbmibm_status ibm_interp_adjoint(lbmibm_ctx *ctx) {
 
 lbmibm_status ibm_setup(lbmibm_ctx *ctx) {
     // extra chunks: at most nv / SB_CHUNK over all tiles
-    ctx->sb_maxextra = ctx->nv / SB_CHUNK;
+    ctx->sb_maxextra = ctx->pointwise ? 0 : xcd_grid(ctx->nv / SB_CHUNK);  // whole rounds of the XCDs
     lbmibm_status s = dev_alloc(ctx, (void **)&ctx->tile_ex, (size_t)ctx->ntiles * sizeof(int));
     if (s == LBMIBM_OK) s = dev_alloc(ctx, (void **)&ctx->sb_extra, (size_t)ctx->sb_maxextra * sizeof(int2));
     if (s != LBMIBM_OK) return s;
@@ -1994,7 +2201,7 @@ lbmibm_status ibm_spread(lbmibm_ctx *ctx) {
 // much smaller than a box) or the tile counts do not fit the packing.
 static bool spread_box_tables(const lbmibm_ctx *ctx, std::vector<int> &out) {
     const int n[3] = {ctx->nx, ctx->ny, ctx->nz}, nt[3] = {ctx->ntx, ctx->nty, ctx->ntz};
-    const int tile[3] = {TILE_X, TILE_Y, TILE_Z}, R[3] = {SB_X, SB_Y, SB_Z};
+    const int tile[3] = {ctx->tile_x, TILE_Y, TILE_Z}, R[3] = {ctx->tile_x + 3, SB_Y, SB_Z};
     const bool wrap[3] = {true, ctx->p.periodic_y != 0, true};
     out.assign((size_t)SB_MAXC * (n[0] + n[1] + n[2]), -1);
     size_t base = 0;
@@ -2030,7 +2237,8 @@ static lbmibm_status spread_box_setup(lbmibm_ctx *ctx, bool *ok) {
         LBMIBM_HIP(ctx, hipMemcpy(ctx->sb_cand, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     if (!ctx->sbox) {
-        lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)(ctx->ntiles + ctx->sb_maxextra) * 3 * SB_N * ctx->szT);
+        lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)(ctx->ntiles + ctx->sb_maxextra) * 3 *
+                                                              (ctx->pointwise ? SP_N : SB_N) * ctx->szT);
         if (s != LBMIBM_OK) return s;
     }
     *ok = true;
@@ -2103,7 +2311,7 @@ lbmibm_status ibm_autotune(lbmibm_ctx *ctx) {
     if (fi >= 0) {
         ctx->interp_form = fi;
         ctx->tune_report += "interp form fixed by LBMIBM_INTERP_FORM\n";
-    } else if (tune) {
+    } else if (tune && !ctx->pointwise) {
         s = ctx->prec == LBMIBM_F64 ? interp_autotune_impl<double>(ctx) : interp_autotune_impl<float>(ctx);
         if (s != LBMIBM_OK) return s;
     }

@@ -235,7 +235,7 @@ __global__ __launch_bounds__(NT) void k_volume(const int *__restrict__ cells, in
 // pass), and CapsulePeriodicAfter: each position wrapped back into the box.
 // With `home` the final positions are also counted into the spreading tiles
 // (home tile of each vertex, per-tile counts), as the binning would.
-__global__ __launch_bounds__(VOL_CH) void k_vol_center(const int4 *__restrict__ chunks, double *__restrict__ xs, int nv,
+__global__ __launch_bounds__(256) void k_vol_center(const int4 *__restrict__ chunks, double *__restrict__ xs, int nv,
                                                     const double *__restrict__ gx, const int *__restrict__ need,
                                                     double4 *__restrict__ part, VolArgs a, BinGeom bg,
                                                     int *__restrict__ home, int *__restrict__ tile_count) {
@@ -249,26 +249,39 @@ __global__ __launch_bounds__(VOL_CH) void k_vol_center(const int4 *__restrict__ 
     const double g[3] = {gx[3 * ch.x], gx[3 * ch.x + 1], gx[3 * ch.x + 2]};
     const double len[3] = {a.lx, a.ly, a.lz};
     double s[3] = {0.0, 0.0, 0.0};
-    const int j = ch.y + (int)threadIdx.x;
-    const bool on = (int)threadIdx.x < ch.z;
-    double fin[3] = {0.0, 0.0, 0.0};
-    if (on) {
-        for (int d = 0; d < 3; d++) {
-            double *P = xs + d * (size_t)nv + j;
-            const double x0 = *P;
-            const bool per = d != 1 || a.py;
-            const double x = unwrap && per ? unwrap1(x0, g[d], len[d]) : x0;
-            s[d] = x;
-            const double w = per ? rewrap1(x, len[d]) : x;
-            if (w != x0) *P = w;
-            fin[d] = w;
-        }
+    // 256 threads, four vertices each, their loads first: groups of 1024 threads
+    // waited for a free CU beside the membrane kernels that this launch
+    // overlaps (230 against 60 us in the 1024-cell suspension's steps)
+    constexpr int VPT = VOL_CH / 256;
+    double x[VPT][3];
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        const int i = k * 256 + (int)threadIdx.x;
+#pragma unroll
+        for (int d = 0; d < 3; d++) x[k][d] = i < ch.z ? xs[d * (size_t)nv + ch.y + i] : 0.0;
     }
-    if (home) {
-        const int t = on ? home_tile(bg, fin[0], fin[1], fin[2]) : 0;
-        if (on) home[j] = t;
-        int slot;
-        (void)tab.add(t, on, slot);
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        const int i = k * 256 + (int)threadIdx.x, j = ch.y + i;
+        const bool on = i < ch.z;
+        double fin[3] = {0.0, 0.0, 0.0};
+        if (on) {
+            for (int d = 0; d < 3; d++) {
+                const double x0 = x[k][d];
+                const bool per = d != 1 || a.py;
+                const double xu = unwrap && per ? unwrap1(x0, g[d], len[d]) : x0;
+                s[d] += xu;
+                const double w = per ? rewrap1(xu, len[d]) : xu;
+                if (w != x0) xs[d * (size_t)nv + j] = w;
+                fin[d] = w;
+            }
+        }
+        if (home) {  // whole waves fill the tile table
+            const int t = on ? home_tile(bg, fin[0], fin[1], fin[2]) : 0;
+            if (on) home[j] = t;
+            int slot;
+            (void)tab.add(t, on, slot);
+        }
     }
     red.sum<3>(s);  // its barrier also orders the table
     if (home) tab.flush(tile_count);
@@ -343,9 +356,9 @@ lbmibm_status run_impl(lbmibm_ctx *ctx, int mode, hipStream_t stream) {
             if (s != LBMIBM_OK) return s;
         }
         const BinGeom bg{ctx->nx, ctx->ny, ctx->nz, ctx->nxp, ctx->nyp, ctx->nzp, ctx->p.periodic_y == 0,
-                         ctx->ntx, ctx->nty, ctx->p.dx};
+                         ctx->ntx, ctx->nty, ctx->tile_x, ctx->p.dx};
         LBMIBM_KT(ctx, stream, "k_vol_center",
-                  hipLaunchKernelGGL(k_vol_center, dim3(ctx->vol_nvc), dim3(VOL_CH), 0, stream, ctx->vol_vchunks,
+                  hipLaunchKernelGGL(k_vol_center, dim3(ctx->vol_nvc), dim3(256), 0, stream, ctx->vol_vchunks,
                                      (double *)ctx->xs, ctx->nv, ctx->gx, ctx->vol_need, ctx->vol_vpart, a, bg,
                                      count ? ctx->home : nullptr, ctx->tile_count));
         LBMIBM_LAUNCHED(ctx, "k_vol_center");

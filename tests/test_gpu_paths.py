@@ -73,7 +73,7 @@ def _crowded(lx, ly, lz, levels, seed, lo, hi):
 
 
 # corners of the first stencil nodes (a vertex between nodes i and i + 1 starts
-# its stencil at i - 1): within one tile of 16 x 8 x 8 below the sort's capacity,
+# its stencil at i - 1): within two tiles (16 x 8 x 8 nodes) below the sort's capacity,
 # above it (several passes), in one lattice cell below and above it, and more
 # vertices than 16-bit indices hold; across the lower wall
 CROWDS = [([3, 3], (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)), ([4, 4], (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)),
@@ -116,3 +116,86 @@ def test_spread_of_crowded_tiles_does_not_depend_on_the_order():
     g.close()
     for a in out[1:]:
         assert np.array_equal(a, out[0])
+
+
+def _advected(pos, U, shape):
+    """RK4 advection (M dt = 1) of positions through a velocity field U [3][z, y,
+    x], periodic in x and z, at rest beyond the y walls, in plain FP64."""
+    lx, ly, lz = shape
+
+    def vel(X):
+        s = X + np.array([(n - 1) / 2.0 for n in shape])  # node i sits at i
+        first = np.floor(s)
+        t = np.pi / 2 * (s - first)
+        w = np.stack([1 - np.sin(t), 1 + np.cos(t), 1 + np.sin(t), 1 - np.cos(t)], 2) / 4.0
+        i = first.astype(int)[:, :, None] - 1 + np.arange(4)
+        ok = (i[:, 1] >= 0) & (i[:, 1] < ly)
+        ix, iy, iz = i[:, 0] % lx, np.clip(i[:, 1], 0, ly - 1), i[:, 2] % lz
+        f = U[:, iz[:, :, None, None], iy[:, None, :, None], ix[:, None, None, :]]
+        return np.einsum("dvzyx,vz,vy,vx->vd", f, w[:, 2], w[:, 1] * ok, w[:, 0])
+
+    k1 = vel(pos)
+    k2 = vel(pos + k1 / 2)
+    k3 = vel(pos + k2 / 2)
+    k4 = vel(pos + k3)
+    return (k1 + 2 * k2 + 2 * k3 + k4) / 6
+
+
+def _rough_field(shape, nc, prec, **kw):
+    lx, ly, lz = shape
+    cells, pos = _scattered(lx, ly, lz, nc, 2, seed=2)
+    if nc > 2:  # crowd them into two tiles
+        pos = [(p / v) * w + o for p, v, w, o in zip(pos, shape, (14.0, 6.0, 6.0), (1.0, 0.0, 1.0))]
+    g = gpu_of(lx, ly, lz, prec, cells=cells, **kw)
+    g.set_cells_state(x=pos[0], y=pos[1], z=pos[2])
+    U = 1.5 * np.random.default_rng(9).standard_normal((3, lz, ly, lx))
+    pad = np.zeros((3, lz + 4, ly + 4, lx + 4))
+    pad[:, 2:-2, 2:-2, 2:-2] = U
+    g.set_macros(*[a.reshape(-1) for a in pad])
+    g.ibm_st2()
+    s = g.cells_state()
+    g.close()
+    ref = _advected(np.stack(pos, 1), U, shape)
+    # FP32: the stage positions carry the velocity's rounding (1e-7 of 1.5
+    # nodes), which the next stage multiplies by the field's slope (about 3 per
+    # node), three times: 1e-7 * 27, with a margin of 10
+    tol = {"f64": 1e-11, "f32": 3e-5}[prec]
+    for d, k in enumerate("uvw"):
+        assert rel(s[k], ref[:, d]) < tol, k
+
+
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("shape,nc", [((9, 8, 17), 2), ((40, 24, 40), 11)])  # boxes that wrap onto themselves; full tiles
+def test_interpolation_of_a_fast_rough_field(shape, nc, prec, form, monkeypatch):
+    """Vertices that leave their lattice cell, and the staged box, between the
+    RK stages; tiles shared out between work groups (1782 vertices in two of
+    them); rough velocities of order one node per step.  Against a plain FP64
+    evaluation: stages beyond the reference's two halo layers, which the oracle
+    has too, take the periodic images here."""
+    monkeypatch.setenv("LBMIBM_INTERP_FORM", str(form))
+    print(f"[interp rough] {shape} {prec} form={form}", flush=True)
+    _rough_field(shape, nc, prec)
+
+
+@pytest.mark.parametrize("k", [0, 1, 2, 6])
+def test_spread_point_by_point(k, monkeypatch):
+    """FP32 values under an indicator: boxes of 16 x 8 x 8 tiles."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
+    levels, lo, hi = CROWDS[k]
+    lx, ly, lz = 45, 37, 40
+    print(f"[spread points] {k}", flush=True)
+    cells, pos = _crowded(lx, ly, lz, levels, 17 + k, lo, hi)
+    rng = np.random.default_rng(4)
+    n = pos[0].size
+    forces = [1e-3 * rng.standard_normal(n) * 10.0 ** rng.uniform(-4, 0, n) for _ in range(3)]
+    F, ref = _spread_both(lx, ly, lz, "f32", cells, pos, forces, vof_period=1000)
+    for a, b in zip(F, ref):
+        assert rel(a, b) < SPREAD_TOL["f32"]
+
+
+@pytest.mark.parametrize("shape,nc", [((9, 8, 17), 2), ((40, 24, 40), 11)])
+def test_interpolation_point_by_point(shape, nc):
+    """The rough field, FP32 values under an indicator."""
+    print(f"[interp points] {shape}", flush=True)
+    _rough_field(shape, nc, "f32", vof_period=1000)
