@@ -199,24 +199,10 @@ lbmibm_status adj_lattice(lbmibm_ctx *ctx, int iter) {
 
 // Padded [n] field <-> [3][N] device array of a given element size.
 lbmibm_status field_get(lbmibm_ctx *ctx, const void *src, bool dbl, double *out) {
-    const long long N = ctx->N;
-    std::vector<double> a(3 * (size_t)N);
-    if (dbl) {
-        LBMIBM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        LBMIBM_HIP(ctx, hipMemcpy(a.data(), src, 3 * (size_t)N * 8, hipMemcpyDeviceToHost));
-    } else {
-        lbmibm_status s = get_T(ctx, a.data(), src, 3 * (size_t)N);
-        if (s != LBMIBM_OK) return s;
-    }
-    std::fill(out, out + 3 * ctx->np, 0.0);
-    for (int iz = 0; iz < ctx->nz; iz++)
-        for (int iy = 0; iy < ctx->ny; iy++)
-            for (int ix = 0; ix < ctx->nx; ix++) {
-                const long long i = ix + (long long)ctx->nx * (iy + (long long)ctx->ny * iz);
-                const long long pi = padded_index(ctx, ix, iy, iz);
-                for (int d = 0; d < 3; d++) out[d * ctx->np + pi] = a[d * N + i];
-            }
-    return LBMIBM_OK;
+    const size_t elem = dbl ? 8 : ctx->szT, fN = (size_t)ctx->N * elem;
+    FieldOut f[3];
+    for (int d = 0; d < 3; d++) f[d] = {(const char *)src + d * fN, out + d * ctx->np};
+    return download_fields(ctx, f, 3, elem, false, true);
 }
 
 lbmibm_status field_set(lbmibm_ctx *ctx, void *dst, bool dbl, const double *in) {

@@ -276,6 +276,7 @@ void free_all(lbmibm_ctx *ctx) {
                     ctx->adh_fadh, ctx->adh_fsum, ctx->adh_nprop, ctx->adh_klist, ctx->adh_calls, ctx->adh_ring, ctx->mw};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    staging_free(ctx);
     if (ctx->graph) (void)hipGraphExecDestroy(ctx->graph);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
@@ -393,6 +394,7 @@ lbmibm_status lbmibm_create(const lbmibm_params *p, const lbmibm_cells *cells, l
         if (s_ != LBMIBM_OK) return fail(s_);    \
     } while (0)
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) return fail(LBMIBM_ERR_HIP);
+    if (staging_init(ctx) != LBMIBM_OK) return fail(LBMIBM_ERR_HIP);
     if (hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess) return fail(LBMIBM_ERR_HIP);
     if (hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess) return fail(LBMIBM_ERR_HIP);
     if (hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess) return fail(LBMIBM_ERR_HIP);
@@ -885,20 +887,12 @@ lbmibm_status lbmibm_thinc_wlic(lbmibm_ctx *ctx) {
 
 lbmibm_status lbmibm_download_vf(lbmibm_ctx *ctx, double *vf) {
     if (!ctx || !vf) return LBMIBM_ERR_ARG;
-    const long long N = ctx->N;
-    std::vector<double> v((size_t)N, 0.0);
-    if (ctx->vof[0]) {
-        LBMIBM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        LBMIBM_HIP(ctx, hipMemcpy(v.data(), ctx->vof[ctx->vof_cur], N * sizeof(double), hipMemcpyDeviceToHost));
+    if (!ctx->vof[0]) {
+        std::fill(vf, vf + ctx->np, 0.0);
+        return LBMIBM_OK;
     }
-    for (int pz = 0; pz < ctx->nzp; pz++)
-        for (int py = 0; py < ctx->nyp; py++)
-            for (int px = 0; px < ctx->nxp; px++) {
-                bool comp;
-                const long long i = padded_image(ctx, px, py, pz, comp);
-                vf[px + (long long)ctx->nxp * (py + (long long)ctx->nyp * pz)] = i < 0 ? 0.0 : v[i];
-            }
-    return LBMIBM_OK;
+    const FieldOut out{ctx->vof[ctx->vof_cur], vf};
+    return download_fields(ctx, &out, 1, sizeof(double), true, true);
 }
 
 lbmibm_status lbmibm_upload_vf(lbmibm_ctx *ctx, const double *vf) {
@@ -1160,33 +1154,12 @@ lbmibm_status lbmibm_download_macros(lbmibm_ctx *ctx, double *dn, double *un, do
         ctx->err = "dn/un/vn/wn/dm need store_macros=1";
         return LBMIBM_ERR_STATE;
     }
-    const long long N = ctx->N;
-    std::vector<double> U(3 * (size_t)N), Ui, R, RM;
-    lbmibm_status s = get_T(ctx, U.data(), ctx->U, 3 * (size_t)N);
-    if (s == LBMIBM_OK && ctx->p.store_macros) {
-        Ui.resize(3 * (size_t)N); R.resize(N); RM.resize(N);
-        s = get_T(ctx, Ui.data(), ctx->Ui, 3 * (size_t)N);
-        if (s == LBMIBM_OK) s = get_T(ctx, R.data(), ctx->rho, N);
-        if (s == LBMIBM_OK) s = get_T(ctx, RM.data(), ctx->rhom, N);
-    }
-    if (s != LBMIBM_OK) return s;
-    for (int pz = 0; pz < ctx->nzp; pz++)
-        for (int py = 0; py < ctx->nyp; py++)
-            for (int px = 0; px < ctx->nxp; px++) {
-                bool comp;
-                const long long i = padded_image(ctx, px, py, pz, comp);
-                if (i < 0) continue;
-                const long long pi = px + (long long)ctx->nxp * (py + (long long)ctx->nyp * pz);
-                if (um) um[pi] = U[i];
-                if (vm) vm[pi] = U[N + i];
-                if (wm) wm[pi] = U[2 * N + i];
-                if (dn) dn[pi] = R[i];
-                if (un) un[pi] = Ui[i];
-                if (vn) vn[pi] = Ui[N + i];
-                if (wn) wn[pi] = Ui[2 * N + i];
-                if (dm) dm[pi] = RM[i];
-            }
-    return LBMIBM_OK;
+    const size_t fN = (size_t)ctx->N * ctx->szT;
+    auto at = [&](const void *p, int d) { return p ? (const char *)p + d * fN : nullptr; };
+    const FieldOut out[8] = {{at(ctx->U, 0), um},  {at(ctx->U, 1), vm},  {at(ctx->U, 2), wm},
+                             {at(ctx->rho, 0), dn}, {at(ctx->Ui, 0), un}, {at(ctx->Ui, 1), vn},
+                             {at(ctx->Ui, 2), wn},  {at(ctx->rhom, 0), dm}};
+    return download_fields(ctx, out, 8, ctx->szT, true, false);
 }
 
 lbmibm_status lbmibm_upload_macros(lbmibm_ctx *ctx, const double *um, const double *vm, const double *wm) {
@@ -1206,20 +1179,10 @@ lbmibm_status lbmibm_upload_macros(lbmibm_ctx *ctx, const double *um, const doub
 
 lbmibm_status lbmibm_download_lattice_force(lbmibm_ctx *ctx, double *fx, double *fy, double *fz) {
     if (!ctx) return LBMIBM_ERR_ARG;
-    const long long N = ctx->N;
-    std::vector<double> F(3 * (size_t)N);
-    lbmibm_status s = get_T(ctx, F.data(), ctx->F, 3 * (size_t)N);
-    if (s != LBMIBM_OK) return s;
-    for (int iz = 0; iz < ctx->nz; iz++)
-        for (int iy = 0; iy < ctx->ny; iy++)
-            for (int ix = 0; ix < ctx->nx; ix++) {
-                const long long i = ix + (long long)ctx->nx * (iy + (long long)ctx->ny * iz);
-                const long long pi = padded_index(ctx, ix, iy, iz);
-                if (fx) fx[pi] = F[i];
-                if (fy) fy[pi] = F[N + i];
-                if (fz) fz[pi] = F[2 * N + i];
-            }
-    return LBMIBM_OK;
+    const size_t fN = (size_t)ctx->N * ctx->szT;
+    const char *F = (const char *)ctx->F;
+    const FieldOut out[3] = {{F, fx}, {F + fN, fy}, {F + 2 * fN, fz}};
+    return download_fields(ctx, out, 3, ctx->szT, false, false);
 }
 
 lbmibm_status lbmibm_upload_lattice_force(lbmibm_ctx *ctx, const double *fx, const double *fy, const double *fz) {
@@ -1246,23 +1209,16 @@ lbmibm_status lbmibm_download_cells(lbmibm_ctx *ctx, double *x, double *y, doubl
     if (!ctx) return LBMIBM_ERR_ARG;
     const size_t nv = ctx->nv;
     if (nv == 0) return LBMIBM_OK;
-    std::vector<double> a(3 * nv);
-    struct { void *src; bool dbl; double *d[3]; } sets[3] = {
-        {ctx->xs, true, {x, y, z}}, {ctx->uvw, false, {u, v, w}}, {ctx->cf, false, {fx, fy, fz}}};
-    LBMIBM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    for (auto &st : sets) {
-        if (!st.d[0] && !st.d[1] && !st.d[2]) continue;
-        if (st.dbl) {
-            LBMIBM_HIP(ctx, hipMemcpy(a.data(), st.src, 3 * nv * sizeof(double), hipMemcpyDeviceToHost));
-        } else {
-            lbmibm_status s = get_T(ctx, a.data(), st.src, 3 * nv);
-            if (s != LBMIBM_OK) return s;
-        }
-        for (int d = 0; d < 3; d++)
-            if (st.d[d]) std::copy(a.begin() + d * nv, a.begin() + (d + 1) * nv, st.d[d]);
+    struct { const void *src; size_t elem; double *d[3]; } sets[3] = {
+        {ctx->xs, 8, {x, y, z}}, {ctx->uvw, ctx->szT, {u, v, w}}, {ctx->cf, ctx->szT, {fx, fy, fz}}};
+    for (const auto &st : sets) {
+        FieldOut out[3];
+        for (int d = 0; d < 3; d++) out[d] = {(const char *)st.src + d * nv * st.elem, st.d[d]};
+        const lbmibm_status s = download_arrays(ctx, out, 3, st.elem, nv);
+        if (s != LBMIBM_OK) return s;
     }
-    if (xd) LBMIBM_HIP(ctx, hipMemcpy(xd, ctx->xd, 3 * nv * sizeof(double), hipMemcpyDeviceToHost));
-    return LBMIBM_OK;
+    const FieldOut all{ctx->xd, xd};
+    return download_arrays(ctx, &all, 1, 8, 3 * nv);
 }
 
 lbmibm_status lbmibm_upload_cells(lbmibm_ctx *ctx, const double *x, const double *y, const double *z,

@@ -4,7 +4,9 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -25,6 +27,8 @@ struct DevStep {
     double amp;
     double wall;
 };
+
+struct Staging;  // download.hip
 
 // Device status words, checked by the host after a synchronisation.
 struct DevStatus {
@@ -318,6 +322,10 @@ struct lbmibm_ctx {
     lbmibm::DevStep *step = nullptr;
     lbmibm::DevStatus *status = nullptr;
 
+    // ring of pinned buffers of the downloads (download.hip), and who uses it
+    lbmibm::Staging *staging = nullptr;
+    std::mutex staging_mutex;
+
     // whole-M-cycle graph
     hipGraphExec_t graph = nullptr;
     bool graph_ready = false;
@@ -346,6 +354,18 @@ lbmibm_status membrane_setup(lbmibm_ctx *ctx);               // membrane.hip
 lbmibm_status membrane_autotune(lbmibm_ctx *ctx);            // membrane.hip
 lbmibm_status ibm_autotune(lbmibm_ctx *ctx);                 // ibm.hip
 lbmibm_status volume_run(lbmibm_ctx *ctx, int mode);         // volume.hip (0 init, 1 correct)
+// A device array (compact lattice [N], or [n]) of `elem` bytes per value, 4
+// or 8, and the host array that takes it in FP64 (null: none).
+struct FieldOut {
+    const void *src;
+    double *dst;
+};
+// Lattice fields into padded host arrays: with the periodic images in the halo
+// or the fluid nodes alone, and with zeros or left as they are elsewhere.
+lbmibm_status download_fields(lbmibm_ctx *ctx, const FieldOut *out, int n, size_t elem, bool images, bool zero);  // download.hip
+lbmibm_status download_arrays(lbmibm_ctx *ctx, const FieldOut *out, int nout, size_t elem, size_t n);  // download.hip
+lbmibm_status staging_init(lbmibm_ctx *ctx);                 // download.hip
+void staging_free(lbmibm_ctx *ctx);                          // download.hip
 lbmibm_status vof_alloc(lbmibm_ctx *ctx);                    // vof.hip
 lbmibm_status vof_front_tracking(lbmibm_ctx *ctx, int *iterations, int *attempts);  // vof.hip (host sync)
 lbmibm_status vof_thinc(lbmibm_ctx *ctx);                    // vof.hip

@@ -199,3 +199,63 @@ def test_interpolation_point_by_point(shape, nc):
     """The rough field, FP32 values under an indicator."""
     print(f"[interp points] {shape}", flush=True)
     _rough_field(shape, nc, "f32", vof_period=1000)
+
+
+# several pieces of the ring in one plane, rows longer than a piece, helper
+# threads (above 8 MB in all), the smallest lattice; a tube
+FRAMES = [((4, 4, 4), {}), ((77, 46, 51), {}), ((77, 46, 51), {"periodic_y": True}), ((140001, 4, 4), {}),
+          ((160, 128, 130), {"periodic_y": True}), ((33, 34, 40), {"tube_radius": 14.0, "e": (0.0, 0.0, 1.0)})]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("k", range(len(FRAMES)))
+def test_downloads_fill_the_padded_frame(k, prec):
+    """Velocities with their periodic images, wall nodes left as they were; the
+    values are whole numbers, so equal to the last bit."""
+    from preprocess_src_amd import native
+    (lx, ly, lz), kw = FRAMES[k]
+    print(f"[frame] {lx}x{ly}x{lz} {kw} {prec}", flush=True)
+    g = gpu_of(lx, ly, lz, prec, store_macros=False, **kw)
+    rng = np.random.default_rng(k)
+    comp = rng.integers(1, 1 << 20, (3, lz, ly, lx)).astype(np.float64)
+    pad = np.zeros((3, lz + 4, ly + 4, lx + 4))
+    pad[:, 2:-2, 2:-2, 2:-2] = comp
+    g.set_macros(*[np.ascontiguousarray(a).reshape(-1) for a in pad])
+    want = np.full_like(pad, -7.0)
+    if "tube_radius" in kw:
+        want[:, :, 2:-2, 2:-2] = np.pad(comp, ((0, 0), (2, 2), (0, 0), (0, 0)), mode="wrap")
+        x, y = np.arange(lx + 4) - 1.5 - lx / 2.0, np.arange(ly + 4) - 1.5 - ly / 2.0
+        want[:, :, np.sqrt(x[None, :] ** 2 + y[:, None] ** 2) > kw["tube_radius"]] = -7.0
+    else:
+        wy = 2 if kw.get("periodic_y") else 0
+        want[:, :, 2 - wy:ly + 2 + wy] = np.pad(comp, ((0, 0), (2, 2), (wy, wy), (2, 2)), mode="wrap")
+    for order in ((0, 1, 2), (2,)):  # all, one alone
+        got = [np.full(g.np_, -7.0) for _ in range(3)]
+        native.check(g.L.lbmibm_download_macros(g.ctx, *([None] * 5),
+                                                *[native.dp(got[d]) if d in order else None for d in range(3)]), g.ctx)
+        for d in range(3):
+            assert np.array_equal(got[d].reshape(want[d].shape), want[d] if d in order else np.full_like(want[d], -7.0))
+    force = [np.full(g.np_, -7.0) for _ in range(3)]  # at rest: 0 on the fluid nodes alone
+    native.check(g.L.lbmibm_download_lattice_force(g.ctx, *map(native.dp, force)), g.ctx)
+    inner = np.full(want[0].shape, -7.0)
+    inner[2:-2, 2:-2, 2:-2] = 0.0
+    for f in force:
+        assert np.array_equal(f.reshape(inner.shape), inner)
+    g.close()
+
+
+def test_download_of_the_indicator_zeroes_the_walls():
+    from preprocess_src_amd import native
+    lx, ly, lz = 29, 18, 23
+    cells, _ = _scattered(lx, ly, lz, 1, 2, seed=1)
+    g = gpu_of(lx, ly, lz, "f32", cells=cells, vof_period=1000)
+    comp = np.random.default_rng(3).uniform(0, 1, (lz, ly, lx))
+    pad = np.zeros((lz + 4, ly + 4, lx + 4))
+    pad[2:-2, 2:-2, 2:-2] = comp
+    native.check(g.L.lbmibm_upload_vf(g.ctx, native.dp(np.ascontiguousarray(pad))), g.ctx)
+    got = np.full(g.np_, -7.0)
+    native.check(g.L.lbmibm_download_vf(g.ctx, native.dp(got)), g.ctx)
+    want = np.zeros_like(pad)
+    want[:, 2:-2] = np.pad(comp, ((2, 2), (0, 0), (2, 2)), mode="wrap")
+    g.close()
+    assert np.array_equal(got.reshape(want.shape), want)
