@@ -319,7 +319,8 @@ struct lbmibm_ctx {
     bool kt_on = false;
     std::vector<KtRec> kt_recs;
     void *adh_fsum = nullptr;
-    lbmibm::DevStep *step = nullptr;
+    lbmibm::DevStep *steps = nullptr;  // [0] the current step's values; [1..] those of a replayed block's steps
+    lbmibm::DevStep *step = nullptr;   // the entry that kernels are launched with
     lbmibm::DevStatus *status = nullptr;
 
     // ring of pinned buffers of the downloads (download.hip), and who uses it
