@@ -74,12 +74,12 @@ __device__ __forceinline__ unsigned long long bid_key(unsigned long long call, i
     return (stamp << 32) | (unsigned long long)(0xFFFFFFFFu - (unsigned)sid);
 }
 
-// Advances the call counter. Stamps must stay below 2^32 (the key keeps 32
+// Advances the call counter (one work group). Stamps must stay below 2^32 (the key keeps 32
 // bits of stamp): when the next call's largest stamp would not, every claim
 // is cleared and the counter restarts at 0, whose stamps outrank a cleared
 // claim. With MAXN = 100 that happens once in about 42 million calls.
-__global__ void __launch_bounds__(256) k_adh_tick(unsigned long long *__restrict__ calls,
-                                                  unsigned long long *__restrict__ claim, long long nrec, int maxn) {
+__device__ __forceinline__ void advance_calls(unsigned long long *__restrict__ calls,
+                                              unsigned long long *__restrict__ claim, long long nrec, int maxn) {
     const unsigned long long next = calls[0] + 1ull;
     const bool wrap = (next + 1ull) * (unsigned long long)(maxn + 2) > 0xFFFFFFFFull;
     if (wrap)
@@ -168,19 +168,27 @@ __global__ __launch_bounds__(AWG) void k_adh_force(AdhDev a, const double *__res
 
 // StoreNeighWall_CUBE_GPU (adhesion.cu:109-206): receptors within LIMIT dx
 // of a knob near the wall, nearest first, ties in scan order, at most MAXN.
+// One wave per knob: its lanes test the candidates 64 at a time, list those in
+// range in scan order in LDS, and count for each one how many come before it.
+// One lane per vertex, inserting into a sorted list in memory, was a chain of
+// dependent reads for each candidate: 63 us for 64 cells with 20 to 40 knobs
+// each, 5 us now.
+constexpr int SEARCH_CAP = 192;  // receptors in range held in LDS per knob; more take the sorted insertion by one lane
 __global__ __launch_bounds__(AWG) void k_adh_search(AdhDev a, const double *__restrict__ xs,
-                                                    const unsigned char *__restrict__ knob, int *__restrict__ id_wall,
+                                                    const int *__restrict__ klist, int nk, int *__restrict__ id_wall,
                                                     double *__restrict__ r_wall) {
 #pragma clang fp contract(off)
-    const int v = blockIdx.x * AWG + threadIdx.x;
-    if (v >= a.nv || !knob[v]) return;  // other vertices keep the lists set up empty
+    __shared__ double lr[AWG / 64][SEARCH_CAP];
+    __shared__ int lid[AWG / 64][SEARCH_CAP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t = blockIdx.x * (AWG / 64) + wave;
+    if (t >= nk) return;  // whole waves leave; nothing here waits for another wave
+    const int v = klist[t];
     int *ids = id_wall + (size_t)v * a.maxn;
     double *rs = r_wall + (size_t)v * a.maxn;
-    for (int k = 0; k < a.maxn; k++) { ids[k] = -1; rs[k] = 1.0e15; }
     const double xi = xs[v], yi = xs[a.nv + v], zi = xs[2 * (size_t)a.nv + v];
-    if (a.ring ? sqrt(xi * xi + yi * yi) < a.radius - a.limit * a.dx  // adhesion.cu:248-249
-               : sqrt(yi * yi) < 0.5 * a.ly - a.limit * a.dx)
-        return;
+    const bool away = a.ring ? sqrt(xi * xi + yi * yi) < a.radius - a.limit * a.dx  // adhesion.cu:248-249
+                             : sqrt(yi * yi) < 0.5 * a.ly - a.limit * a.dx;
     const int iz = (int)((zi - (-a.lz / 2.0)) / a.dzw);
     const int span = a.limit * (int)(a.dx / a.dzw);
     // Only columns within LIMIT dx can pass the range test: an x window on
@@ -200,26 +208,56 @@ __global__ __launch_bounds__(AWG) void k_adh_search(AdhDev a, const double *__re
         ra0 = max(0, (int)floor((xi - a.limit * a.dx) / a.dxw) + a.nxw / 2 - 1);
         ra1 = min(a.nxw - 1, (int)ceil((xi + a.limit * a.dx) / a.dxw) + a.nxw / 2 + 1);
     }
-    int cnt = 0;
-    for (int i = 0; i < 2 * span; i++) {
-        int jz = iz + i - (span - 1);
+    const int ncol = ra1 - ra0 + 1 + (rb1 - rb0 + 1);
+    const long long total = away || ncol <= 0 || span <= 0 ? 0 : 2LL * span * ncol;
+    // candidate n in scan order; false out of range
+    auto candidate = [&](long long n, int &id, double &r) {
+        int jz = iz + (int)(n / ncol) - (span - 1);
         double zj = (jz - a.nzw / 2) * a.dzw;
         if (jz < 0) { jz += a.nzw; zj += a.lz; }
         else if (jz >= a.nzw) { jz -= a.nzw; zj -= a.lz; }
-        for (int k = ra0, kend = ra1 + (rb1 - rb0 + 1); k <= kend; k++) {
-            const int jx = k <= ra1 ? k : rb0 + (k - ra1 - 1);
-            const int id = jz * a.nxw + jx;
-            double xj, yj, zr;
-            receptor(a, id, xj, yj, zr);
-            const double r = sqrt((xj - xi) * (xj - xi) + (yj - yi) * (yj - yi) + (zj - zi) * (zj - zi));
-            if (r > a.limit * a.dx) continue;
-            int pos = cnt < a.maxn ? cnt : a.maxn;
+        const int k = ra0 + (int)(n % ncol), jx = k <= ra1 ? k : rb0 + (k - ra1 - 1);
+        id = jz * a.nxw + jx;
+        double xj, yj, zr;
+        receptor(a, id, xj, yj, zr);
+        r = sqrt((xj - xi) * (xj - xi) + (yj - yi) * (yj - yi) + (zj - zi) * (zj - zi));
+        return !(r > a.limit * a.dx);
+    };
+    long long cnt = 0;
+    for (long long n0 = 0; n0 < total; n0 += 64) {
+        int id = 0;
+        double r = 0.0;
+        const bool in = n0 + lane < total && candidate(n0 + lane, id, r);
+        const unsigned long long m = __ballot(in);
+        const long long at = cnt + __popcll(m & ((1ull << lane) - 1ull));
+        if (in && at < SEARCH_CAP) { lr[wave][at] = r; lid[wave][at] = id; }
+        cnt += __popcll(m);
+    }
+    const int kept = (int)min(cnt, (long long)a.maxn);
+    for (int k = kept + lane; k < a.maxn; k += 64) { ids[k] = -1; rs[k] = 1.0e15; }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (cnt <= SEARCH_CAP) {
+        for (int i = lane; i < (int)cnt; i += 64) {
+            const double r = lr[wave][i];
+            int rank = 0;
+            for (int j = 0; j < (int)cnt; j++) rank += j < i ? !(lr[wave][j] > r) : r > lr[wave][j];
+            if (rank < a.maxn) { ids[rank] = lid[wave][i]; rs[rank] = r; }
+        }
+    } else if (lane == 0) {
+        int have = 0;
+        for (long long n = 0; n < total; n++) {
+            int id;
+            double r;
+            if (!candidate(n, id, r)) continue;
+            int pos = have;
             while (pos > 0 && rs[pos - 1] > r) pos--;
             if (pos >= a.maxn) continue;
-            for (int k = (cnt < a.maxn ? cnt : a.maxn - 1); k > pos; k--) { ids[k] = ids[k - 1]; rs[k] = rs[k - 1]; }
+            for (int k = have < a.maxn ? have : a.maxn - 1; k > pos; k--) { ids[k] = ids[k - 1]; rs[k] = rs[k - 1]; }
             ids[pos] = id;
             rs[pos] = r;
-            if (cnt < a.maxn) cnt++;
+            if (have < a.maxn) have++;
         }
     }
 }
@@ -231,8 +269,11 @@ __global__ __launch_bounds__(AWG) void k_adh_detach(AdhDev a, const double *__re
                                                     double *__restrict__ r_ij, int *__restrict__ is_attached,
                                                     int *__restrict__ pos, int *__restrict__ active,
                                                     const DevStep *__restrict__ st, int init,
-                                                    const int *__restrict__ klist, int nk) {
+                                                    const int *__restrict__ klist, int nk,
+                                                    unsigned long long *__restrict__ calls,
+                                                    unsigned long long *__restrict__ claim, long long nrec) {
 #pragma clang fp contract(off)
+    if (blockIdx.x == 0) advance_calls(calls, claim, nrec, a.maxn);
     const int t = blockIdx.x * AWG + threadIdx.x;
     if (t >= nk * a.ns) return;
     const int v = klist[t / a.ns], sid = v * a.ns + t % a.ns;
@@ -260,71 +301,109 @@ __global__ __launch_bounds__(AWG) void k_adh_detach(AdhDev a, const double *__re
     r_ij[sid] = dr;
 }
 
-// One attachment round: each active spring proposes its next acceptable
-// free candidate and bids for it with its id.
-__global__ __launch_bounds__(AWG) void k_adh_propose(AdhDev a, const int *__restrict__ id_wall,
-                                                     const double *__restrict__ r_wall,
-                                                     const int *__restrict__ is_attached, int *__restrict__ pos,
-                                                     int *__restrict__ active, int *__restrict__ prop,
-                                                     unsigned long long *__restrict__ claim, const DevStep *__restrict__ st,
-                                                     int init, int *__restrict__ nprop, int round,
-                                                     const int *__restrict__ klist, int nk,
-                                                     const unsigned long long *__restrict__ calls) {
-    // after a round without proposals nothing changes any more
-    if (round > 0 && nprop[round - 1] == 0) return;
-    const int t = blockIdx.x * AWG + threadIdx.x;
-    if (t >= nk * a.ns) return;
-    const int v = klist[t / a.ns], sid = v * a.ns + t % a.ns;
-    prop[sid] = -1;
-    if (!active[sid]) return;
-    const double u = init ? 0.0 : adh_uniform(a.seed, st->iter, sid);
-    int c = pos[sid];
+// One attachment round, in two halves.  Each active spring proposes its next
+// acceptable free candidate (returned; -1: none) and bids for it with its id.
+struct AdhRound {
+    const int *id_wall, *klist;
+    const double *r_wall;
+    int *is_attached, *attach, *pos, *active, *prop;
+    double *r_ij;
+    unsigned long long *claim;
+    const unsigned long long *calls;
+    const DevStep *st;
+    int init, nk;
+};
+__device__ __forceinline__ int adh_propose(const AdhDev &a, const AdhRound &q, int round, unsigned long long call,
+                                           int sid) {
+    const int v = sid / a.ns;
+    const double u = q.init ? 0.0 : adh_uniform(a.seed, q.st->iter, sid);
+    int c = q.pos[sid], id = -1;
     for (; c < a.maxn; c++) {
-        const int id = id_wall[(size_t)v * a.maxn + c];
+        id = q.id_wall[(size_t)v * a.maxn + c];
         if (id == -1) continue;
-        if (!init) {
+        if (!q.init) {
             double dr;
-            if (p_on(a, r_wall[(size_t)v * a.maxn + c], dr) <= u) continue;
+            if (p_on(a, q.r_wall[(size_t)v * a.maxn + c], dr) <= u) continue;
         }
-        if (is_attached[id]) continue;
+        if (q.is_attached[id]) continue;
         break;
     }
     if (c >= a.maxn) {
-        active[sid] = 0;
-        return;
+        q.active[sid] = 0;
+        return -1;
     }
-    pos[sid] = c;
-    const int id = id_wall[(size_t)v * a.maxn + c];
-    prop[sid] = id;
-    atomicMax(claim + id, bid_key(*calls, round, a.maxn, sid));
-    atomicAdd(nprop + round, 1);
+    q.pos[sid] = c;
+    atomicMax(q.claim + id, bid_key(call, round, a.maxn, sid));
+    return id;
+}
+// The highest bid takes the receptor, the others go on to their next candidate.
+__device__ __forceinline__ void adh_resolve(const AdhDev &a, const AdhRound &q, int round, unsigned long long call,
+                                            int sid, int id) {
+    // bids are made in L2: read there
+    if (__hip_atomic_load(q.claim + id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+        bid_key(call, round, a.maxn, sid)) {
+        q.attach[sid] = id;
+        q.is_attached[id] = 1;
+        if (!q.init) {
+            double dr;
+            (void)p_on(a, q.r_wall[(size_t)(sid / a.ns) * a.maxn + q.pos[sid]], dr);
+            q.r_ij[sid] = dr;
+        }
+        q.active[sid] = 0;
+    } else {
+        q.pos[sid] = q.pos[sid] + 1;
+    }
 }
 
-__global__ __launch_bounds__(AWG) void k_adh_resolve(AdhDev a, const double *__restrict__ r_wall,
-                                                     int *__restrict__ attach, double *__restrict__ r_ij,
-                                                     int *__restrict__ is_attached, int *__restrict__ pos,
-                                                     int *__restrict__ active, const int *__restrict__ prop,
-                                                     const unsigned long long *__restrict__ claim, int init,
-                                                     const int *__restrict__ nprop, int round,
-                                                     const int *__restrict__ klist, int nk,
-                                                     const unsigned long long *__restrict__ calls) {
-    if (nprop[round] == 0) return;
+// Round 0, which meets every free spring: a launch per half.
+__global__ __launch_bounds__(AWG) void k_adh_propose(AdhDev a, AdhRound q) {
     const int t = blockIdx.x * AWG + threadIdx.x;
-    if (t >= nk * a.ns) return;
-    const int sid = klist[t / a.ns] * a.ns + t % a.ns;
-    const int id = prop[sid];
-    if (id < 0) return;
-    if (claim[id] == bid_key(*calls, round, a.maxn, sid)) {
-        attach[sid] = id;
-        is_attached[id] = 1;
-        if (!init) {
-            double dr;
-            (void)p_on(a, r_wall[(size_t)(sid / a.ns) * a.maxn + pos[sid]], dr);
-            r_ij[sid] = dr;
+    if (t >= q.nk * a.ns) return;
+    const int sid = q.klist[t / a.ns] * a.ns + t % a.ns;
+    q.prop[sid] = q.active[sid] ? adh_propose(a, q, 0, *q.calls, sid) : -1;
+}
+__global__ __launch_bounds__(AWG) void k_adh_resolve(AdhDev a, AdhRound q) {
+    const int t = blockIdx.x * AWG + threadIdx.x;
+    if (t >= q.nk * a.ns) return;
+    const int sid = q.klist[t / a.ns] * a.ns + t % a.ns;
+    const int id = q.prop[sid];
+    if (id >= 0) adh_resolve(a, q, 0, *q.calls, sid, id);
+}
+
+// The other rounds, which only the losers of the one before take part in, in
+// one work group that lists them and stops after a round without proposals.
+// A pair of launches for each of the MAXN + 1 rounds, most of them empty, took
+// 34 launches and about 95 us per step with MAXN = 16 (202 with the usual
+// 100); this takes 12 us, the first round 15.  Every spring advances or retires in every
+// round, so MAXN more rounds are enough.
+__global__ __launch_bounds__(1024) void k_adh_rounds(AdhDev a, AdhRound q, int *__restrict__ list) {
+    __shared__ int n, made;
+    if (threadIdx.x == 0) n = 0;
+    __syncthreads();
+    for (int t = threadIdx.x; t < q.nk * a.ns; t += 1024) {
+        const int sid = q.klist[t / a.ns] * a.ns + t % a.ns;
+        if (q.active[sid]) list[atomicAdd(&n, 1)] = sid;
+    }
+    __syncthreads();
+    const int m = n;
+    const unsigned long long call = *q.calls;
+    for (int round = 1; round <= a.maxn; round++) {
+        if (threadIdx.x == 0) made = 0;
+        __syncthreads();
+        for (int k = threadIdx.x; k < m; k += 1024) {
+            const int sid = list[k];
+            const int id = q.active[sid] ? adh_propose(a, q, round, call, sid) : -1;
+            q.prop[sid] = id;
+            if (id >= 0) made = 1;
         }
-        active[sid] = 0;
-    } else {
-        pos[sid] = pos[sid] + 1;
+        __threadfence();  // the bids, before they are read
+        __syncthreads();
+        if (!made) return;
+        for (int k = threadIdx.x; k < m; k += 1024) {
+            const int sid = list[k], id = q.prop[sid];
+            if (id >= 0) adh_resolve(a, q, round, call, sid, id);
+        }
+        __syncthreads();
     }
 }
 
@@ -369,24 +448,17 @@ lbmibm_status adh_bell(lbmibm_ctx *ctx, int init) {
     const long long nsp = (long long)ctx->adh_nk * a.ns;  // springs of the knobs
     const int *kl = ctx->adh_klist;
     const int nk = ctx->adh_nk;
-    hipLaunchKernelGGL(k_adh_search, dim3(ablocks(a.nv)), dim3(AWG), 0, st, a, (const double *)ctx->xs,
-                       (const unsigned char *)ctx->adh_knob, ctx->adh_idw, ctx->adh_rw);
+    const AdhRound q{ctx->adh_idw, kl, ctx->adh_rw, ctx->adh_isatt, ctx->adh_attach, ctx->adh_pos, ctx->adh_active,
+                     ctx->adh_prop, ctx->adh_rij, ctx->adh_claim, ctx->adh_calls, (const DevStep *)ctx->step, init, nk};
+    hipLaunchKernelGGL(k_adh_search, dim3(ablocks(64LL * nk)), dim3(AWG), 0, st, a, (const double *)ctx->xs, kl, nk,
+                       ctx->adh_idw, ctx->adh_rw);
     hipLaunchKernelGGL(k_adh_detach, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, (const double *)ctx->xs,
                        (const unsigned char *)ctx->adh_knob, ctx->adh_attach, ctx->adh_rij, ctx->adh_isatt,
-                       ctx->adh_pos, ctx->adh_active, (const DevStep *)ctx->step, init, kl, nk);
-    hipLaunchKernelGGL(k_afill<int>, dim3(1), dim3(64), 0, st, ctx->adh_nprop, (size_t)(a.maxn + 1), 0);
-    hipLaunchKernelGGL(k_adh_tick, dim3(1), dim3(256), 0, st, ctx->adh_calls, ctx->adh_claim,
-                       (long long)a.nxw * a.nzw, a.maxn);
-    for (int r = 0; r <= a.maxn; r++) {  // each round retires or advances every active spring
-        hipLaunchKernelGGL(k_adh_propose, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, (const int *)ctx->adh_idw,
-                           (const double *)ctx->adh_rw, (const int *)ctx->adh_isatt, ctx->adh_pos, ctx->adh_active,
-                           ctx->adh_prop, ctx->adh_claim, (const DevStep *)ctx->step, init, ctx->adh_nprop, r, kl,
-                           nk, (const unsigned long long *)ctx->adh_calls);
-        hipLaunchKernelGGL(k_adh_resolve, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, (const double *)ctx->adh_rw,
-                           ctx->adh_attach, ctx->adh_rij, ctx->adh_isatt, ctx->adh_pos, ctx->adh_active,
-                           (const int *)ctx->adh_prop, (const unsigned long long *)ctx->adh_claim, init,
-                           (const int *)ctx->adh_nprop, r, kl, nk, (const unsigned long long *)ctx->adh_calls);
-    }
+                       ctx->adh_pos, ctx->adh_active, (const DevStep *)ctx->step, init, kl, nk, ctx->adh_calls,
+                       ctx->adh_claim, (long long)a.nxw * a.nzw);
+    hipLaunchKernelGGL(k_adh_propose, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, q);
+    hipLaunchKernelGGL(k_adh_resolve, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, q);
+    hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, ctx->adh_list);
     LBMIBM_LAUNCHED(ctx, "k_adh_*");
     return LBMIBM_OK;
 }
@@ -463,7 +535,7 @@ lbmibm_status adhesion_setup(lbmibm_ctx *ctx, const lbmibm_adhesion_params *h, c
         void **bufs[] = {&ctx->adh_knob, (void **)&ctx->adh_idw, (void **)&ctx->adh_rw, (void **)&ctx->adh_attach,
                          (void **)&ctx->adh_rij, (void **)&ctx->adh_pos, (void **)&ctx->adh_active,
                          (void **)&ctx->adh_prop, (void **)&ctx->adh_isatt, (void **)&ctx->adh_claim,
-                         (void **)&ctx->adh_calls, (void **)&ctx->adh_fadh, (void **)&ctx->adh_nprop,
+                         (void **)&ctx->adh_calls, (void **)&ctx->adh_fadh, (void **)&ctx->adh_list,
                          (void **)&ctx->adh_klist, &ctx->adh_fsum, (void **)&ctx->adh_ring};
         for (void **p : bufs) {
             if (*p) (void)hipFree(*p);
@@ -485,7 +557,7 @@ lbmibm_status adhesion_setup(lbmibm_ctx *ctx, const lbmibm_adhesion_params *h, c
     al((void **)&ctx->adh_claim, nrec * sizeof(unsigned long long));
     al((void **)&ctx->adh_calls, sizeof(unsigned long long));
     al((void **)&ctx->adh_fadh, 3 * nv * sizeof(double));
-    al((void **)&ctx->adh_nprop, (size_t)(h->max_neighwall + 1) * sizeof(int));
+    al((void **)&ctx->adh_list, std::max<size_t>(klist.size() * h->springs_per_knob, 1) * sizeof(int));
     al((void **)&ctx->adh_klist, std::max<size_t>(klist.size(), 1) * sizeof(int));
     al(&ctx->adh_fsum, 3 * nv * ctx->szT);
     std::vector<double> ring;

@@ -259,3 +259,33 @@ def test_download_of_the_indicator_zeroes_the_walls():
     want[:, 2:-2] = np.pad(comp, ((2, 2), (0, 0), (2, 2)), mode="wrap")
     g.close()
     assert np.array_equal(got.reshape(want.shape), want)
+
+
+# more receptors in range than the search holds in LDS, and long lists; few
+# receptors for many springs, which lose round after round; one candidate each
+SPRINGS = [dict(receptor_density=64.0, max_neighwall=100), dict(receptor_density=1.0, springs_per_knob=12),
+           dict(max_neighwall=1), dict(receptor_density=16.0, max_neighwall=100, springs_per_knob=40)]
+
+
+@pytest.mark.parametrize("k", range(len(SPRINGS)))
+def test_receptor_lists_and_attachment_rounds(k):
+    """Lists and attachments are whole numbers: equal to the oracle's."""
+    from tests.test_adhesion import LY, _pair
+    print(f"[springs] {SPRINGS[k]}", flush=True)
+    o, g, st, nrec = _pair("f64", extra=SPRINGS[k], tau=0.9, p=5e-6, b=5e-3)
+    X, Y, Z = o.node_coords()
+    vel = 4e-3 * (Y + LY / 2) / LY
+    vel[o.bc == 2] = 0.0
+    o.init_fluid(None, vel, None, None)
+    g.set_equilibrium(None, vel, None, None)
+    o.volume_init()
+    g.volume_init()
+    for it in range(5):
+        gs = g.adhesion_state(nrec)
+        for name in ("id_wall", "attach", "is_attached"):
+            assert np.array_equal(gs[name], st[name]), (it, name)
+        if it < 4:
+            assert o.step(it + 1)[0] == 0
+            g.step(it + 1)
+    assert (st["attach"] >= 0).sum() > 5
+    g.close()
