@@ -36,8 +36,8 @@ namespace {
 constexpr double FT_UNIT = 17592186044416.0;  // 2^44 fixed-point units per 1/dx
 constexpr int VWG = 256;
 constexpr int FT_MAX_ATTEMPTS = 10;
-constexpr int SOR_CHUNKS = 4;  // x-pair chunks of VWG per work-group of k_sor_rows
-constexpr int CHECK_WG = 1024;
+constexpr int SOR_WG = 512;   // work-group size of k_sor_rows
+constexpr int SOR_GROUPS = 1024;  // and their largest number: as many as the chip runs at once
 
 struct FtGeom {
     int nx, ny, nz;  // padded sizes
@@ -298,134 +298,150 @@ __global__ void k_ft_start(SorCtl *__restrict__ ctl, const double *__restrict__ 
     }
 }
 
-// One colour of the COMP and WALL rows.  One lane per x-pair of a row: the
+// Residual norm of one iteration from the partial sums of r^2 (the padding
+// rows, all equal, contribute npad x_pad^2) and the stop test of
+// matrix_solver.cu:198-205.  Called by a whole work group, the same result in
+// every thread of every group.
+__device__ SorCtl sor_check(SorCtl st, const double *__restrict__ part, int nparts, double npad, int itrmax,
+                            double residual, double *lds) {
+#pragma clang fp contract(off)
+    if (st.done) return st;
+    double s = 0.0;
+    for (int k = threadIdx.x; k < nparts; k += blockDim.x) s += part[k];
+    s = block_sum(s, lds);
+    __shared__ double total;
+    if (threadIdx.x == 0) total = s;
+    __syncthreads();
+    const double rr = total + npad * (st.xpad * st.xpad);
+    st.xpad = st.xpad + 1.3 * (0.0 - 1.0 * st.xpad);
+    st.iter++;
+    st.err = sqrt(rr / st.bb);
+    if (st.err < residual) {
+        st.done = 1;
+        st.conv_iter = st.iter;
+    } else if (st.iter >= itrmax) {
+        st.done = 2;
+    }
+    return st;
+}
+
+// The stop test of the iteration before: its partial sums and the criterion.
+struct SorTest {
+    const double *part;  // of the previous iteration; nparts = 0: checked already
+    int nparts, itrmax;
+    double npad, residual;
+};
+
+// One colour of the SOR iteration: the COMP and WALL rows, and with them the
+// BUFF rows x_i - x_image = 0 of that colour.  One lane per x-pair of a row: the
 // lane takes the node of colour C, so a wave reads and writes a contiguous
-// stretch of the row.  A work-group takes SOR_CHUNKS consecutive stretches
+// stretch of the row.  A work-group takes `chunks` consecutive stretches
 // and the work-groups of one XCD a contiguous range of planes (their
 // neighbour planes stay in that XCD's L2); one partial sum of r^2 per
 // work-group.
+//
+// A BUFF row is read by the other colour only, and comes after its image's
+// update where that has the same colour (an even number of nodes away): then
+// the image's lane takes it along, with the value it has just formed.
+// Otherwise the image is of the other colour, which this launch does not
+// write, and the BUFF node's own lane takes it.  The first colour also makes the
+// stop test of the iteration before, every work group for itself.
+//
+// Launches and latency bound it, the arrays stay in the caches: 128x64x64
+// nodes took 21.5 us per iteration with the BUFF rows and the test in launches
+// of their own (2 x 3.5 and 2.6 us) and four stretches one after another,
+// 12.5 now (15 with the test and groups of 1024, 13 with groups of 256).  So every load of a lane is issued before the test, and one
+// stretch per group is taken until the groups fill the chip; more of
+// them would read each other's sums longer than they save.
 template <int C>
-__global__ __launch_bounds__(VWG) void k_sor_rows(FtGeom g, double *__restrict__ x, const double *__restrict__ b,
-                                                  const SorCtl *__restrict__ ctl, double *__restrict__ part, double a,
-                                                  int nblocks) {
+__global__ __launch_bounds__(SOR_WG) void k_sor_rows(FtGeom g, double *__restrict__ x, const double *__restrict__ b,
+                                                     const SorCtl *__restrict__ ctl, SorCtl *__restrict__ next,
+                                                     SorTest test, double *__restrict__ part, double a, int nblocks,
+                                                     int chunks) {
 #pragma clang fp contract(off)
-    __shared__ double lds[VWG / 64];
-    if (ctl->done) return;
+    __shared__ double lds[SOR_WG / 64];
     const int lb = xcd_block(nblocks);
     if (lb >= nblocks) return;
+    SorCtl st = *ctl;
     const unsigned nxh = (unsigned)(g.nx + 1) >> 1, nyu = (unsigned)g.ny;
+    const int lx = g.nx - 4, lz = g.nz - 4;
+    double *xc = x + (size_t)C * g.half;
+    const double *xo = x + (size_t)(1 - C) * g.half;
+    // where node (ix, iy, iz) of colour C or 1 - C sits in its array
+    auto at = [&](int ix, int iy, int iz) { return (unsigned)(ix >> 1) + nxh * ((unsigned)iy + nyu * (unsigned)iz); };
     double r2 = 0.0;
-    for (int k = 0; k < SOR_CHUNKS; k++) {
-    const unsigned t = ((unsigned)lb * SOR_CHUNKS + k) * VWG + threadIdx.x;
-    const unsigned row = t / nxh;
-    if (row < nyu * (unsigned)g.nz) {
+    for (int c = 0; c < chunks; c++) {
+        const unsigned t = ((unsigned)lb * chunks + c) * SOR_WG + threadIdx.x;
+        const unsigned row = t / nxh;
         const unsigned izu = row / nyu;
         const int iy = (int)(row - izu * nyu), iz = (int)izu;
-        const int ix = 2 * (int)(t - row * nxh) + ((C + iy + iz) & 1);
-        if (ix < g.nx) {
-            // own colour C at k + nxh*row; the neighbours, of colour 1-C, at
-            // their own x >> 1 in rows row, row -+ 1 (y), row -+ ny (z)
-            const unsigned k = t - row * nxh;
-            double *xc = x + (size_t)C * g.half;
-            const double *xo = x + (size_t)(1 - C) * g.half;
-            const unsigned i = k + nxh * row;
-            const int kind = ft_kind(g, ix, iy, iz);
-            const bool wall = kind == FT_WALL, comp = kind == FT_COMP;
-            if (comp || wall) {
-                double sum, bi = 0.0;
-                if (comp) {
-                    const unsigned rowz = nxh * (unsigned)g.ny;
-                    const unsigned xm = ((unsigned)ix - 1) >> 1, xp = ((unsigned)ix + 1) >> 1;
-                    const unsigned r0 = nxh * row;
-                    sum = 0.0;
-                    sum += a * xo[k + r0 - rowz];
-                    sum += a * xo[k + r0 - nxh];
-                    sum += a * xo[xm + r0];
-                    sum += 1.0 * xc[i];
-                    sum += a * xo[xp + r0];
-                    sum += a * xo[k + r0 + nxh];
-                    sum += a * xo[k + r0 + rowz];
-                    bi = b[(size_t)C * g.half + i];
-                } else {
-                    sum = 1.0 * xc[i];
-                }
-                const double r = bi - sum;
-                xc[i] = xc[i] + 1.3 * r;
+        const unsigned k = t - row * nxh;
+        const int ix = 2 * (int)k + ((C + iy + iz) & 1);
+        const bool on = row < nyu * (unsigned)g.nz && ix < g.nx;
+        // own colour C at k + nxh*row; the neighbours, of colour 1-C, at
+        // their own x >> 1 in rows row, row -+ 1 (y), row -+ ny (z)
+        const unsigned i = on ? k + nxh * row : 0;
+        const int kind = on ? ft_kind(g, ix, iy, iz) : -1;
+        const bool comp = kind == FT_COMP;
+        // the BUFF nodes that this one is the image of: x halo (not in the
+        // tube, where that is wall), z halo, both
+        const int hx = g.tube_col ? -1 : ix < 4 ? ix + lx : ix >= g.nx - 4 ? ix - lx : -1;
+        const int hz = iz < 4 ? iz + lz : iz >= g.nz - 4 ? iz - lz : -1;
+        const bool sx = comp && hx >= 0 && !(lx & 1), sz = comp && hz >= 0 && !(lz & 1);
+        const bool sxz = comp && hx >= 0 && hz >= 0 && !((lx + lz) & 1);
+        const unsigned jx = sx ? at(hx, iy, iz) : i, jz = sz ? at(ix, iy, hz) : i, jxz = sxz ? at(hx, iy, hz) : i;
+        // or this one's image, where that is of the other colour
+        const int mx = ix <= 1 ? ix + lx : (ix >= g.nx - 2 ? ix - lx : ix);
+        const int mz = iz <= 1 ? iz + lz : (iz >= g.nz - 2 ? iz - lz : iz);
+        const bool odd = kind == FT_BUFF && ((mx + mz - ix - iz) & 1);
+        const unsigned rowz = nxh * nyu, r0 = nxh * row;
+        const unsigned xm = ((unsigned)ix - 1) >> 1, xp = ((unsigned)ix + 1) >> 1;
+        const double own = xc[i], bx = xc[jx], bz = xc[jz], bxz = xc[jxz], other = xo[odd ? at(mx, iy, mz) : i];
+        const double bi = b[(size_t)C * g.half + i];
+        const double zm = xo[comp ? k + r0 - rowz : i], ym = xo[comp ? k + r0 - nxh : i], xl = xo[comp ? xm + r0 : i];
+        const double xr = xo[comp ? xp + r0 : i], yp = xo[comp ? k + r0 + nxh : i], zp = xo[comp ? k + r0 + rowz : i];
+        if (C == 0 && c == 0 && test.nparts > 0)
+            st = sor_check(st, test.part, test.nparts, test.npad, test.itrmax, test.residual, lds);
+        if (C == 0 && c == 0 && lb == 0 && threadIdx.x == 0) *next = st;
+        if (st.done) return;  // nothing changes any more
+        if (comp) {
+            double sum = 0.0;
+            sum += a * zm;
+            sum += a * ym;
+            sum += a * xl;
+            sum += 1.0 * own;
+            sum += a * xr;
+            sum += a * yp;
+            sum += a * zp;
+            const double r = bi - sum;
+            const double now = own + 1.3 * r;
+            xc[i] = now;
+            r2 += r * r;
+            auto image = [&](bool take, unsigned j, double old) {
+                if (!take) return;
+                const double r = 0.0 - (old - now);
+                xc[j] = old + 1.3 * r;
                 r2 += r * r;
-            }
+            };
+            image(sx, jx, bx);
+            image(sz, jz, bz);
+            image(sxz, jxz, bxz);
+        } else if (kind == FT_WALL || odd) {
+            const double r = 0.0 - (kind == FT_WALL ? 1.0 * own : own - other);
+            xc[i] = own + 1.3 * r;
+            r2 += r * r;
         }
-    }
     }
     const double s = block_sum(r2, lds);
     if (threadIdx.x == 0) part[lb] = s;
 }
 
-// One colour of the BUFF rows x_i - x_image = 0: the x halo (all z) then
-// the z halo (COMP x), y within the COMP range.
-template <int C>
-__global__ __launch_bounds__(VWG) void k_sor_buff(FtGeom g, double *__restrict__ x, const SorCtl *__restrict__ ctl,
-                                                  double *__restrict__ part) {
-#pragma clang fp contract(off)
-    __shared__ double lds[VWG / 64];
-    if (ctl->done) return;
-    const long long t = (long long)blockIdx.x * VWG + threadIdx.x;
-    const long long ny4 = g.ny - 4, nx4 = g.nx - 4;
-    const long long n1 = 4 * ny4 * g.nz, n2 = 4 * nx4 * ny4;
-    double r2 = 0.0;
-    if (t < n1 + n2) {
-        int ix, iy, iz;
-        if (t < n1) {
-            const int a = (int)(t & 3);
-            const long long rest = t >> 2;
-            ix = a < 2 ? a : g.nx - 4 + a;
-            iy = 2 + (int)(rest % ny4);
-            iz = (int)(rest / ny4);
-        } else {
-            const long long u = t - n1;
-            const int a = (int)(u & 3);
-            const long long rest = u >> 2;
-            iz = a < 2 ? a : g.nz - 4 + a;
-            ix = 2 + (int)(rest % nx4);
-            iy = 2 + (int)(rest / nx4);
-        }
-        if (((ix + iy + iz) & 1) == C && ft_kind(g, ix, iy, iz) == FT_BUFF) {
-            const int jx = ix <= 1 ? ix + (g.nx - 4) : (ix >= g.nx - 2 ? ix - (g.nx - 4) : ix);
-            const int jz = iz <= 1 ? iz + (g.nz - 4) : (iz >= g.nz - 2 ? iz - (g.nz - 4) : iz);
-            const long long i = packed(g, ix, iy, iz), j = packed(g, jx, iy, jz);
-            const double r = 0.0 - (x[i] - x[j]);
-            x[i] = x[i] + 1.3 * r;
-            r2 = r * r;
-        }
-    }
-    const double s = block_sum(r2, lds);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-// Residual norm of one iteration (the padding rows, all equal, contribute
-// npad x_pad^2) and the stop test of matrix_solver.cu:198-205.
-__global__ __launch_bounds__(CHECK_WG) void k_sor_check(SorCtl *__restrict__ ctl, const double *__restrict__ part,
-                                                         int nparts, double npad, int itrmax, double residual) {
-#pragma clang fp contract(off)
-    __shared__ double lds[CHECK_WG / 64];
-    if (ctl->done) return;
-    double s = 0.0;
-    for (int k = threadIdx.x; k < nparts; k += blockDim.x) s += part[k];
-    s = block_sum(s, lds);
-    if (threadIdx.x == 0) {
-        const double xp = ctl->xpad;
-        const double rr = s + npad * (xp * xp);
-        ctl->xpad = xp + 1.3 * (0.0 - 1.0 * xp);
-        const int it = ctl->iter + 1;
-        ctl->iter = it;
-        const double err = sqrt(rr / ctl->bb);
-        ctl->err = err;
-        if (err < residual) {
-            ctl->done = 1;
-            ctl->conv_iter = it;
-        } else if (it >= itrmax) {
-            ctl->done = 2;
-        }
-    }
+// The stop test of the last iteration of a batch, whose state the host reads.
+__global__ __launch_bounds__(SOR_WG) void k_sor_check(SorCtl *__restrict__ ctl, SorTest test) {
+    __shared__ double lds[SOR_WG / 64];
+    const SorCtl st = sor_check(*ctl, test.part, test.nparts, test.npad, test.itrmax, test.residual, lds);
+    __syncthreads();
+    if (threadIdx.x == 0) *ctl = st;
 }
 
 __global__ __launch_bounds__(VWG) void k_ft_extract(FtGeom g, const double *__restrict__ x, double *__restrict__ vf,
@@ -580,11 +596,13 @@ FtGeom ft_geom(const lbmibm_ctx *ctx) {
 inline unsigned blocks_of(long long n) { return (unsigned)((n + VWG - 1) / VWG); }
 
 long long sor_row_threads(const FtGeom &g) { return (long long)((g.nx + 1) / 2) * g.ny * g.nz; }
-int sor_row_blocks(const FtGeom &g) {
-    return (int)((sor_row_threads(g) + (long long)VWG * SOR_CHUNKS - 1) / ((long long)VWG * SOR_CHUNKS));
+int sor_chunks(const FtGeom &g) {
+    const long long per = (long long)SOR_WG * SOR_GROUPS;
+    return (int)((sor_row_threads(g) + per - 1) / per);
 }
-long long sor_buff_threads(const FtGeom &g) {
-    return 4LL * (g.ny - 4) * g.nz + 4LL * (g.nx - 4) * (g.ny - 4);
+int sor_row_blocks(const FtGeom &g) {
+    const long long per = (long long)SOR_WG * sor_chunks(g);
+    return (int)((sor_row_threads(g) + per - 1) / per);
 }
 
 int expand_pow2(long long n) {  // etc.cu:425-446
@@ -602,8 +620,7 @@ int expand_pow2(long long n) {  // etc.cu:425-446
 lbmibm_status vof_alloc(lbmibm_ctx *ctx) {
     if (ctx->vof[0]) return LBMIBM_OK;
     const FtGeom g = ft_geom(ctx);
-    const long long nb_rows = sor_row_blocks(g), nb_buff = blocks_of(sor_buff_threads(g));
-    ctx->ft_nparts = (int)(2 * (nb_rows + nb_buff));
+    ctx->ft_nparts = 4 * sor_row_blocks(g);  // two colours, two iterations
     const long long nparts = std::max<long long>(ctx->ft_nparts, blocks_of(g.np));
     lbmibm_status s = dev_alloc(ctx, (void **)&ctx->vof[0], ctx->N * sizeof(double));
     if (s == LBMIBM_OK) s = dev_alloc(ctx, (void **)&ctx->vof[1], ctx->N * sizeof(double));
@@ -611,7 +628,7 @@ lbmibm_status vof_alloc(lbmibm_ctx *ctx) {
     if (s == LBMIBM_OK) s = dev_alloc(ctx, (void **)&ctx->ft_x, 2 * g.half * sizeof(double));
     if (s == LBMIBM_OK) s = dev_alloc(ctx, (void **)&ctx->ft_b, 2 * g.half * sizeof(double));
     if (s == LBMIBM_OK) s = dev_alloc(ctx, (void **)&ctx->ft_part, nparts * sizeof(double));
-    if (s == LBMIBM_OK) s = dev_alloc(ctx, &ctx->ft_ctl, sizeof(SorCtl));
+    if (s == LBMIBM_OK) s = dev_alloc(ctx, &ctx->ft_ctl, 2 * sizeof(SorCtl));
     if (s != LBMIBM_OK) return s;
     for (int k = 0; k < 2; k++) {
         hipLaunchKernelGGL(k_vfill<double>, dim3(blocks_of(ctx->N)), dim3(VWG), 0, ctx->stream, ctx->vof[k],
@@ -646,14 +663,14 @@ lbmibm_status vof_front_tracking(lbmibm_ctx *ctx, int *iterations, int *attempts
     LBMIBM_LAUNCHED(ctx, "k_ft_rhs");
     // per-block sums of b^2 are in ft_part until k_ft_start adds them up
     const int nb_b = (int)blocks_of(g.np);
-    const unsigned nb_rows = sor_row_blocks(g), nb_buff = blocks_of(sor_buff_threads(g));
+    const unsigned nb_rows = sor_row_blocks(g);
     const unsigned grid_rows = xcd_grid(nb_rows);
     double *part = ctx->ft_part;
-    double *p_r0 = part, *p_b0 = part + nb_rows, *p_r1 = part + nb_rows + nb_buff, *p_b1 = p_r1 + nb_rows;
     SorCtl *ctl = (SorCtl *)ctx->ft_ctl;
     const double a = (1.0 / (g.dx * g.dx)) / (-6.0 / (g.dx * g.dx));  // fronttrack.cu:97-110, 294-311
     const long long mn = 1LL << expand_pow2(g.np);
     const double npad = (double)(mn - g.np);
+    const int nparts = (int)(2 * nb_rows), chunks = sor_chunks(g);
     // b.b of the first start, kept for the restarts (b does not change)
     hipLaunchKernelGGL(k_ft_start, dim3(1), dim3(VWG), 0, st, ctl, (const double *)part, nb_b, 0.0);
     LBMIBM_LAUNCHED(ctx, "k_ft_start");
@@ -670,24 +687,30 @@ lbmibm_status vof_front_tracking(lbmibm_ctx *ctx, int *iterations, int *attempts
         h.xpad = (double)cnt;
         h.bb = bb;
         LBMIBM_HIP(ctx, hipMemcpyAsync(ctl, &h, sizeof(SorCtl), hipMemcpyHostToDevice, st));
+        // an iteration keeps its partial sums and the state that its first
+        // colour formed in one of two places, the next one in the other
+        int cur = 0;
+        auto test_of = [&](int k, bool checked) {
+            return SorTest{part + (size_t)k * nparts, checked ? 0 : nparts, ctx->p.sor_itrmax, npad, ctx->p.sor_residual};
+        };
         int batch = 16;
         int issued = 0;
         for (;;) {
             for (int k = 0; k < batch; k++) {
-                hipLaunchKernelGGL(k_sor_rows<0>, dim3(grid_rows), dim3(VWG), 0, st, g, ctx->ft_x,
-                                   (const double *)ctx->ft_b, (const SorCtl *)ctl, p_r0, a, (int)nb_rows);
-                hipLaunchKernelGGL(k_sor_buff<0>, dim3(nb_buff), dim3(VWG), 0, st, g, ctx->ft_x, (const SorCtl *)ctl,
-                                   p_b0);
-                hipLaunchKernelGGL(k_sor_rows<1>, dim3(grid_rows), dim3(VWG), 0, st, g, ctx->ft_x,
-                                   (const double *)ctx->ft_b, (const SorCtl *)ctl, p_r1, a, (int)nb_rows);
-                hipLaunchKernelGGL(k_sor_buff<1>, dim3(nb_buff), dim3(VWG), 0, st, g, ctx->ft_x, (const SorCtl *)ctl,
-                                   p_b1);
-                hipLaunchKernelGGL(k_sor_check, dim3(1), dim3(CHECK_WG), 0, st, ctl, (const double *)part,
-                                   (int)(2 * (nb_rows + nb_buff)), npad, ctx->p.sor_itrmax, ctx->p.sor_residual);
+                const int old = cur;
+                cur ^= 1;
+                double *p = part + (size_t)cur * nparts;
+                hipLaunchKernelGGL(k_sor_rows<0>, dim3(grid_rows), dim3(SOR_WG), 0, st, g, ctx->ft_x,
+                                   (const double *)ctx->ft_b, (const SorCtl *)(ctl + old), ctl + cur,
+                                   test_of(old, k == 0), p, a, (int)nb_rows, chunks);
+                hipLaunchKernelGGL(k_sor_rows<1>, dim3(grid_rows), dim3(SOR_WG), 0, st, g, ctx->ft_x,
+                                   (const double *)ctx->ft_b, (const SorCtl *)(ctl + cur), (SorCtl *)nullptr,
+                                   SorTest{}, p + nb_rows, a, (int)nb_rows, chunks);
             }
+            hipLaunchKernelGGL(k_sor_check, dim3(1), dim3(SOR_WG), 0, st, ctl + cur, test_of(cur, false));
             LBMIBM_LAUNCHED(ctx, "k_sor_*");
             issued += batch;
-            LBMIBM_HIP(ctx, hipMemcpyAsync(&h, ctl, sizeof(SorCtl), hipMemcpyDeviceToHost, st));
+            LBMIBM_HIP(ctx, hipMemcpyAsync(&h, ctl + cur, sizeof(SorCtl), hipMemcpyDeviceToHost, st));
             LBMIBM_HIP(ctx, hipStreamSynchronize(st));
             if (h.done) break;
             if (issued > ctx->p.sor_itrmax + 1) {  // the device test stops by ITRMAX

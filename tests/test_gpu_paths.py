@@ -289,3 +289,48 @@ def test_receptor_lists_and_attachment_rounds(k):
             g.step(it + 1)
     assert (st["attach"] >= 0).sum() > 5
     g.close()
+
+
+# the halo's image of either colour on each axis, the smallest lattice, several
+# work groups
+SORS = [(20, 16, 18), (21, 16, 18), (20, 17, 19), (23, 16, 21), (4, 14, 4), (70, 30, 61)]
+
+
+@pytest.mark.parametrize("k", range(len(SORS)))
+def test_front_tracking_of_every_halo_parity(k):
+    from preprocess_src_amd import mesh
+    shape = SORS[k]
+    print(f"[front parity] {shape}", flush=True)
+    cells = mesh.assemble([2], np.array([[0.3, 0.2, -0.4]]), np.eye(3)[None], min(shape) / 4.5, shape="sphere")
+    kw = dict(sor_itrmax=200000, sor_residual=1e-10)
+    o = oracle_of(*shape, cells=cells, **kw)
+    g = gpu_of(*shape, "f64", cells=cells, vof_period=4, **kw)
+    rc, its, att = o.front_tracking()
+    assert rc == 0
+    gits, gatt = g.front_tracking()
+    assert gatt == att and abs(gits - its) <= 1, (gits, its)
+    keep = o.bc != 2
+    # two solves of the same system, stopped at a residual of 1e-10
+    assert rel(g.vf()[keep], o.vf[keep]) < 1e-8
+    first = g.vf()
+    g.front_tracking()
+    assert np.array_equal(g.vf(), first)
+    g.close()
+
+
+def test_front_tracking_of_several_stretches_per_group():
+    """More x pairs than 1024 work groups of 512 take in one stretch each."""
+    from preprocess_src_amd import mesh
+    shape = (300, 10, 300)
+    print(f"[front stretches] {shape}", flush=True)
+    cells = mesh.assemble([2], np.array([[0.3, 0.2, -0.4]]), np.eye(3)[None], 2.5, shape="sphere")
+    kw = dict(sor_itrmax=200000, sor_residual=1e-2)
+    o = oracle_of(*shape, cells=cells, **kw)
+    g = gpu_of(*shape, "f64", cells=cells, vof_period=4, **kw)
+    rc, its, att = o.front_tracking()
+    assert rc == 0
+    gits, gatt = g.front_tracking()
+    assert gatt == att and gits == its, (gits, its)
+    keep = o.bc != 2
+    assert rel(g.vf()[keep], o.vf[keep]) < 1e-10  # the same iterate of the same sweeps
+    g.close()
