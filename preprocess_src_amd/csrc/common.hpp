@@ -376,7 +376,6 @@ lbmibm_status adhesion_step(lbmibm_ctx *ctx);                // adhesion.hip
 inline const void *spread_force(const lbmibm_ctx *ctx) { return ctx->adh_on ? ctx->adh_fsum : ctx->cf; }
 // both classes on the given stream (not the context's main stream)
 lbmibm_status volume_run_on(lbmibm_ctx *ctx, int mode, hipStream_t stream);  // volume.hip
-lbmibm_status ibm_count_begin(lbmibm_ctx *ctx, hipStream_t stream);  // ibm.hip: zero the tile counts
 lbmibm_status ibm_count_end(lbmibm_ctx *ctx, hipStream_t stream);    // ibm.hip: tile offsets and orders
 // the positions changed: the bins and the tile counts are stale
 inline void invalidate_bins(lbmibm_ctx *ctx) {

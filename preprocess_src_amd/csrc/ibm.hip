@@ -269,6 +269,39 @@ __device__ void heavy_first_order(const int *load, int n, int *hist, int *order)
     __syncthreads();
 }
 
+// The heavy-first tile orders of the spreading (by candidate count: own bin
+// and the bins below on each axis) and of the interpolation (by own count).
+// They only steer the dispatch order, and tile loads change slowly with the
+// cells, so they are refreshed on every TILE_ORDER_PERIOD-th binning (a call
+// counter on the device, so captured graphs refresh them too); any
+// permutation is a valid order, the initial one is the identity.
+constexpr int TILE_ORDER_PERIOD = 16;
+
+__device__ void tile_orders(const int *__restrict__ tile_count, int ntiles, const IbmGeom &g, const TileGeom &tg,
+                            int *__restrict__ tile_cand, int *__restrict__ order_spread,
+                            int *__restrict__ order_interp, int *__restrict__ calls) {
+    __shared__ int sh[256];
+    __shared__ int call;
+    if (threadIdx.x == 0) call = (*calls)++;
+    __syncthreads();
+    if (call % TILE_ORDER_PERIOD != 0) return;
+    for (int t = threadIdx.x; t < ntiles; t += 1024) {
+        const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
+        int sxs[4], sys[4], szs[4];
+        const int nsx = source_tiles(tx, tx * tg.tx, g.nx, tg.tx, true, sxs);
+        const int nsy = source_tiles(ty, ty * TILE_Y, g.ny, TILE_Y, !g.walls, sys);
+        const int nsz = source_tiles(tz, tz * TILE_Z, g.nz, TILE_Z, true, szs);
+        int c = 0;
+        for (int iz = 0; iz < nsz; iz++)
+            for (int iy = 0; iy < nsy; iy++)
+                for (int ix = 0; ix < nsx; ix++) c += tile_count[sxs[ix] + tg.ntx * (sys[iy] + tg.nty * szs[iz])];
+        tile_cand[t] = c;
+    }
+    __syncthreads();
+    heavy_first_order(tile_cand, ntiles, sh, order_spread);
+    heavy_first_order(tile_count, ntiles, sh, order_interp);
+}
+
 // Vertices per work group of k_spread_box, and the work groups of a tile.
 constexpr int SB_CHUNK = 800;
 __host__ __device__ __forceinline__ int spread_chunks(int cnt) { return (cnt + SB_CHUNK - 1) / SB_CHUNK; }
@@ -276,12 +309,16 @@ __host__ __device__ __forceinline__ int spread_chunks(int cnt) { return (cnt + S
 // Exclusive scans over the tiles, in one work group, 1024 tiles per round: the
 // bins' offsets, and the extra chunks of the tiles that k_spread_box shares
 // out (listed in `extra`, (-1, 0) behind the last); and the maximum of the
-// per-block force maxima.  Both scans ride in one 64-bit wave scan, one barrier a round.
+// per-block force maxima.  Both scans ride in one 64-bit wave scan, one barrier
+// a round.  The tile orders follow in the same launch (of their own they took
+// 5 us a step, nearly always to find that they are not due).
 __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile_count, int *__restrict__ tile_off,
                                                     int *__restrict__ tile_cur, int ntiles,
                                                     const float *__restrict__ blk_fmax, int nblk,
                                                     unsigned *__restrict__ absmax, int *__restrict__ tile_ex,
-                                                    int2 *__restrict__ extra, int maxextra) {
+                                                    int2 *__restrict__ extra, int maxextra, IbmGeom g, TileGeom tg,
+                                                    int *__restrict__ tile_cand, int *__restrict__ order_spread,
+                                                    int *__restrict__ order_interp, int *__restrict__ order_calls) {
     __shared__ unsigned long long wtot[2][16];
     __shared__ float wmax[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -326,40 +363,7 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile
         for (int w = 1; w < 16; w++) fm = fmaxf(fm, wmax[w]);
         *absmax = __float_as_uint(fm);
     }
-}
-
-// The heavy-first tile orders of the spreading (by candidate count: own bin
-// and the bins below on each axis) and of the interpolation (by own count).
-// They only steer the dispatch order, and tile loads change slowly with the
-// cells, so they are refreshed on every TILE_ORDER_PERIOD-th binning (a call
-// counter on the device, so captured graphs refresh them too); any
-// permutation is a valid order, the initial one is the identity.
-constexpr int TILE_ORDER_PERIOD = 16;
-
-__global__ __launch_bounds__(1024) void k_tile_order(const int *__restrict__ tile_count, int ntiles, IbmGeom g,
-                                                     TileGeom tg, int *__restrict__ tile_cand,
-                                                     int *__restrict__ order_spread, int *__restrict__ order_interp,
-                                                     int *__restrict__ calls) {
-    __shared__ int sh[256];
-    __shared__ int call;
-    if (threadIdx.x == 0) call = (*calls)++;
-    __syncthreads();
-    if (call % TILE_ORDER_PERIOD != 0) return;
-    for (int t = threadIdx.x; t < ntiles; t += 1024) {
-        const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
-        int sxs[4], sys[4], szs[4];
-        const int nsx = source_tiles(tx, tx * tg.tx, g.nx, tg.tx, true, sxs);
-        const int nsy = source_tiles(ty, ty * TILE_Y, g.ny, TILE_Y, !g.walls, sys);
-        const int nsz = source_tiles(tz, tz * TILE_Z, g.nz, TILE_Z, true, szs);
-        int c = 0;
-        for (int iz = 0; iz < nsz; iz++)
-            for (int iy = 0; iy < nsy; iy++)
-                for (int ix = 0; ix < nsx; ix++) c += tile_count[sxs[ix] + tg.ntx * (sys[iy] + tg.nty * szs[iz])];
-        tile_cand[t] = c;
-    }
-    __syncthreads();
-    heavy_first_order(tile_cand, ntiles, sh, order_spread);
-    heavy_first_order(tile_count, ntiles, sh, order_interp);
+    tile_orders(tile_count, ntiles, g, tg, tile_cand, order_spread, order_interp, order_calls);
 }
 
 // Spreading data of a vertex, stored in bin order next to its first stencil
@@ -719,25 +723,64 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the cell of a vertex's first stencil node (x, z wrapped at binning; y
     // raw: with walls it may lie below the lattice in the first tile row), -1
-    // when this tile is not a valid home or the cell is another chunk's
+    // when this tile is not a valid home
     auto key_of = [&](short4 n0) {
         int y1 = n0.y - 3;
         if (!g.walls) wrap_index(y1, g.ny);
         const int bx = n0.x - ox, by = y1 - oy + 3, bz = n0.z - oz;
         if (bx < 0 || bx >= TILE_X || bz < 0 || bz >= TILE_Z || by < 0 || by >= SB_Y) return -1;
-        if (nch > 1 && (bx + 5 * by + 3 * bz) % nch != chunk) return -1;
         return bx + TILE_X * (by + SB_Y * bz);
     };
     for (int k = tid; k < 3 * SB_N; k += WG_) acc[k] = 0ull;
     for (int k = tid; k <= SB_KEYS; k += WG_) start[k] = 0;
     if (tid == 0) nsel = 0;
     __syncthreads();
-    int n = cnt;
+    // exclusive scan of the key counts, KPT consecutive keys per thread, the total behind the last
+    auto scan_keys = [&] {
+        int own[KPT], before = 0;
+#pragma unroll
+        for (int k = 0; k < KPT; k++) {
+            own[k] = KPT * tid + k < SB_KEYS ? start[KPT * tid + k] : 0;
+            before += own[k];
+        }
+        int incl = before;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(incl, o);
+            if (lane >= o) incl += t;
+        }
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        int base = incl - before;
+#pragma unroll
+        for (int w = 0; w < NW; w++)
+            if (w < wave) base += wsum[w];
+#pragma unroll
+        for (int k = 0; k < KPT; k++) {
+            if (KPT * tid + k <= SB_KEYS) start[KPT * tid + k] = base;
+            base += own[k];
+        }
+    };
+    int n = cnt, lo = 0, hi = cnt;
     if (nch > 1) {
+        // this chunk's cells: a stretch of the tile's vertices in the order of
+        // their cells (a share by the cells' numbers alone gave a flat membrane
+        // that runs diagonally through the tile to one chunk whole)
+        for (int i = tid; i < cnt; i += WG_) {
+            const int k = key_of(node0[off + i]);
+            if (k >= 0) atomicAdd(&start[k], 1);
+        }
+        __syncthreads();
+        scan_keys();
+        __syncthreads();
+        const int all = __builtin_amdgcn_readfirstlane(start[SB_KEYS]);
+        lo = (int)((long long)all * chunk / nch);
+        hi = (int)((long long)all * (chunk + 1) / nch);
 #pragma unroll 2
         for (int i0 = 0; i0 < cnt; i0 += WG_) {  // whole waves: one counter update per wave
             const int i = i0 + tid;
-            const bool take = i < cnt && key_of(node0[off + min(i, cnt - 1)]) >= 0;
+            const int k = key_of(node0[off + min(i, cnt - 1)]);
+            const bool take = i < cnt && k >= 0 && start[max(k, 0)] >= lo && start[max(k, 0)] < hi;
             const unsigned long long m = __ballot(take);
             int at = 0;
             if (lane == 0) at = atomicAdd(&nsel, __popcll(m));
@@ -745,9 +788,13 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
             if (take && at < SB_CAP) wk.id[at] = i;
         }
         __syncthreads();
-        n = nsel;
+        n = __builtin_amdgcn_readfirstlane(nsel);
     }
     const bool sorted = n <= SB_CAP;
+    if (nch > 1 && sorted) {
+        for (int k = tid; k <= SB_KEYS; k += WG_) start[k] = 0;
+        __syncthreads();
+    }
     // this thread's vertices, all loads first
     int key[SB_VPT], id[SB_VPT], r[SB_VPT];
     SpreadRec<T> sr[SB_VPT];
@@ -790,35 +837,10 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
     for (int o = 32; o > 0; o >>= 1) fm = fmaxf(fm, __shfl_xor(fm, o));
     if (lane == 0) wmax[wave] = fm;
     __syncthreads();
-    // exclusive scan of the key counts, KPT consecutive keys per thread
-    {
-        int own[KPT], before = 0;
+    if (sorted) scan_keys();  // otherwise the tile's own scan stays, for the bounds
+    fm = wmax[0];
 #pragma unroll
-        for (int k = 0; k < KPT; k++) {
-            own[k] = KPT * tid + k < SB_KEYS ? start[KPT * tid + k] : 0;
-            before += own[k];
-        }
-        int incl = before;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(incl, o);
-            if (lane >= o) incl += t;
-        }
-        if (lane == 63) wsum[wave] = incl;
-        __syncthreads();
-        int base = incl - before;
-        fm = wmax[0];
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-            if (w < wave) base += wsum[w];
-            fm = fmaxf(fm, wmax[w]);
-        }
-#pragma unroll
-        for (int k = 0; k < KPT; k++) {
-            if (KPT * tid + k <= SB_KEYS) start[KPT * tid + k] = base;
-            base += own[k];
-        }
-    }
+    for (int w = 1; w < NW; w++) fm = fmaxf(fm, wmax[w]);
     // the float rounding of a double |f| may round down
     const double fmax = (double)fm * (1.0 + 0x1p-20);
     double scale = 1.0;
@@ -953,7 +975,7 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
         const T w1 = (T)(1.0 / (64.0 * g.dx * g.dx * g.dx));
         for (int i = tid; i < cnt; i += WG_) {
             const int kc = key_of(node0[off + i]);
-            if (kc < 0) continue;
+            if (kc < 0 || start[kc] < lo || start[kc] >= hi) continue;
             const SpreadRec<T> s = rec[off + i];
             T wx[4], wy[4], wz[4];
             stencil_weights<T>(s.t[0], wx);
@@ -1916,17 +1938,15 @@ BinGeom bin_geom(const lbmibm_ctx *ctx) {
 }
 
 // The offsets and orders of the tiles from their counts (k_tile_scan with no
-// force maxima, k_tile_order).
+// force maxima).
 lbmibm_status tile_offsets(lbmibm_ctx *ctx, hipStream_t stream, int nblk_fmax) {
     const IbmGeom g = geom_of(ctx);
     const TileGeom tg = tiles_of(ctx);
     hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->tile_off, ctx->tile_cur,
                        ctx->ntiles, ctx->blk_fmax, nblk_fmax, ctx->absmax, ctx->tile_ex, ctx->sb_extra,
-                       ctx->sb_maxextra);
+                       ctx->sb_maxextra, g, tg, ctx->tile_cand, ctx->order_spread, ctx->order_interp,
+                       ctx->order_calls);
     LBMIBM_LAUNCHED(ctx, "k_tile_scan");
-    hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->ntiles, g, tg,
-                       ctx->tile_cand, ctx->order_spread, ctx->order_interp, ctx->order_calls);
-    LBMIBM_LAUNCHED(ctx, "k_tile_order");
     return LBMIBM_OK;
 }
 
@@ -2184,13 +2204,6 @@ lbmibm_status ibm_setup(lbmibm_ctx *ctx) {
                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds64));
     LBMIBM_HIP(ctx, hipFuncSetAttribute((const void *)k_advect_adj_scatter<float>,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds64));
-    return LBMIBM_OK;
-}
-
-lbmibm_status ibm_count_begin(lbmibm_ctx *ctx, hipStream_t stream) {
-    hipLaunchKernelGGL(k_zero_int, dim3((ctx->ntiles + 255) / 256), dim3(256), 0, stream, ctx->tile_count,
-                       ctx->ntiles);
-    LBMIBM_LAUNCHED(ctx, "k_zero_int");
     return LBMIBM_OK;
 }
 

@@ -119,9 +119,13 @@ __device__ void cell_center(const double *__restrict__ xs, int nv, int v0, int v
 // would store it.
 __global__ __launch_bounds__(256) void k_vol_sums(const int4 *__restrict__ chunks, const double *__restrict__ xs,
                                                   int nv, const int *__restrict__ ele, const double *__restrict__ gx,
-                                                  double2 *__restrict__ part, VolArgs a) {
+                                                  double2 *__restrict__ part, VolArgs a, int *__restrict__ counts,
+                                                  int ncounts) {
     __shared__ double sh[128];
     WgReduce red{sh, 0};
+    // and the tile counters that k_vol_center adds to, cleared here instead of
+    // by a launch between the two (5 us a step)
+    for (int k = blockIdx.x * 256 + threadIdx.x; k < ncounts; k += gridDim.x * 256) counts[k] = 0;
     const int4 ch = chunks[blockIdx.x];
     const double g[3] = {gx[3 * ch.x], gx[3 * ch.x + 1], gx[3 * ch.x + 2]};
     double pv = 0.0, pa = 0.0;
@@ -311,10 +315,15 @@ __global__ __launch_bounds__(256) void k_vol_fin(const int4 *__restrict__ crange
 
 lbmibm_status run_impl(lbmibm_ctx *ctx, int mode, hipStream_t stream) {
     VolArgs a{ctx->nx * ctx->p.dx, ctx->ny * ctx->p.dx, ctx->nz * ctx->p.dx, ctx->p.periodic_y};
+    // the corrected positions are final until the next interpolation: they are
+    // counted into the spreading tiles here (spread form 1, whose scatter then
+    // needs no count of its own)
+    const bool count = mode == 1 && ctx->spread_form == 1 && ctx->nv > 0 && ctx->tile_count;
     if (mode == 1) {
         LBMIBM_KT(ctx, stream, "k_vol_sums",
                   hipLaunchKernelGGL(k_vol_sums, dim3(ctx->vol_ne), dim3(256), 0, stream, ctx->vol_echunks,
-                                     (const double *)ctx->xs, ctx->nv, ctx->ele, ctx->gx, ctx->vol_epart, a));
+                                     (const double *)ctx->xs, ctx->nv, ctx->ele, ctx->gx, ctx->vol_epart, a,
+                                     count ? ctx->tile_count : nullptr, count ? ctx->ntiles : 0));
         LBMIBM_LAUNCHED(ctx, "k_vol_sums");
     }
     // cells of up to VOL_SMALL vertices with 256 threads, larger ones with
@@ -347,14 +356,6 @@ lbmibm_status run_impl(lbmibm_ctx *ctx, int mode, hipStream_t stream) {
         LBMIBM_HIP(ctx, hipStreamWaitEvent(ctx->stream, ctx->ev_vjoin, 0));
     }
     if (mode == 1) {
-        // the corrected positions are final until the next interpolation:
-        // count them into the spreading tiles here (spread form 1, whose
-        // scatter then needs no count of its own)
-        const bool count = ctx->spread_form == 1 && ctx->nv > 0 && ctx->tile_count;
-        if (count) {
-            lbmibm_status s = ibm_count_begin(ctx, stream);
-            if (s != LBMIBM_OK) return s;
-        }
         const BinGeom bg{ctx->nx, ctx->ny, ctx->nz, ctx->nxp, ctx->nyp, ctx->nzp, ctx->p.periodic_y == 0,
                          ctx->ntx, ctx->nty, ctx->tile_x, ctx->p.dx};
         LBMIBM_KT(ctx, stream, "k_vol_center",

@@ -334,3 +334,23 @@ def test_front_tracking_of_several_stretches_per_group():
     keep = o.bc != 2
     assert rel(g.vf()[keep], o.vf[keep]) < 1e-10  # the same iterate of the same sweeps
     g.close()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("normal", [(1, 1, -1), (1, 2, 3), (0, 0, 1)])
+def test_spread_of_a_flat_membrane_through_full_tiles(normal, prec, monkeypatch):
+    """Vertices on a plane through one tile, which is shared out: the plane's
+    cells are a few diagonals, rows or one layer of the tile."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
+    lx, ly, lz = 40, 32, 40
+    print(f"[membrane] {normal} {prec}", flush=True)
+    cells, pos = _crowded(lx, ly, lz, [4], 5, (9.0, 9.0, 9.0), (16.9, 16.9, 16.9))
+    n = np.array(normal, float)
+    mid = [13.0 - (m - 1) / 2.0 for m in (lx, ly, lz)]
+    off = sum(a * (p - c) for a, p, c in zip(n, pos, mid)) / (n @ n)
+    pos = [np.clip(p - a * off, c - 3.9, c + 3.9) for p, a, c in zip(pos, n, mid)]
+    rng = np.random.default_rng(4)
+    forces = [1e-3 * rng.standard_normal(pos[0].size) for _ in range(3)]
+    F, ref = _spread_both(lx, ly, lz, prec, cells, pos, forces)
+    for a, b in zip(F, ref):
+        assert rel(a, b) < SPREAD_TOL[prec]
