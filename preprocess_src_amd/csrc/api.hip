@@ -722,6 +722,7 @@ lbmibm_status lbmibm_create(const lbmibm_params *p, const lbmibm_cells *cells, l
         CK(lattice_fill(ctx, ctx->rho, (size_t)N, 1.0, false));
         CK(lattice_fill(ctx, ctx->rhom, (size_t)N, 1.0, false));
     }
+    staging_reserve(ctx);
     CK(set_step(ctx, 0, false));
     CK(membrane_autotune(ctx));
     CK(ibm_autotune(ctx));

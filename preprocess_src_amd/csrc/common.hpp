@@ -366,6 +366,7 @@ struct FieldOut {
 lbmibm_status download_fields(lbmibm_ctx *ctx, const FieldOut *out, int n, size_t elem, bool images, bool zero);  // download.hip
 lbmibm_status download_arrays(lbmibm_ctx *ctx, const FieldOut *out, int nout, size_t elem, size_t n);  // download.hip
 lbmibm_status staging_init(lbmibm_ctx *ctx);                 // download.hip
+void staging_reserve(lbmibm_ctx *ctx);                       // download.hip
 void staging_free(lbmibm_ctx *ctx);                          // download.hip
 lbmibm_status vof_alloc(lbmibm_ctx *ctx);                    // vof.hip
 lbmibm_status vof_front_tracking(lbmibm_ctx *ctx, int *iterations, int *attempts);  // vof.hip (host sync)

@@ -20,8 +20,8 @@
 namespace lbmibm {
 
 // Ring of a context: RING pieces of at most PIECE bytes (one lattice row where
-// that is longer), allocated at the first download (pinning costs 0.2 ms per
-// MB), freed with the context.
+// that is longer), allocated with the context (pinning costs 0.2 ms per MB)
+// and freed with it.
 constexpr size_t PIECE = 512 << 10;
 constexpr int RING = 8;
 // Threads besides the caller's: one for every 8 MB, at most 4.  On three fields
@@ -66,6 +66,13 @@ static lbmibm_status staging_room(lbmibm_ctx *ctx, size_t piece) {
     LBMIBM_HIP(ctx, hipHostMalloc(&st->buf, RING * piece, hipHostMallocPortable));
     st->piece = piece;
     return LBMIBM_OK;
+}
+
+void staging_reserve(lbmibm_ctx *ctx) {
+    if (staging_room(ctx, 1) != LBMIBM_OK) {  // the first download tries again
+        (void)hipGetLastError();
+        ctx->err.clear();
+    }
 }
 
 // Copies pieces 0..n-1 (source(i, &bytes) names piece i) and hands each to
