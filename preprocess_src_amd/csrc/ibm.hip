@@ -2223,6 +2223,7 @@ static bool spread_box_tables(const lbmibm_ctx *ctx, std::vector<int> &out) {
     const int n[3] = {ctx->nx, ctx->ny, ctx->nz}, nt[3] = {ctx->ntx, ctx->nty, ctx->ntz};
     const int tile[3] = {ctx->tile_x, TILE_Y, TILE_Z}, R[3] = {ctx->tile_x + 3, SB_Y, SB_Z};
     const bool wrap[3] = {true, ctx->p.periodic_y != 0, true};
+    if (n[0] < 5) return false;  // rows that a box of TILE_XW + 3 nodes meets more than SB_MAXC times
     out.assign((size_t)SB_MAXC * (n[0] + n[1] + n[2]), -1);
     size_t base = 0;
     for (int a = 0; a < 3; a++) {
