@@ -219,7 +219,8 @@ struct lbmibm_ctx {
     int bicg_var[3] = {0, 0, 0};  // shape variant of the on-chip classes, form of class 2 (autotuned)
     int interp_form = 0;          // 0: tiles staged in LDS, 1: one thread per vertex, rows from memory (autotuned)
     int spread_form = 0;          // 0: source bins per tile, 1: home boxes + gather (autotuned)
-    void *sbox = nullptr;         // [ntiles + sb_maxextra][3][SB_N] staging boxes of spread form 1
+    void *sbox = nullptr;         // [ntiles][3][SB_N] staging boxes of spread form 1
+    void *sb_chunks = nullptr;    // [2 sb_maxextra] fixed-point boxes of the tiles that are shared out
     int *tile_ex = nullptr;       // [ntiles] first extra chunk of each tile (spread form 1)
     int2 *sb_extra = nullptr;     // [sb_maxextra] tile and chunk of the extra work groups, (-1, 0) unused
     int sb_maxextra = 0;

@@ -670,15 +670,26 @@ constexpr int SPREAD_BOX_WG = 512;
 constexpr int SB_MAXC = 4;  // box entries per lattice coordinate and axis (k_spread_gather)
 constexpr int SB_KEYS = TILE_X * SB_Y * TILE_Z;  // cells of a tile; y from -3 (below the wall in the first tile row)
 // A tile of more than SB_CHUNK vertices is shared out by its cells between
-// several work groups, each with a box of its own (the tile's own one and
-// extra ones, which k_spread_combine adds to it): 64 cells of radius 4 fill 159 of
-// 1024 tiles with up to 2490 vertices, and the launch would end with the fullest.
-// SPAN: sorted vertices per wave and batch; with these two work groups fit a
+// several work groups, each with a box of its own, which k_spread_combine adds
+// up: 64 cells of radius 4 fill 159 of 1024 tiles with up to 2490 vertices, and
+// the launch would end with the fullest.  Those boxes stay in fixed point (ChunkBox),
+// so that the tile's sum is rounded to T once, as that of a tile of one chunk.
+// SPAN: sorted vertices per wave and batch; with these three work groups fit a
 // CU's LDS.
 constexpr int SB_VPT = 2, SB_CAP = SB_VPT * SPREAD_BOX_WG;
 template <typename T> constexpr int SB_SPAN = sizeof(T) == 4 ? 32 : 16;
 static_assert(SB_CAP > SB_CHUNK, "the sort takes a chunk and a spread about it");
 typedef double double_x4 __attribute__((ext_vector_type(4)));
+
+// The fixed-point sums of one chunk of a tile that is shared out, and their
+// scale: a power of two, or infinity where the chunk's forces are all 0 (and 0
+// where one is infinite, which gives a tile without finite sums).  The boxes of the
+// extra chunks first, at the number of the chunk; behind them those of the
+// first chunks, at the number of the tile's first extra chunk.
+struct ChunkBox {
+    long long v[3 * SB_N];
+    double scale;
+};
 
 template <typename T>
 __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_spread_box(const SpreadRec<T> *__restrict__ rec,
@@ -687,7 +698,9 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
                                                               const int *__restrict__ tile_count,
                                                               const int *__restrict__ tile_off, T *__restrict__ S,
                                                               IbmGeom g, TileGeom tg, const int *__restrict__ order,
-                                                              const int2 *__restrict__ extra, int maxextra) {
+                                                              const int2 *__restrict__ extra, int maxextra,
+                                                              const int *__restrict__ tile_ex,
+                                                              ChunkBox *__restrict__ chunks) {
     constexpr int WG_ = SPREAD_BOX_WG, NW = WG_ / 64, SPAN = SB_SPAN<T>, BATCH = NW * SPAN;
     constexpr int KPT = (SB_KEYS + WG_) / WG_;  // keys per thread of the scan, and the total
     // REC values per sorted vertex: sin and cos of the x, y and z fractions, the
@@ -705,15 +718,14 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
     __shared__ int wsum[NW], nsel;
     __shared__ float wmax[NW];
     // the extra chunks of full tiles first, then every tile's first chunk
-    int tile, chunk = 0, slot;
+    int tile, chunk = 0;
     if ((int)blockIdx.x < maxextra) {
         const int2 ex = extra[blockIdx.x];
         if (ex.x < 0) return;  // not so many chunks
         tile = ex.x;
         chunk = ex.y;
-        slot = tg.ntiles + blockIdx.x;
     } else {
-        tile = slot = order[blockIdx.x - maxextra];
+        tile = order[blockIdx.x - maxextra];
     }
     const int cnt = tile_count[tile], off = tile_off[tile];
     if (cnt == 0) return;  // whole work group leaves together; the gather skips empty tiles
@@ -994,35 +1006,79 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
         __syncthreads();
     }
     const double inv_scale = 1.0 / scale;
-    T *St = S + (size_t)slot * 3 * SB_N;
+    T *St = S + (size_t)tile * 3 * SB_N;
+    ChunkBox *box = chunks + (nch == 1 ? 0 : chunk > 0 ? (int)blockIdx.x : maxextra + tile_ex[tile]);
     for (int k0 = tid; k0 < 3 * SB_N; k0 += 4 * WG_) {  // four reads, then four stores
         unsigned long long a[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) a[j] = acc[min(k0 + j * WG_, 3 * SB_N - 1)];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (k0 + j * WG_ < 3 * SB_N) St[k0 + j * WG_] = (T)FixedPoint<T>::real(a[j], inv_scale);
+        for (int j = 0; j < 4; j++) {
+            const int k = k0 + j * WG_;
+            if (k >= 3 * SB_N) continue;
+            if (nch > 1) box->v[k] = FixedPoint<T>::value(a[j]);
+            else St[k] = (T)FixedPoint<T>::real(a[j], inv_scale);
+        }
     }
+    if (nch > 1 && tid == 0) box->scale = fmax > 0.0 ? scale : HUGE_VAL;
 }
 
-// Adds the extra boxes of each tile that was shared out to the tile's own box,
-// chunk by chunk: work group e takes the tile whose first extra chunk is e, the
-// others leave at once (5 us on 64 cells, 15 us on the 1024-cell suspension).
-// The gather adding them itself took 64 instead of 44 us on that suspension:
-// the loop over chunks keeps its loads from being issued together.
+// Adds the chunks' boxes of each tile that was shared out into the tile's box:
+// work groups (e, .) take the tile whose first extra chunk is e, the others
+// leave at once.  The sum is formed in fixed point at the coarsest of the chunks'
+// scales, which is the one that all of the tile's vertices in one work group would
+// have had, and rounded to T at the end; boxes rounded to FP32 and added in FP32
+// lost up to 2.8 times as much where the chunks' sums cancel.  That costs twice
+// the bytes: 64 cells 5.8 -> 7.9 us here and 33.5 -> 34.2 in k_spread_box, the
+// 1024-cell suspension 13.4 -> 20.5 and 198 -> 205.  The boxes are read once: past
+// the caches, or they would drive out those that the gather reads next (62 instead
+// of 55 us).  The gather adding the chunks itself took 64 instead of 44 us: the
+// loop over them keeps its loads from being issued together.
+constexpr int COMBINE_WG = 256, COMBINE_PER = 4;  // threads and values of each; blockIdx.y: stretch of the box
+constexpr int COMBINE_PARTS = (3 * SB_N + COMBINE_WG * COMBINE_PER - 1) / (COMBINE_WG * COMBINE_PER);
 template <typename T>
-__global__ __launch_bounds__(1024) void k_spread_combine(T *__restrict__ S, const int2 *__restrict__ extra,
-                                                         const int *__restrict__ tile_count, int ntiles) {
+__global__ __launch_bounds__(COMBINE_WG) void k_spread_combine(T *__restrict__ S, const ChunkBox *__restrict__ chunks,
+                                                         const int2 *__restrict__ extra,
+                                                         const int *__restrict__ tile_count, int maxextra) {
     const int2 ex = extra[blockIdx.x];
     if (ex.x < 0 || ex.y != 1) return;
     const int nx = spread_chunks(tile_count[ex.x]) - 1;
-    T *own = S + (size_t)ex.x * 3 * SB_N;
-    const T *more = S + (size_t)(ntiles + blockIdx.x) * 3 * SB_N;
-    for (int k = threadIdx.x; k < 3 * SB_N; k += 1024) {
-        T a = own[k];
-        for (int c = 0; c < nx; c++) a += more[(size_t)c * 3 * SB_N + k];
-        own[k] = a;
+    const ChunkBox *first = chunks + maxextra + blockIdx.x, *more = chunks + blockIdx.x;
+    // the coarsest scale (positive doubles order as their bits)
+    __shared__ unsigned long long coarsest;
+    if (threadIdx.x == 0) coarsest = (unsigned long long)__double_as_longlong(first->scale);
+    __syncthreads();
+    for (int c = threadIdx.x; c < nx; c += COMBINE_WG)
+        atomicMin(&coarsest, (unsigned long long)__double_as_longlong(more[c].scale));
+    constexpr int PER = COMBINE_PER;
+    const int k0 = (int)blockIdx.y * COMBINE_WG * PER + (int)threadIdx.x;
+    int k[PER];
+    long long v[PER], sum[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        k[j] = min(k0 + COMBINE_WG * j, 3 * SB_N - 1);
+        v[j] = __builtin_nontemporal_load(&first->v[k[j]]);
+        sum[j] = 0;
     }
+    __syncthreads();
+    const double scale = __longlong_as_double((long long)coarsest);
+    const int e = ilogb(scale);
+    for (int c = 0; c <= nx; c++) {  // the next box's values while these are added
+        const double t = c == 0 ? first->scale : more[c - 1].scale;
+        // at most 62: a chunk without forces, at infinity, holds zeros
+        const int sh = scale > 0.0 ? (int)min((long long)ilogb(t) - e, 62ll) : 0;
+        const long long half = sh > 0 ? 1ll << (sh - 1) : 0;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            sum[j] += (v[j] + half) >> sh;
+            if (c < nx) v[j] = __builtin_nontemporal_load(&more[c].v[k[j]]);
+        }
+    }
+    const double inv = 1.0 / scale;
+    T *own = S + (size_t)ex.x * 3 * SB_N;
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+        if (k0 + COMBINE_WG * j < 3 * SB_N) own[k[j]] = (T)((double)sum[j] * inv);
 }
 
 // Spreading, form 1, point by point (lbmibm_ctx::pointwise): every vertex adds
@@ -1998,11 +2054,12 @@ template <typename T> lbmibm_status spread_launch(lbmibm_ctx *ctx, int form) {
                                          ctx->stream,
                                          (const SpreadRec<T> *)ctx->srec, ctx->node0, ctx->home_list, ctx->tile_count,
                                          ctx->tile_off, (T *)ctx->sbox, g, tg, ctx->order_interp, ctx->sb_extra,
-                                         ctx->sb_maxextra));
+                                         ctx->sb_maxextra, ctx->tile_ex, (ChunkBox *)ctx->sb_chunks));
             LBMIBM_LAUNCHED(ctx, "k_spread_box");
             if (ctx->sb_maxextra > 0) {
-                hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra), dim3(1024), 0,
-                                   ctx->stream, (T *)ctx->sbox, ctx->sb_extra, ctx->tile_count, ctx->ntiles);
+                hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra, COMBINE_PARTS), dim3(COMBINE_WG), 0,
+                                   ctx->stream, (T *)ctx->sbox, (const ChunkBox *)ctx->sb_chunks, ctx->sb_extra,
+                                   ctx->tile_count, ctx->sb_maxextra);
                 LBMIBM_LAUNCHED(ctx, "k_spread_combine");
             }
         }
@@ -2258,8 +2315,9 @@ static lbmibm_status spread_box_setup(lbmibm_ctx *ctx, bool *ok) {
         LBMIBM_HIP(ctx, hipMemcpy(ctx->sb_cand, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     if (!ctx->sbox) {
-        lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)(ctx->ntiles + ctx->sb_maxextra) * 3 *
-                                                              (ctx->pointwise ? SP_N : SB_N) * ctx->szT);
+        lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)ctx->ntiles * 3 * (ctx->pointwise ? SP_N : SB_N) * ctx->szT);
+        if (s == LBMIBM_OK && ctx->sb_maxextra > 0)
+            s = dev_alloc(ctx, &ctx->sb_chunks, 2 * (size_t)ctx->sb_maxextra * sizeof(ChunkBox));
         if (s != LBMIBM_OK) return s;
     }
     *ok = true;

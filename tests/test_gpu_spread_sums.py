@@ -1,0 +1,85 @@
+"""The sums of the spreading: what they are rounded to, and that their bits do
+not depend on the order in which the binning places the vertices."""
+import numpy as np
+import pytest
+
+from tests.pairs import gpu_of
+from tests.test_gpu_paths import CROWDS, _crowded
+
+pytestmark = pytest.mark.gpu
+
+SHAPE = (48, 40, 40)
+EPS = {"f64": 2.0 ** -53, "f32": 2.0 ** -24}  # half a unit in the last place, relative
+
+
+def _on_nodes(level, lo, hi, seed, on_node=None):
+    """One cell whose vertices sit on lattice nodes lo <= i <= hi: their weights
+    are 1/4, 1/2, 1/4 per axis, with no rounding."""
+    from preprocess_src_amd import mesh
+    cells = mesh.assemble([level], np.zeros((1, 3)), np.eye(3)[None], 3.0)
+    rng = np.random.default_rng(seed)
+    n = cells["x"].size
+    at = np.stack([rng.integers(a, b + 1, n) for a, b in zip(lo, hi)], 1)
+    return cells, at, [at[:, d] - (SHAPE[d] - 1) / 2.0 for d in range(3)]
+
+
+def _exact(at, force):
+    """Sums of the forces on each node with those weights, and of their absolute
+    values: whole numbers of 2^-6 of the force's unit, in 64-bit integers."""
+    lx, ly, lz = SHAPE
+    s, a = np.zeros((2, lz, ly, lx), np.int64)
+    w = {-1: 1, 0: 2, 1: 1}
+    for i in w:
+        for j in w:
+            for k in w:
+                q = w[i] * w[j] * w[k]
+                idx = (at[:, 2] + k, at[:, 1] + j, at[:, 0] + i)
+                np.add.at(s, idx, q * force)
+                np.add.at(a, idx, q * np.abs(force))
+    return s, a
+
+
+def _spread(prec, cells, pos, forces):
+    g = gpu_of(*SHAPE, prec, cells=cells)
+    g.set_cells_state(x=pos[0], y=pos[1], z=pos[2], fx=forces[0], fy=forces[1], fz=forces[2])
+    g.ibm_st1()
+    F = [f.reshape(SHAPE[2] + 4, SHAPE[1] + 4, SHAPE[0] + 4)[2:-2, 2:-2, 2:-2] for f in g.lattice_force()]
+    g.close()
+    return F
+
+
+# vertices of one tile (nodes 9..16 of each axis, whose stencils start in 8..15)
+# below the share of 800, shared out between 4 and 13 work groups, and in so few
+# lattice cells that a chunk does not fit the sort
+FULL = [(3, (9, 9, 9), (16, 16, 16)), (4, (9, 9, 9), (16, 16, 16)), (5, (9, 9, 9), (16, 16, 16)),
+        (5, (11, 12, 12), (12, 13, 12))]
+
+
+@pytest.mark.parametrize("signs", ["one", "by stretch"])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("k", range(len(FULL)))
+def test_sum_of_one_tile_is_rounded_once(k, prec, signs, monkeypatch):
+    """The forces of a tile's vertices on a node, whole numbers here, are summed
+    exactly and rounded once, however many work groups share the tile: half a
+    unit in the last place of the result and the quantum of the fixed point
+    (one per term: 2^-46 of the bound that the scale is taken from in FP32,
+    2^-61 in FP64)."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
+    level, lo, hi = FULL[k]
+    print(f"[one tile] {k} {prec} {signs}", flush=True)
+    cells, at, pos = _on_nodes(level, lo, hi, 3 + k)
+    n = len(at)
+    rng = np.random.default_rng(k)
+    forces = []
+    for _ in range(3):
+        f = rng.integers(1, 1 << 22, n)
+        if signs != "one":  # the sums of the lower and the upper half nearly cancel
+            f = np.where(at[:, 2] <= (lo[2] + hi[2]) / 2 if hi[2] > lo[2] else at[:, 0] <= lo[0], f, -f)
+        forces.append(f)
+    F = _spread(prec, cells, pos, [f.astype(np.float64) for f in forces])
+    bound = n * float(1 << 22) / 8.0
+    quantum = n * bound * 2.0 ** (-46 if prec == "f32" else -61)
+    for got, f in zip(F, forces):
+        s, _ = _exact(at, f)
+        want = s / 64.0  # exact: fewer than 53 bits
+        assert np.all(np.abs(got - want) <= EPS[prec] * np.abs(want) + quantum)
