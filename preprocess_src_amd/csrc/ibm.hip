@@ -31,6 +31,8 @@
 //   - Interpolation: one work group per tile stages the velocity of the tile
 //     plus a 3/4-node halo in LDS once and runs the four frozen-field RK
 //     stages of its vertices from LDS, one lane per vertex.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace lbmibm {
@@ -1159,7 +1161,10 @@ __global__ __launch_bounds__(SPREAD_BOX_WG) void k_spread_points(const SpreadRec
 // Sums, per lattice node, the box entries of k_spread_box that map to it, in
 // a fixed order (deterministic).  cx/cy/cz list for each coordinate of an axis
 // up to SB_MAXC entries (tile index along the axis) * 32 + box coordinate,
-// padded with -1 (built once on the host).
+// padded with -1 (built once on the host).  The boxes are added in FP64 and the sum
+// is rounded to T once: tiles of 8 nodes put more of them into a node than those of
+// 16 did.  Boxes of 16x8x8 tiles (lbmibm_ctx::pointwise) are added in T, as they
+// always were.
 template <typename T, int TX>
 __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, const int *__restrict__ tile_count,
                                                        const int *__restrict__ cx, const int *__restrict__ cy,
@@ -1186,7 +1191,8 @@ __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, 
         ey[i] = cy[SB_MAXC * y + i];
         ez[i] = cz[SB_MAXC * z + i];
     }
-    T a0 = T(0), a1 = T(0), a2 = T(0);
+    using Sum = std::conditional_t<TX == TILE_X, double, T>;
+    Sum a0 = Sum(0), a1 = Sum(0), a2 = Sum(0);
 #pragma unroll
     for (int iz = 0; iz < SB_MAXC; iz++) {
         if (ez[iz] < 0) break;
@@ -1214,9 +1220,9 @@ __global__ __launch_bounds__(256) void k_spread_gather(const T *__restrict__ S, 
                 if (cnt[ix] > 0) { a0 += v0[ix]; a1 += v1[ix]; a2 += v2[ix]; }
         }
     }
-    F[n] = a0;
-    F[N + n] = a1;
-    F[2 * N + n] = a2;
+    F[n] = (T)a0;
+    F[N + n] = (T)a1;
+    F[2 * N + n] = (T)a2;
 }
 
 // ---- interpolation + advection ------------------------------------------------

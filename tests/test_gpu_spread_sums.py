@@ -83,3 +83,24 @@ def test_sum_of_one_tile_is_rounded_once(k, prec, signs, monkeypatch):
         s, _ = _exact(at, f)
         want = s / 64.0  # exact: fewer than 53 bits
         assert np.all(np.abs(got - want) <= EPS[prec] * np.abs(want) + quantum)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_sum_of_several_tiles_is_rounded_once(prec, monkeypatch):
+    """Vertices around a corner of eight tiles, forces so small in whole numbers
+    that every tile's sums fit 24 bits: the nodes that several tiles add to hold
+    the exact sum rounded once."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
+    print(f"[eight tiles] {prec}", flush=True)
+    cells, at, pos = _on_nodes(3, (15, 15, 15), (18, 18, 18), 11)  # stencils start in 14..17, the tiles at 16
+    rng = np.random.default_rng(2)
+    forces = [rng.integers(1, 1 << 15, len(at)) for _ in range(3)]
+    tile = ((at >= 17) * [1, 2, 4]).sum(1)
+    for f in forces:
+        for t in range(8):
+            assert _exact(at[tile == t], f[tile == t])[1].max() < 1 << 24
+    F = _spread(prec, cells, pos, [f.astype(np.float64) for f in forces])
+    T = np.float32 if prec == "f32" else np.float64
+    for got, f in zip(F, forces):
+        want = (_exact(at, f)[0] / 64.0).astype(T)
+        assert np.array_equal(got, want.astype(np.float64))
