@@ -87,20 +87,23 @@ def test_sum_of_one_tile_is_rounded_once(k, prec, signs, monkeypatch):
 
 @pytest.mark.parametrize("prec", ["f64", "f32"])
 def test_sum_of_several_tiles_is_rounded_once(prec, monkeypatch):
-    """Vertices around a corner of eight tiles, forces so small in whole numbers
-    that every tile's sums fit 24 bits: the nodes that several tiles add to hold
-    the exact sum rounded once."""
+    """Vertices around a corner of eight tiles: whole-number forces whose sums
+    fit 24 bits in every tile's box, but not together.  The nodes hold the
+    exact sum rounded once."""
     monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
     print(f"[eight tiles] {prec}", flush=True)
-    cells, at, pos = _on_nodes(3, (15, 15, 15), (18, 18, 18), 11)  # stencils start in 14..17, the tiles at 16
-    rng = np.random.default_rng(2)
-    forces = [rng.integers(1, 1 << 15, len(at)) for _ in range(3)]
-    tile = ((at >= 17) * [1, 2, 4]).sum(1)
-    for f in forces:
-        for t in range(8):
-            assert _exact(at[tile == t], f[tile == t])[1].max() < 1 << 24
-    F = _spread(prec, cells, pos, [f.astype(np.float64) for f in forces])
+    cells, at, pos = _on_nodes(3, (16, 16, 16), (17, 17, 17), 11)  # stencils start in 15 and 16, the tiles at 16
+    tile = ((at == 17) * [1, 2, 4]).sum(1)
     T = np.float32 if prec == "f32" else np.float64
-    for got, f in zip(F, forces):
-        want = (_exact(at, f)[0] / 64.0).astype(T)
-        assert np.array_equal(got, want.astype(np.float64))
+    rng = np.random.default_rng(2)
+    wide = 0
+    for _ in range(8):
+        forces = [rng.integers(1 << 14, 1 << 15, len(at)) >> 1 for _ in range(3)]
+        F = _spread(prec, cells, pos, [f.astype(np.float64) for f in forces])
+        for got, f in zip(F, forces):
+            for t in range(8):
+                assert _exact(at[tile == t], f[tile == t])[1].max() < 1 << 24
+            s = _exact(at, f)[0]
+            wide += int((s >= 1 << 24).sum())
+            assert np.array_equal(got, (s / 64.0).astype(T).astype(np.float64))
+    assert wide >= 100  # sums that FP32 does not hold
