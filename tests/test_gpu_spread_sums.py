@@ -107,3 +107,29 @@ def test_sum_of_several_tiles_is_rounded_once(prec, monkeypatch):
             wide += int((s >= 1 << 24).sum())
             assert np.array_equal(got, (s / 64.0).astype(T).astype(np.float64))
     assert wide >= 100  # sums that FP32 does not hold
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("k", [1, 3, 4, 5])
+def test_home_boxes_do_not_depend_on_the_order_of_the_binning(k, prec, monkeypatch):
+    """Tiles of more than 800 vertices, cells of many, chunks beyond the sort's
+    capacity: every repeated binning places a tile's vertices in the order in
+    which its work groups arrive; the lattice force keeps its bits."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", "1")
+    levels, lo, hi = CROWDS[k]
+    print(f"[binning order] {k} {prec}", flush=True)
+    cells, pos = _crowded(*SHAPE, levels, 17 + k, lo, hi)
+    rng = np.random.default_rng(4)
+    n = pos[0].size
+    forces = [1e-3 * rng.standard_normal(n) * 10.0 ** rng.uniform(-4, 0, n) for _ in range(3)]
+    g = gpu_of(*SHAPE, prec, cells=cells)
+    first = None
+    for _ in range(8):
+        g.set_cells_state(x=pos[0], y=pos[1], z=pos[2], fx=forces[0], fy=forces[1], fz=forces[2])
+        g.ibm_st1()
+        F = np.concatenate(g.lattice_force())
+        if first is None:
+            first = F
+        assert np.array_equal(F, first)
+    g.close()
+    assert np.abs(first).max() > 0.0
