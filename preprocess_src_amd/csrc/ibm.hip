@@ -1624,10 +1624,108 @@ __global__ __launch_bounds__(256) void k_interp_vert(const T *__restrict__ U, co
 }
 
 // Interpolation point by point (lbmibm_ctx::pointwise): FP32 products summed in
-// the order of the stencil.  A lane keeps the 192 values of its cell, which
-// the stages nearly always share, and work groups of one wave spread the few
-// vertices of such runs over the chip (3204 of them: 25 us, 33 from tiles
-// in LDS, 47 with the rows of a z plane read again by every stage).
+// the order of the stencil, from row(kz, ky, component, kx).
+template <typename Row>
+__device__ __forceinline__ void point_sum(const float wx[4], const float wy[4], const float wz[4], float &ur,
+                                          float &vr, float &wr, Row row) {
+    ur = vr = wr = 0.0f;
+#pragma unroll
+    for (int kz = 0; kz < 4; kz++) {
+        const float wz64 = wz[kz] * (1.0f / 64.0f);
+#pragma unroll
+        for (int ky = 0; ky < 4; ky++) {
+            const float wyz = wy[ky] * wz64;
+#pragma unroll
+            for (int kx = 0; kx < 4; kx++) {
+                const float dlt = wx[kx] * wyz;
+                ur = fmaf(dlt, row(kz, ky, 0, kx), ur);
+                vr = fmaf(dlt, row(kz, ky, 1, kx), vr);
+                wr = fmaf(dlt, row(kz, ky, 2, kx), wr);
+            }
+        }
+    }
+}
+
+// Form 0: one work group per tile of TILE_XW nodes stages its velocity box in
+// LDS, and every stage reads its 64 nodes from there.  Form 1 (k_interp_points)
+// takes less on a few thousand vertices, which fill few tiles (64 cells of 2562: 43
+// instead of 88 us), this one on many (the 1024-cell suspension: 221 instead of
+// 410 us); both are timed at creation.  Stencils that leave the box read memory,
+// with the same products in the same order: the two forms give the same bits.
+constexpr int PX = TILE_XW + 5, PN = PX * RY * RZ;
+constexpr int POINT_WG = 512;
+__global__ __launch_bounds__(POINT_WG) void k_interp_point_tiles(
+    const float *__restrict__ U, const double *xin, double *xo, float *__restrict__ uvw, double *__restrict__ xd,
+    const int *__restrict__ tile_count, const int *__restrict__ tile_off, const int *__restrict__ home_list, int nv,
+    IbmGeom g, TileGeom tg, AdvectArgs a, const int *__restrict__ order) {
+    __shared__ float Us[3 * PN];  // [3][RZ][RY][PX]
+    const int tile = order[blockIdx.x];
+    const int cnt = tile_count[tile], off = tile_off[tile];
+    if (cnt == 0) return;  // whole work group leaves together
+    const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
+    const int bx = tx * TILE_XW - RLO, by = ty * TILE_Y - RLO, bz = tz * TILE_Z - RLO;
+    const size_t N = (size_t)g.nx * g.ny * g.nz;
+    for (int k = threadIdx.x; k < PN; k += POINT_WG) {
+        const int rx = k % PX, ry = (k / PX) % RY, rz = k / (PX * RY);
+        // the box may span an axis more than once on small lattices
+        const int ix = pmod(bx + rx, g.nx), iz = pmod(bz + rz, g.nz);
+        int iy = by + ry;
+        const bool ok = !g.walls || (iy >= 0 && iy < g.ny);
+        if (!g.walls) iy = pmod(iy, g.ny);
+        const size_t n = ok ? (size_t)ix + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz) : 0;
+#pragma unroll
+        for (int d = 0; d < 3; d++) Us[d * PN + k] = ok ? U[d * N + n] : 0.0f;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < cnt; i += POINT_WG) {
+        const int j = home_list[off + i];
+        advect_vertex<float>(
+            j, xin[j], xin[nv + j], xin[2 * (size_t)nv + j], xo, uvw, xd, nv, a,
+            [&](int, double x, double y, double z, bool unit, float &ur, float &vr, float &wr) {
+                int x1, y1, z1;
+                float wx[4], wy[4], wz[4];
+                stencil3<float>(g, x, y, z, unit, x1, y1, z1, wx, wy, wz);
+                int rx = x1 - bx, ry = y1 - by, rz = z1 - bz;
+                if (rx < 0) rx += g.nx; else if (rx >= g.nx) rx -= g.nx;
+                if (rz < 0) rz += g.nz; else if (rz >= g.nz) rz -= g.nz;
+                if (!g.walls) { if (ry < 0) ry += g.ny; else if (ry >= g.ny) ry -= g.ny; }
+                if (rx >= 0 && rx <= PX - 4 && ry >= 0 && ry <= RY - 4 && rz >= 0 && rz <= RZ - 4) {
+                    const float *box = Us + rx + PX * (ry + RY * rz);
+                    point_sum(wx, wy, wz, ur, vr, wr,
+                              [&](int kz, int ky, int d, int kx) { return box[d * PN + PX * (ky + RY * kz) + kx]; });
+                    return;
+                }
+                ur = vr = wr = 0.0f;
+#pragma unroll 1
+                for (int kz = 0; kz < 4; kz++) {
+                    int iz = z1 + kz;
+                    if (!wrap_index(iz, g.nz)) continue;
+                    const float wz64 = sel4(wz, kz) * (1.0f / 64.0f);
+#pragma unroll 1
+                    for (int ky = 0; ky < 4; ky++) {
+                        int iy = y1 + ky;
+                        if (!(g.walls ? iy >= 0 && iy < g.ny : wrap_index(iy, g.ny))) continue;
+                        const float wyz = sel4(wy, ky) * wz64;
+                        const float *u = U + (size_t)g.nx * ((size_t)iy + (size_t)g.ny * iz);
+#pragma unroll 1
+                        for (int kx = 0; kx < 4; kx++) {
+                            int ix = x1 + kx;
+                            if (!wrap_index(ix, g.nx)) continue;
+                            const float dlt = sel4(wx, kx) * wyz;
+                            ur = fmaf(dlt, u[ix], ur);
+                            vr = fmaf(dlt, u[N + ix], vr);
+                            wr = fmaf(dlt, u[2 * N + ix], wr);
+                        }
+                    }
+                }
+            });
+    }
+}
+
+// Form 1: a lane keeps the 192 values of its cell, which the stages nearly
+// always share, and work groups of one wave spread a few vertices over the chip
+// (3204 of them: 25 us, 33 from tiles in LDS, 47 with the rows of a z plane read
+// again by every stage).
 __global__ __launch_bounds__(64) void k_interp_points(const float *__restrict__ U, const double *xin, double *xo,
                                                       float *__restrict__ uvw, double *__restrict__ xd,
                                                       const int *__restrict__ home_list, int nv, IbmGeom g,
@@ -1678,22 +1776,7 @@ __global__ __launch_bounds__(64) void k_interp_points(const float *__restrict__ 
                     }
                 }
             }
-            ur = vr = wr = 0.0f;
-#pragma unroll
-            for (int kz = 0; kz < 4; kz++) {
-                const float wz64 = wz[kz] * (1.0f / 64.0f);
-#pragma unroll
-                for (int ky = 0; ky < 4; ky++) {
-                    const float wyz = wy[ky] * wz64;
-#pragma unroll
-                    for (int kx = 0; kx < 4; kx++) {
-                        const float dlt = wx[kx] * wyz;
-                        ur = fmaf(dlt, r[kz][ky][0][kx], ur);
-                        vr = fmaf(dlt, r[kz][ky][1][kx], vr);
-                        wr = fmaf(dlt, r[kz][ky][2][kx], wr);
-                    }
-                }
-            }
+            point_sum(wx, wy, wz, ur, vr, wr, [&](int kz, int ky, int d, int kx) { return r[kz][ky][d][kx]; });
         });
 }
 
@@ -2120,7 +2203,15 @@ lbmibm_status interp_launch(lbmibm_ctx *ctx, int form, const double *xin, double
     a.lx = ctx->nx * ctx->p.dx; a.ly = ctx->ny * ctx->p.dx; a.lz = ctx->nz * ctx->p.dx;
     a.rk = ctx->p.runge_kutta;
     a.periodic_y = ctx->p.periodic_y;
-    if (ctx->pointwise) {  // one form
+    if (ctx->pointwise && form == 0) {
+        LBMIBM_KT(ctx, ctx->stream, "k_interp_point_tiles",
+                  hipLaunchKernelGGL(k_interp_point_tiles, dim3(ctx->ntiles), dim3(POINT_WG), 0, ctx->stream,
+                                     (const float *)ctx->U, xin, xo, (float *)uvw, xd, ctx->tile_count, ctx->tile_off,
+                                     ctx->home_list, ctx->nv, geom_of(ctx), tiles_of(ctx), a, ctx->order_interp));
+        LBMIBM_LAUNCHED(ctx, "k_interp_point_tiles");
+        return LBMIBM_OK;
+    }
+    if (ctx->pointwise) {
         LBMIBM_KT(ctx, ctx->stream, "k_interp_points",
                   hipLaunchKernelGGL(k_interp_points, dim3((ctx->nv + 63) / 64), dim3(64), 0, ctx->stream,
                                      (const float *)ctx->U, xin, xo, (float *)uvw, xd, ctx->home_list, ctx->nv,
@@ -2396,7 +2487,7 @@ lbmibm_status ibm_autotune(lbmibm_ctx *ctx) {
     if (fi >= 0) {
         ctx->interp_form = fi;
         ctx->tune_report += "interp form fixed by LBMIBM_INTERP_FORM\n";
-    } else if (tune && !ctx->pointwise) {
+    } else if (tune) {
         s = ctx->prec == LBMIBM_F64 ? interp_autotune_impl<double>(ctx) : interp_autotune_impl<float>(ctx);
         if (s != LBMIBM_OK) return s;
     }
