@@ -271,9 +271,14 @@ __global__ __launch_bounds__(AWG) void k_adh_detach(AdhDev a, const double *__re
                                                     const DevStep *__restrict__ st, int init,
                                                     const int *__restrict__ klist, int nk,
                                                     unsigned long long *__restrict__ calls,
-                                                    unsigned long long *__restrict__ claim, long long nrec) {
+                                                    unsigned long long *__restrict__ claim, long long nrec,
+                                                    int *__restrict__ more, int *__restrict__ made) {
 #pragma clang fp contract(off)
-    if (blockIdx.x == 0) advance_calls(calls, claim, nrec, a.maxn);
+    if (blockIdx.x == 0) {
+        advance_calls(calls, claim, nrec, a.maxn);
+        if (threadIdx.x < 2) more[threadIdx.x] = 0;
+        for (int r = threadIdx.x; r <= a.maxn; r += AWG) made[r] = 0;
+    }
     const int t = blockIdx.x * AWG + threadIdx.x;
     if (t >= nk * a.ns) return;
     const int v = klist[t / a.ns], sid = v * a.ns + t % a.ns;
@@ -312,9 +317,21 @@ struct AdhRound {
     const unsigned long long *calls;
     const DevStep *st;
     int init, nk;
+    int *more, *list[2];  // [2] springs that go on after round 0, and after the rounds of k_adh_round: numbers, ids
+    int *made;            // [maxn + 1] whether a round of k_adh_round had proposals
 };
+// whether a receptor has a winner already; since_call: it may have one by a bid
+// of an earlier round of this call, which nobody has entered yet
+__device__ __forceinline__ bool adh_taken(const AdhDev &a, const AdhRound &q, int round, unsigned long long call,
+                                          bool since_call, int id) {
+    if (q.is_attached[id]) return true;
+    if (!since_call) return false;
+    const unsigned long long bid = q.claim[id];
+    // the smallest keys of round 0 and of this one: those of a spring above all ids
+    return bid >= bid_key(call, 0, a.maxn, -1) && bid < bid_key(call, round, a.maxn, -1);
+}
 __device__ __forceinline__ int adh_propose(const AdhDev &a, const AdhRound &q, int round, unsigned long long call,
-                                           int sid) {
+                                           int sid, bool since_call = false) {
     const int v = sid / a.ns;
     const double u = q.init ? 0.0 : adh_uniform(a.seed, q.st->iter, sid);
     int c = q.pos[sid], id = -1;
@@ -325,7 +342,7 @@ __device__ __forceinline__ int adh_propose(const AdhDev &a, const AdhRound &q, i
             double dr;
             if (p_on(a, q.r_wall[(size_t)v * a.maxn + c], dr) <= u) continue;
         }
-        if (q.is_attached[id]) continue;
+        if (adh_taken(a, q, round, call, since_call, id)) continue;
         break;
     }
     if (c >= a.maxn) {
@@ -336,8 +353,8 @@ __device__ __forceinline__ int adh_propose(const AdhDev &a, const AdhRound &q, i
     atomicMax(q.claim + id, bid_key(call, round, a.maxn, sid));
     return id;
 }
-// The highest bid takes the receptor, the others go on to their next candidate.
-__device__ __forceinline__ void adh_resolve(const AdhDev &a, const AdhRound &q, int round, unsigned long long call,
+// The highest bid takes the receptor (true), the others go on to their next candidate.
+__device__ __forceinline__ bool adh_resolve(const AdhDev &a, const AdhRound &q, int round, unsigned long long call,
                                             int sid, int id) {
     // bids are made in L2: read there
     if (__hip_atomic_load(q.claim + id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
@@ -350,44 +367,67 @@ __device__ __forceinline__ void adh_resolve(const AdhDev &a, const AdhRound &q, 
             q.r_ij[sid] = dr;
         }
         q.active[sid] = 0;
-    } else {
-        q.pos[sid] = q.pos[sid] + 1;
+        return true;
     }
+    q.pos[sid] = q.pos[sid] + 1;
+    return false;
 }
 
-// Round 0, which meets every free spring: a launch per half.
+// Round 0, which meets every free spring: a launch per half.  The losers are
+// listed (in any order: the bids decide) for the other rounds.
 __global__ __launch_bounds__(AWG) void k_adh_propose(AdhDev a, AdhRound q) {
     const int t = blockIdx.x * AWG + threadIdx.x;
     if (t >= q.nk * a.ns) return;
     const int sid = q.klist[t / a.ns] * a.ns + t % a.ns;
     q.prop[sid] = q.active[sid] ? adh_propose(a, q, 0, *q.calls, sid) : -1;
 }
+// The lanes' springs that are `on` behind those listed already; whole waves.
+__device__ __forceinline__ void adh_append(int *__restrict__ more, int *__restrict__ list, bool on, int sid) {
+    const int lane = threadIdx.x & 63;
+    const unsigned long long m = __ballot(on);
+    if (!m) return;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(more, __popcll(m));
+    at = __shfl(at, 0) + __popcll(m & ((1ull << lane) - 1ull));
+    if (on) list[at] = sid;
+}
 __global__ __launch_bounds__(AWG) void k_adh_resolve(AdhDev a, AdhRound q) {
     const int t = blockIdx.x * AWG + threadIdx.x;
-    if (t >= q.nk * a.ns) return;
-    const int sid = q.klist[t / a.ns] * a.ns + t % a.ns;
-    const int id = q.prop[sid];
-    if (id >= 0) adh_resolve(a, q, 0, *q.calls, sid, id);
+    int sid = 0;
+    bool lost = false;
+    if (t < q.nk * a.ns) {
+        sid = q.klist[t / a.ns] * a.ns + t % a.ns;
+        const int id = q.prop[sid];
+        lost = id >= 0 && !adh_resolve(a, q, 0, *q.calls, sid, id);
+        if (lost) q.prop[sid] = -1;
+    }
+    adh_append(q.more, q.list[0], lost, sid);
 }
 
-// The other rounds, which only the losers of the one before take part in, in
-// one work group that lists them and stops after a round without proposals.
-// A pair of launches for each of the MAXN + 1 rounds, most of them empty, took
-// 34 launches and about 95 us per step with MAXN = 16 (202 with the usual
-// 100); this takes 12 us, the first round 15.  Every spring advances or retires in every
-// round, so MAXN more rounds are enough.
-__global__ __launch_bounds__(1024) void k_adh_rounds(AdhDev a, AdhRound q, int *__restrict__ list) {
-    __shared__ int n, made;
-    if (threadIdx.x == 0) n = 0;
-    __syncthreads();
-    for (int t = threadIdx.x; t < q.nk * a.ns; t += 1024) {
-        const int sid = q.klist[t / a.ns] * a.ns + t % a.ns;
-        if (q.active[sid]) list[atomicAdd(&n, 1)] = sid;
-    }
-    __syncthreads();
-    const int m = n;
+// The other rounds, which only the losers of the one before take part in.
+// Every spring advances or retires in every round, so MAXN more rounds are
+// enough.  Here they run in one work group, which stops after a round without
+// proposals: `first` and the later ones of a list (0: the losers of round 0, where
+// they are at most `most`; 1: those of the rounds of k_adh_round).
+//
+// A pair of launches for each of the MAXN + 1 rounds, most of them empty, took 34
+// launches and 95 us per step for 64 cells with 40 knobs of 2 springs and
+// MAXN = 16 (27 now, 12 of them here).  But a thousand losers are what one CU
+// takes in the time of a launch: all rounds in one group took 2.45 ms of a step
+// with 363 000 springs and 34.7 ms with 1.8 million (MAXN = 100), 0.50 and 2.2
+// in pairs of launches, 0.22 and 0.95 now.  ROUNDS_SPRINGS: with 8100 springs, of
+// which a third is near the wall, the group alone takes 0.09 ms, the pairs took
+// 0.25; below, the nine or ten launches that find nothing to do would cost 20 us of
+// every step.
+constexpr int ROUNDS_GROUP = 1024;
+constexpr int ROUNDS_SPRINGS = 8192;  // springs up to which no other launches are made
+__global__ __launch_bounds__(1024) void k_adh_rounds(AdhDev a, AdhRound q, int which, int first, int most) {
+    __shared__ int made;
+    const int m = q.more[which];
+    const int *list = q.list[which];
+    if (m > most) return;
     const unsigned long long call = *q.calls;
-    for (int round = 1; round <= a.maxn; round++) {
+    for (int round = first; round <= a.maxn; round++) {
         if (threadIdx.x == 0) made = 0;
         __syncthreads();
         for (int k = threadIdx.x; k < m; k += 1024) {
@@ -401,10 +441,39 @@ __global__ __launch_bounds__(1024) void k_adh_rounds(AdhDev a, AdhRound q, int *
         if (!made) return;
         for (int k = threadIdx.x; k < m; k += 1024) {
             const int sid = list[k], id = q.prop[sid];
-            if (id >= 0) adh_resolve(a, q, round, call, sid, id);
+            if (id >= 0) (void)adh_resolve(a, q, round, call, sid, id);
         }
         __syncthreads();
     }
+}
+// More losers: a launch per round, over the whole chip, for the first few of
+// them.  A spring first learns how its bid of the round before ended, then makes
+// the next; receptors that somebody won in that round are told by the bids on them,
+// whether the winner has entered itself yet or not.  The `last` launch only
+// enters the winners, and lists the losers.  Eight launches: with four the
+// 1.8 million springs leave so many losers that a step takes 1 ms more, with six
+// 0.03; a launch for every round up to MAXN takes 0.25 ms more where MAXN is 100.
+constexpr int ROUND_GROUPS = 512, ROUND_LAUNCHES = 8;
+__global__ __launch_bounds__(AWG) void k_adh_round(AdhDev a, AdhRound q, int round, bool last, int most) {
+    const int m = q.more[0];
+    if (m <= most || (round > 1 && q.made[round - 1] == 0)) return;
+    const unsigned long long call = *q.calls;
+    bool any = false;
+    for (int k0 = blockIdx.x * AWG; k0 < m; k0 += ROUND_GROUPS * AWG) {  // whole waves
+        const int k = k0 + threadIdx.x;
+        const int sid = k < m ? q.list[0][k] : 0;
+        bool on = k < m && q.active[sid];
+        int id = on ? q.prop[sid] : -1;
+        if (id >= 0) on = !adh_resolve(a, q, round - 1, call, sid, id);
+        if (last) {
+            adh_append(q.more + 1, q.list[1], on, sid);
+        } else if (on) {
+            id = adh_propose(a, q, round, call, sid, true);
+            q.prop[sid] = id;
+            any = any || id >= 0;
+        }
+    }
+    if (__any(any) && (threadIdx.x & 63) == 0) q.made[round] = 1;
 }
 
 template <typename V> __global__ void k_afill(V *__restrict__ p, size_t n, V v) {
@@ -449,16 +518,25 @@ lbmibm_status adh_bell(lbmibm_ctx *ctx, int init) {
     const int *kl = ctx->adh_klist;
     const int nk = ctx->adh_nk;
     const AdhRound q{ctx->adh_idw, kl, ctx->adh_rw, ctx->adh_isatt, ctx->adh_attach, ctx->adh_pos, ctx->adh_active,
-                     ctx->adh_prop, ctx->adh_rij, ctx->adh_claim, ctx->adh_calls, (const DevStep *)ctx->step, init, nk};
+                     ctx->adh_prop, ctx->adh_rij, ctx->adh_claim, ctx->adh_calls, (const DevStep *)ctx->step, init, nk,
+                     ctx->adh_list, {ctx->adh_list + 2, ctx->adh_list + 2 + nsp}, ctx->adh_made};
     hipLaunchKernelGGL(k_adh_search, dim3(ablocks(64LL * nk)), dim3(AWG), 0, st, a, (const double *)ctx->xs, kl, nk,
                        ctx->adh_idw, ctx->adh_rw);
     hipLaunchKernelGGL(k_adh_detach, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, (const double *)ctx->xs,
                        (const unsigned char *)ctx->adh_knob, ctx->adh_attach, ctx->adh_rij, ctx->adh_isatt,
                        ctx->adh_pos, ctx->adh_active, (const DevStep *)ctx->step, init, kl, nk, ctx->adh_calls,
-                       ctx->adh_claim, (long long)a.nxw * a.nzw);
+                       ctx->adh_claim, (long long)a.nxw * a.nzw, q.more, q.made);
     hipLaunchKernelGGL(k_adh_propose, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, q);
     hipLaunchKernelGGL(k_adh_resolve, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, q);
-    hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, ctx->adh_list);
+    const bool few = nsp <= ROUNDS_SPRINGS;
+    const int most = few ? INT_MAX : ROUNDS_GROUP;
+    hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, 0, 1, most);
+    if (!few) {
+        const int n = std::min(ROUND_LAUNCHES, a.maxn);
+        for (int r = 1; r <= n + 1; r++)
+            hipLaunchKernelGGL(k_adh_round, dim3(ROUND_GROUPS), dim3(AWG), 0, st, a, q, r, r > n, most);
+        hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, 1, n + 1, INT_MAX);
+    }
     LBMIBM_LAUNCHED(ctx, "k_adh_*");
     return LBMIBM_OK;
 }
@@ -535,7 +613,7 @@ lbmibm_status adhesion_setup(lbmibm_ctx *ctx, const lbmibm_adhesion_params *h, c
         void **bufs[] = {&ctx->adh_knob, (void **)&ctx->adh_idw, (void **)&ctx->adh_rw, (void **)&ctx->adh_attach,
                          (void **)&ctx->adh_rij, (void **)&ctx->adh_pos, (void **)&ctx->adh_active,
                          (void **)&ctx->adh_prop, (void **)&ctx->adh_isatt, (void **)&ctx->adh_claim,
-                         (void **)&ctx->adh_calls, (void **)&ctx->adh_fadh, (void **)&ctx->adh_list,
+                         (void **)&ctx->adh_calls, (void **)&ctx->adh_fadh, (void **)&ctx->adh_list, (void **)&ctx->adh_made,
                          (void **)&ctx->adh_klist, &ctx->adh_fsum, (void **)&ctx->adh_ring};
         for (void **p : bufs) {
             if (*p) (void)hipFree(*p);
@@ -557,7 +635,8 @@ lbmibm_status adhesion_setup(lbmibm_ctx *ctx, const lbmibm_adhesion_params *h, c
     al((void **)&ctx->adh_claim, nrec * sizeof(unsigned long long));
     al((void **)&ctx->adh_calls, sizeof(unsigned long long));
     al((void **)&ctx->adh_fadh, 3 * nv * sizeof(double));
-    al((void **)&ctx->adh_list, std::max<size_t>(klist.size() * h->springs_per_knob, 1) * sizeof(int));
+    al((void **)&ctx->adh_list, (2 + 2 * klist.size() * h->springs_per_knob) * sizeof(int));
+    al((void **)&ctx->adh_made, (size_t)(h->max_neighwall + 2) * sizeof(int));
     al((void **)&ctx->adh_klist, std::max<size_t>(klist.size(), 1) * sizeof(int));
     al(&ctx->adh_fsum, 3 * nv * ctx->szT);
     std::vector<double> ring;

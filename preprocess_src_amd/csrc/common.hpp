@@ -308,7 +308,8 @@ struct lbmibm_ctx {
     double adh_dxw = 0.0, adh_dzw = 0.0;
     void *adh_knob = nullptr;
     int *adh_idw = nullptr, *adh_attach = nullptr, *adh_pos = nullptr, *adh_active = nullptr, *adh_prop = nullptr;
-    int *adh_isatt = nullptr, *adh_list = nullptr;  // list: springs that go on after the first round
+    int *adh_isatt = nullptr, *adh_list = nullptr;  // list: numbers and ids of the springs that go on to later rounds
+    int *adh_made = nullptr;                          // [MAXN + 2] rounds that had proposals
     unsigned long long *adh_claim = nullptr;          // per receptor: the highest bid key
     unsigned long long *adh_calls = nullptr;          // [1] calls of the Bell update so far
     int *adh_klist = nullptr, adh_nk = 0;  // the knob vertices

@@ -1,0 +1,40 @@
+"""Attachment rounds of so many springs that they run over the whole chip."""
+import numpy as np
+import pytest
+
+from tests.test_adhesion import LY, _knobs, _cell, _pair
+
+pytestmark = pytest.mark.gpu
+
+# more springs than one work group takes without further launches (8192), more
+# losers than it takes (1024): rounds beyond the eight launches, fewer of them than
+# launches, one; springs that find few receptors
+MANY = [dict(springs_per_knob=420, max_neighwall=100, receptor_density=16.0),
+        dict(springs_per_knob=420, max_neighwall=5), dict(springs_per_knob=420, max_neighwall=1),
+        dict(springs_per_knob=600, max_neighwall=9, receptor_density=1.0)]
+
+
+@pytest.mark.parametrize("k", range(len(MANY)))
+def test_rounds_of_many_springs(k):
+    """Lists and attachments are whole numbers: equal to the oracle's."""
+    print(f"[many springs] {MANY[k]}", flush=True)
+    assert int(_knobs(_cell()).sum()) * MANY[k]["springs_per_knob"] > 8192
+    o, g, st, nrec = _pair("f64", extra=MANY[k], tau=0.9, p=5e-6, b=5e-3)
+    X, Y, Z = o.node_coords()
+    vel = 4e-3 * (Y + LY / 2) / LY
+    vel[o.bc == 2] = 0.0
+    o.init_fluid(None, vel, None, None)
+    g.set_equilibrium(None, vel, None, None)
+    o.volume_init()
+    g.volume_init()
+    for it in range(5):
+        gs = g.adhesion_state(nrec)
+        for name in ("id_wall", "attach", "is_attached"):
+            assert np.array_equal(gs[name], st[name]), (it, name)
+        if it < 4:
+            assert o.step(it + 1)[0] == 0
+            g.step(it + 1)
+    near = (st["id_wall"].reshape(-1, MANY[k]["max_neighwall"])[:, 0] >= 0).sum()
+    assert near * MANY[k]["springs_per_knob"] > 2 * 1024
+    assert (st["attach"] >= 0).sum() > 5
+    g.close()
