@@ -168,12 +168,15 @@ __global__ __launch_bounds__(AWG) void k_adh_force(AdhDev a, const double *__res
 
 // StoreNeighWall_CUBE_GPU (adhesion.cu:109-206): receptors within LIMIT dx
 // of a knob near the wall, nearest first, ties in scan order, at most MAXN.
-// One wave per knob: its lanes test the candidates 64 at a time, list those in
-// range in scan order in LDS, and count for each one how many come before it.
-// One lane per vertex, inserting into a sorted list in memory, was a chain of
-// dependent reads for each candidate: 63 us for 64 cells with 20 to 40 knobs
-// each, 5 us now.
-constexpr int SEARCH_CAP = 192;  // receptors in range held in LDS per knob; more take the sorted insertion by one lane
+// One wave per knob: its lanes test the candidates 64 at a time and list those in
+// range in scan order in LDS.  When the list is full it is ranked (for each one, how
+// many come before it) and cut to the MAXN nearest, and from then on only
+// candidates nearer than the last of them are listed.  One lane per vertex,
+// inserting into a sorted list in memory, was a chain of dependent reads for each
+// candidate: 63 us for 64 cells with 20 to 40 knobs each, 5 us now.  With 64
+// receptors per unit area (more than 256 in range) the lane's insertion took 0.75 ms of
+// a step with MAXN = 16 and 4.3 ms with 100; this takes 0.04 and 0.12.
+constexpr int SEARCH_CAP = 256;  // entries in LDS per knob; lists that fill them (MAXN > 192) take the insertion by one lane
 __global__ __launch_bounds__(AWG) void k_adh_search(AdhDev a, const double *__restrict__ xs,
                                                     const int *__restrict__ klist, int nk, int *__restrict__ id_wall,
                                                     double *__restrict__ r_wall) {
@@ -209,56 +212,97 @@ __global__ __launch_bounds__(AWG) void k_adh_search(AdhDev a, const double *__re
         ra1 = min(a.nxw - 1, (int)ceil((xi + a.limit * a.dx) / a.dxw) + a.nxw / 2 + 1);
     }
     const int ncol = ra1 - ra0 + 1 + (rb1 - rb0 + 1);
-    const long long total = away || ncol <= 0 || span <= 0 ? 0 : 2LL * span * ncol;
-    // candidate n in scan order; false out of range
-    auto candidate = [&](long long n, int &id, double &r) {
-        int jz = iz + (int)(n / ncol) - (span - 1);
+    const int nrow = away || ncol <= 0 ? 0 : 2 * span;
+    // candidate (row, col) in scan order; false out of range
+    auto candidate = [&](int row, int col, int &id, double &r) {
+        int jz = iz + row - (span - 1);
         double zj = (jz - a.nzw / 2) * a.dzw;
         if (jz < 0) { jz += a.nzw; zj += a.lz; }
         else if (jz >= a.nzw) { jz -= a.nzw; zj -= a.lz; }
-        const int k = ra0 + (int)(n % ncol), jx = k <= ra1 ? k : rb0 + (k - ra1 - 1);
+        const int k = ra0 + col, jx = k <= ra1 ? k : rb0 + (k - ra1 - 1);
         id = jz * a.nxw + jx;
         double xj, yj, zr;
         receptor(a, id, xj, yj, zr);
         r = sqrt((xj - xi) * (xj - xi) + (yj - yi) * (yj - yi) + (zj - zi) * (zj - zi));
         return !(r > a.limit * a.dx);
     };
-    long long cnt = 0;
-    for (long long n0 = 0; n0 < total; n0 += 64) {
+    auto in_step = [] {  // the wave's LDS accesses before, and those after
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    int have = 0;
+    auto rank_of = [&](int i) {
+        const double r = lr[wave][i];
+        int rank = 0;
+        for (int j = 0; j < have; j++) rank += j < i ? !(lr[wave][j] > r) : r > lr[wave][j];
+        return rank;
+    };
+    bool full = false, serial = false;
+    double worst = 0.0;  // distance of the last of MAXN, where there are so many
+    const int nc = max(ncol, 1);
+    int row = lane / nc, col = lane % nc;
+    while (__any(row < nrow)) {
         int id = 0;
         double r = 0.0;
-        const bool in = n0 + lane < total && candidate(n0 + lane, id, r);
+        const bool in = row < nrow && candidate(row, col, id, r) && !(full && !(worst > r));
+        row += 64 / nc;
+        col += 64 % nc;
+        if (col >= nc) { col -= nc; row++; }
         const unsigned long long m = __ballot(in);
-        const long long at = cnt + __popcll(m & ((1ull << lane) - 1ull));
-        if (in && at < SEARCH_CAP) { lr[wave][at] = r; lid[wave][at] = id; }
-        cnt += __popcll(m);
+        const int at = have + __popcll(m & ((1ull << lane) - 1ull));
+        if (in) { lr[wave][at] = r; lid[wave][at] = id; }
+        have += __popcll(m);
+        if (have <= SEARCH_CAP - 64) continue;
+        if (a.maxn > SEARCH_CAP - 64) {
+            serial = true;
+            break;
+        }
+        in_step();
+        int to[SEARCH_CAP / 64], ids_[SEARCH_CAP / 64];
+        double rs_[SEARCH_CAP / 64];
+#pragma unroll
+        for (int j = 0; j < SEARCH_CAP / 64; j++) {
+            const int i = lane + 64 * j;
+            to[j] = a.maxn;
+            if (i < have) {
+                to[j] = rank_of(i);
+                rs_[j] = lr[wave][i];
+                ids_[j] = lid[wave][i];
+            }
+        }
+        in_step();
+#pragma unroll
+        for (int j = 0; j < SEARCH_CAP / 64; j++)
+            if (to[j] < a.maxn) { lr[wave][to[j]] = rs_[j]; lid[wave][to[j]] = ids_[j]; }
+        in_step();
+        have = a.maxn;
+        full = true;
+        worst = lr[wave][a.maxn - 1];
     }
-    const int kept = (int)min(cnt, (long long)a.maxn);
-    for (int k = kept + lane; k < a.maxn; k += 64) { ids[k] = -1; rs[k] = 1.0e15; }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (cnt <= SEARCH_CAP) {
-        for (int i = lane; i < (int)cnt; i += 64) {
-            const double r = lr[wave][i];
-            int rank = 0;
-            for (int j = 0; j < (int)cnt; j++) rank += j < i ? !(lr[wave][j] > r) : r > lr[wave][j];
-            if (rank < a.maxn) { ids[rank] = lid[wave][i]; rs[rank] = r; }
+    if (!serial) {
+        in_step();
+        for (int k = min(have, a.maxn) + lane; k < a.maxn; k += 64) { ids[k] = -1; rs[k] = 1.0e15; }
+        for (int i = lane; i < have; i += 64) {
+            const int rank = rank_of(i);
+            if (rank < a.maxn) { ids[rank] = lid[wave][i]; rs[rank] = lr[wave][i]; }
         }
     } else if (lane == 0) {
-        int have = 0;
-        for (long long n = 0; n < total; n++) {
-            int id;
-            double r;
-            if (!candidate(n, id, r)) continue;
-            int pos = have;
-            while (pos > 0 && rs[pos - 1] > r) pos--;
-            if (pos >= a.maxn) continue;
-            for (int k = have < a.maxn ? have : a.maxn - 1; k > pos; k--) { ids[k] = ids[k - 1]; rs[k] = rs[k - 1]; }
-            ids[pos] = id;
-            rs[pos] = r;
-            if (have < a.maxn) have++;
-        }
+        int cnt = 0;
+        for (row = 0; row < nrow; row++)
+            for (col = 0; col < ncol; col++) {
+                int id;
+                double r;
+                if (!candidate(row, col, id, r)) continue;
+                int pos = cnt;
+                while (pos > 0 && rs[pos - 1] > r) pos--;
+                if (pos >= a.maxn) continue;
+                for (int k = cnt < a.maxn ? cnt : a.maxn - 1; k > pos; k--) { ids[k] = ids[k - 1]; rs[k] = rs[k - 1]; }
+                ids[pos] = id;
+                rs[pos] = r;
+                if (cnt < a.maxn) cnt++;
+            }
+        for (int k = cnt; k < a.maxn; k++) { ids[k] = -1; rs[k] = 1.0e15; }
     }
 }
 

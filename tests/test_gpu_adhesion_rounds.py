@@ -38,3 +38,21 @@ def test_rounds_of_many_springs(k):
     assert near * MANY[k]["springs_per_knob"] > 2 * 1024
     assert (st["attach"] >= 0).sum() > 5
     g.close()
+
+
+# several hundred to ten thousand receptors in range: the list is cut over and
+# over, to one entry, to the longest that it can be cut to, and where it cannot
+DENSE = [(64.0, 1), (64.0, 16), (64.0, 100), (64.0, 192), (64.0, 193), (100.0, 64), (900.0, 16), (900.0, 300)]
+
+
+@pytest.mark.parametrize("density,maxn", DENSE)
+def test_lists_of_dense_receptors(density, maxn):
+    print(f"[dense] {density} {maxn}", flush=True)
+    extra = dict(receptor_density=density, max_neighwall=maxn, springs_per_knob=1)
+    o, g, st, nrec = _pair("f64", extra=extra, tau=0.9, p=5e-6, b=5e-3)
+    gs = g.adhesion_state(nrec)
+    g.close()
+    assert np.array_equal(gs["id_wall"], st["id_wall"])
+    assert np.allclose(gs["r_wall"], st["r_wall"], rtol=1e-14, atol=0)
+    assert np.array_equal(gs["attach"], st["attach"])
+    assert (st["id_wall"].reshape(-1, maxn)[:, -1] >= 0).any()  # full lists
