@@ -37,19 +37,19 @@ __device__ DevStep step_of(int it, const StepParams &p) {
 // The values of step `iter`, or of the step after the current one (iter < 0).
 __global__ void k_set_step(DevStep *s, int iter, StepParams p) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    s[0] = step_of(iter >= 0 ? iter : s[0].iter + 1, p);
+    *s = step_of(iter >= 0 ? iter : s->iter + 1, p);
 }
 
-// The values of the next n steps into s[1..n], the last of them also into
-// s[0]: one launch per replayed block.  One launch per step, each a node of the
+// The values of the next n steps into block[0..n-1], the last of them also
+// into *now: one launch per replayed block.  One launch per step, each a node of the
 // graph that the next kernel waits for, took 2 us and its gap out of 11 us
 // for a step on 64x32x32 FP64 nodes.
-__global__ __launch_bounds__(64) void k_set_steps(DevStep *s, int n, StepParams p) {
-    const int it = s[0].iter;
+__global__ __launch_bounds__(64) void k_set_steps(DevStep *now, DevStep *block, int n, StepParams p) {
+    const int it = now->iter;
     __syncthreads();
     for (int k = threadIdx.x; k < n; k += 64) {
-        s[1 + k] = step_of(it + 1 + k, p);
-        if (k == n - 1) s[0] = s[1 + k];
+        block[k] = step_of(it + 1 + k, p);
+        if (k == n - 1) *now = block[k];
     }
 }
 
@@ -232,7 +232,7 @@ lbmibm_status join_volume(lbmibm_ctx *ctx) {
 // bending reads cel->x, so with BR != 0 the correction is joined first.
 lbmibm_status enqueue_step(lbmibm_ctx *ctx, int iter, bool device_advance, bool overlap_volume) {
     // within a replayed block the values are there already (k_set_steps)
-    lbmibm_status s = ctx->step == ctx->steps ? set_step(ctx, device_advance ? -1 : iter, false) : LBMIBM_OK;
+    lbmibm_status s = ctx->step == ctx->step_now ? set_step(ctx, device_advance ? -1 : iter, false) : LBMIBM_OK;
     const int M = ctx->p.m;
     if (s == LBMIBM_OK && (iter - 1) % M == 0 && ctx->nc > 0) {
         if (ctx->p.br != 0.0) s = join_volume(ctx);
@@ -276,7 +276,7 @@ void free_all(lbmibm_ctx *ctx) {
                     ctx->xd, ctx->uvw, ctx->cf, ctx->c0, ctx->s0, ctx->nref, ctx->tt, ctx->rg, ctx->tp, ctx->qv, ctx->qp,
                     ctx->qi, ctx->coef, ctx->bv, ctx->rv, ctx->rh, ctx->pv, ctx->vv, ctx->tv, ctx->gscale,
                     ctx->normal, ctx->vol0, ctx->vol, ctx->area, ctx->gx, ctx->bicg_iters, ctx->vol_passes,
-                    ctx->steps, ctx->status, ctx->node0, ctx->home, ctx->home_list, ctx->tile_count,
+                    ctx->step_now, ctx->step_block, ctx->status, ctx->node0, ctx->home, ctx->home_list, ctx->tile_count,
                     ctx->tile_off, ctx->tile_cur, ctx->order_calls, ctx->blk_fmax, ctx->absmax, ctx->nbr, ctx->bicg_cells[0],
                     ctx->bicg_cells[1], ctx->bicg_cells[2], ctx->vol_cells[0], ctx->vol_cells[1], ctx->dsv,
                     ctx->vol_echunks, ctx->vol_vchunks, ctx->vol_crange, ctx->vol_epart, ctx->vol_vpart,
@@ -317,14 +317,15 @@ static StepParams step_params(const lbmibm_ctx *ctx) {
 // Lattice steps of a replayed block: whole M-cycles and an even number of
 // lattice steps, so that the population buffers are back in place, repeated to at
 // least 8 steps: a step's volume correction overlaps the next step's
-// membrane force, except across block ends.
-static int block_steps(int M) {
-    const int L0 = (M % 2 == 0) ? M : 2 * M;
+// membrane force, except across block ends.  (More than an int holds, for the
+// largest M: no run is that long.)
+static long long block_steps(long long M) {
+    const long long L0 = (M % 2 == 0) ? M : 2 * M;
     return L0 * ((8 + L0 - 1) / L0);
 }
 
 lbmibm_status set_step(lbmibm_ctx *ctx, int iter, bool) {
-    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, ctx->stream, ctx->steps, iter, step_params(ctx));
+    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, ctx->stream, ctx->step_now, iter, step_params(ctx));
     LBMIBM_LAUNCHED(ctx, "k_set_step");
     return LBMIBM_OK;
 }
@@ -447,8 +448,8 @@ lbmibm_status lbmibm_create(const lbmibm_params *p, const lbmibm_cells *cells, l
         CK(dev_alloc(ctx, &ctx->mw, 2 * (size_t)p->lx * p->lz * szT));
         CK(lattice_fill(ctx, ctx->mw, 2 * (size_t)p->lx * p->lz, 0.0, false));
     }
-    CK(dev_alloc(ctx, (void **)&ctx->steps, (1 + (size_t)block_steps(p->m)) * sizeof(DevStep)));
-    ctx->step = ctx->steps;
+    CK(dev_alloc(ctx, (void **)&ctx->step_now, sizeof(DevStep)));
+    ctx->step = ctx->step_now;
     CK(dev_alloc(ctx, (void **)&ctx->status, sizeof(DevStatus)));
 
     if (cells && cells->nc > 0) {
@@ -832,7 +833,9 @@ lbmibm_status lbmibm_run(lbmibm_ctx *ctx, int iter0, int nsteps, int use_graph) 
     if (s != LBMIBM_OK) return s;
     const int M = ctx->p.m;
     if (ctx->p.vof_period > 0) use_graph = 0;  // front tracking synchronises with the host
-    const int L = block_steps(M);
+    const long long block = block_steps(M);
+    const bool replay = use_graph && block <= nsteps;
+    const int L = replay ? (int)block : 0;
     // LBMIBM_OVERLAP_VOLUME=0 keeps the volume correction on the stream
     const char *ov = getenv("LBMIBM_OVERLAP_VOLUME");
     const bool overlap = !(ov && ov[0] == '0');
@@ -845,7 +848,7 @@ lbmibm_status lbmibm_run(lbmibm_ctx *ctx, int iter0, int nsteps, int use_graph) 
         it++;
     }
     if (s == LBMIBM_OK) s = join_volume(ctx);  // nothing pending across a capture boundary
-    if (s == LBMIBM_OK && use_graph && end - it >= L) {
+    if (s == LBMIBM_OK && replay && end - it >= L) {
         if (ctx->graph_ready && (ctx->graph_cur != ctx->cur || ctx->graph_force_zero != ctx->force_zero))
             ctx->graph_ready = false;
         if (!ctx->graph_ready && ctx->graph) {  // recorded before a state change: released once it has run
@@ -859,15 +862,20 @@ lbmibm_status lbmibm_run(lbmibm_ctx *ctx, int iter0, int nsteps, int use_graph) 
             // the block's first spreading must bin: on replay the positions
             // are the previous block's, whatever the host flag says now
             invalidate_bins(ctx);
+            if (!ctx->step_block) {  // a context's blocks are all of one length
+                s = dev_alloc(ctx, (void **)&ctx->step_block, (size_t)L * sizeof(DevStep));
+                if (s != LBMIBM_OK) return s;
+            }
             hipGraph_t g = nullptr;
             LBMIBM_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-            hipLaunchKernelGGL(k_set_steps, dim3(1), dim3(64), 0, ctx->stream, ctx->steps, L, step_params(ctx));
+            hipLaunchKernelGGL(k_set_steps, dim3(1), dim3(64), 0, ctx->stream, ctx->step_now,
+                               ctx->step_block, L, step_params(ctx));
             lbmibm_status cs = hipGetLastError() == hipSuccess ? LBMIBM_OK : LBMIBM_ERR_HIP;
             for (int k = 0; k < L && cs == LBMIBM_OK; k++) {
-                ctx->step = ctx->steps + 1 + k;
+                ctx->step = ctx->step_block + k;
                 cs = enqueue_step(ctx, it + k + 1, true, overlap);
             }
-            ctx->step = ctx->steps;
+            ctx->step = ctx->step_now;
             if (cs == LBMIBM_OK) cs = join_volume(ctx);
             hipError_t e = hipStreamEndCapture(ctx->stream, &g);
             if (cs != LBMIBM_OK) return cs;

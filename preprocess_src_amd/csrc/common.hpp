@@ -321,7 +321,8 @@ struct lbmibm_ctx {
     bool kt_on = false;
     std::vector<KtRec> kt_recs;
     void *adh_fsum = nullptr;
-    lbmibm::DevStep *steps = nullptr;  // [0] the current step's values; [1..] those of a replayed block's steps
+    lbmibm::DevStep *step_now = nullptr;    // [1] the current step's values
+    lbmibm::DevStep *step_block = nullptr;  // those of the steps of a replayed block, allocated with the first one
     lbmibm::DevStep *step = nullptr;   // the entry that kernels are launched with
     lbmibm::DevStatus *status = nullptr;
 
