@@ -75,10 +75,23 @@ void staging_reserve(lbmibm_ctx *ctx) {
     }
 }
 
+// Whether two of the host arrays, of n values each, share memory.
+static bool overlap(const std::vector<FieldOut> &out, size_t n) {
+    for (size_t i = 0; i < out.size(); i++)
+        for (size_t j = 0; j < i; j++) {
+            const uintptr_t a = (uintptr_t)out[i].dst, b = (uintptr_t)out[j].dst;
+            if ((a < b ? b - a : a - b) < n * sizeof(double)) return true;
+        }
+    return false;
+}
+
 // Copies pieces 0..n-1 (source(i, &bytes) names piece i) and hands each to
-// take(i, data), in any order, on several threads.  take writes disjoint memory.
+// take(i, data), in any order, on several threads; take writes disjoint memory.
+// Or in their order, on the caller's alone: where arrays share memory (a caller may
+// give one place for all that it does not want), what comes last remains.
 template <typename Source, typename Take>
-static lbmibm_status staged(lbmibm_ctx *ctx, size_t n, size_t piece, size_t total, Source source, Take take) {
+static lbmibm_status staged(lbmibm_ctx *ctx, size_t n, size_t piece, size_t total, bool in_order, Source source,
+                            Take take) {
     if (n == 0) return LBMIBM_OK;
     const std::lock_guard<std::mutex> lock(ctx->staging_mutex);  // callers may share a context's ring
     lbmibm_status s = staging_room(ctx, piece);
@@ -107,7 +120,7 @@ static lbmibm_status staged(lbmibm_ctx *ctx, size_t n, size_t piece, size_t tota
         return true;
     };
     std::vector<std::thread> pool;
-    const size_t want = std::min({(size_t)MAX_THREADS, total / PER_THREAD, n - 1});
+    const size_t want = in_order ? 0 : std::min({(size_t)MAX_THREADS, total / PER_THREAD, n - 1});
     try {
         pool.reserve(want);
         for (size_t t = 0; t < want; t++) pool.emplace_back([&] { while (work(true)) {} });
@@ -225,7 +238,7 @@ lbmibm_status download_fields(lbmibm_ctx *ctx, const FieldOut *all, int nall, si
     const size_t row = (size_t)f.nx * elem, rows = (size_t)f.ny * f.nz;
     const size_t per = std::min(std::max<size_t>(PIECE / row, 1), rows), pieces = (rows + per - 1) / per;
     return staged(
-        ctx, out.size() * pieces, per * row, out.size() * rows * row,
+        ctx, out.size() * pieces, per * row, out.size() * rows * row, overlap(out, (size_t)ctx->np),
         [&](size_t i, size_t *bytes) {
             const size_t r0 = i % pieces * per;
             *bytes = (std::min(r0 + per, rows) - r0) * row;
@@ -248,7 +261,7 @@ lbmibm_status download_arrays(lbmibm_ctx *ctx, const FieldOut *all, int nall, si
         if (all[i].dst) out.push_back(all[i]);
     const size_t per = std::min(PIECE / elem, n), pieces = n ? (n + per - 1) / per : 0;
     return staged(
-        ctx, out.size() * pieces, per * elem, out.size() * n * elem,
+        ctx, out.size() * pieces, per * elem, out.size() * n * elem, overlap(out, n),
         [&](size_t i, size_t *bytes) {
             const size_t a = i % pieces * per;
             *bytes = (std::min(a + per, n) - a) * elem;
