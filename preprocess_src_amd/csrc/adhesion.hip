@@ -219,6 +219,7 @@ __global__ __launch_bounds__(AWG) void k_adh_search(AdhDev a, const double *__re
         double zj = (jz - a.nzw / 2) * a.dzw;
         if (jz < 0) { jz += a.nzw; zj += a.lz; }
         else if (jz >= a.nzw) { jz -= a.nzw; zj -= a.lz; }
+        if (jz < 0 || jz >= a.nzw) return false;  // more than a period away: LIMIT dx beyond the box
         const int k = ra0 + col, jx = k <= ra1 ? k : rb0 + (k - ra1 - 1);
         id = jz * a.nxw + jx;
         double xj, yj, zr;
