@@ -729,7 +729,7 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
     } else {
         tile = order[blockIdx.x - maxextra];
     }
-    const int cnt = tile_count[tile], off = tile_off[tile];
+    const int cnt = tile_count[tile], off = tile_off[tile], ex0 = tile_ex[tile];
     if (cnt == 0) return;  // whole work group leaves together; the gather skips empty tiles
     const int nch = spread_chunks(cnt);
     const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
@@ -1009,7 +1009,7 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
     }
     const double inv_scale = 1.0 / scale;
     T *St = S + (size_t)tile * 3 * SB_N;
-    ChunkBox *box = chunks + (nch == 1 ? 0 : chunk > 0 ? (int)blockIdx.x : maxextra + tile_ex[tile]);
+    ChunkBox *box = chunks + (nch == 1 ? 0 : chunk > 0 ? (int)blockIdx.x : maxextra + ex0);
     for (int k0 = tid; k0 < 3 * SB_N; k0 += 4 * WG_) {  // four reads, then four stores
         unsigned long long a[4];
 #pragma unroll
@@ -1031,8 +1031,8 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
 // scales, which is the one that all of the tile's vertices in one work group would
 // have had, and rounded to T at the end; boxes rounded to FP32 and added in FP32
 // lost up to 2.8 times as much where the chunks' sums cancel.  That costs twice
-// the bytes: 64 cells 5.8 -> 7.9 us here and 33.5 -> 34.2 in k_spread_box, the
-// 1024-cell suspension 13.4 -> 20.5 and 198 -> 205.  The boxes are read once: past
+// the bytes: 64 cells 5.8 -> 7.1 us here and 33.4 -> 34.1 in k_spread_box, the
+// 1024-cell suspension 13.3 -> 18.6 and 198 -> 205.  The boxes are read once: past
 // the caches, or they would drive out those that the gather reads next (62 instead
 // of 55 us).  The gather adding the chunks itself took 64 instead of 44 us: the
 // loop over them keeps its loads from being issued together.
@@ -1044,28 +1044,24 @@ __global__ __launch_bounds__(COMBINE_WG) void k_spread_combine(T *__restrict__ S
                                                          const int *__restrict__ tile_count, int maxextra) {
     const int2 ex = extra[blockIdx.x];
     if (ex.x < 0 || ex.y != 1) return;
-    const int nx = spread_chunks(tile_count[ex.x]) - 1;
     const ChunkBox *first = chunks + maxextra + blockIdx.x, *more = chunks + blockIdx.x;
-    // the coarsest scale (positive doubles order as their bits)
-    __shared__ unsigned long long coarsest;
-    if (threadIdx.x == 0) coarsest = (unsigned long long)__double_as_longlong(first->scale);
-    __syncthreads();
-    for (int c = threadIdx.x; c < nx; c += COMBINE_WG)
-        atomicMin(&coarsest, (unsigned long long)__double_as_longlong(more[c].scale));
+    // every load that does not need the number of chunks, beside that of the number
     constexpr int PER = COMBINE_PER;
     const int k0 = (int)blockIdx.y * COMBINE_WG * PER + (int)threadIdx.x;
     int k[PER];
-    long long v[PER], sum[PER];
+    long long v[PER], next[PER], sum[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         k[j] = min(k0 + COMBINE_WG * j, 3 * SB_N - 1);
         v[j] = __builtin_nontemporal_load(&first->v[k[j]]);
+        next[j] = __builtin_nontemporal_load(&more[0].v[k[j]]);
         sum[j] = 0;
     }
-    __syncthreads();
-    const double scale = __longlong_as_double((long long)coarsest);
+    const int nx = spread_chunks(tile_count[ex.x]) - 1;
+    double scale = fmin(first->scale, more[0].scale);  // the coarsest
+    for (int c = 1; c < nx; c++) scale = fmin(scale, more[c].scale);
     const int e = ilogb(scale);
-    for (int c = 0; c <= nx; c++) {  // the next box's values while these are added
+    for (int c = 0; c <= nx; c++) {  // the next but one box's values while these are added
         const double t = c == 0 ? first->scale : more[c - 1].scale;
         // at most 62: a chunk without forces, at infinity, holds zeros
         const int sh = scale > 0.0 ? (int)min((long long)ilogb(t) - e, 62ll) : 0;
@@ -1073,7 +1069,8 @@ __global__ __launch_bounds__(COMBINE_WG) void k_spread_combine(T *__restrict__ S
 #pragma unroll
         for (int j = 0; j < PER; j++) {
             sum[j] += (v[j] + half) >> sh;
-            if (c < nx) v[j] = __builtin_nontemporal_load(&more[c].v[k[j]]);
+            v[j] = next[j];
+            if (c + 1 < nx) next[j] = __builtin_nontemporal_load(&more[c + 1].v[k[j]]);
         }
     }
     const double inv = 1.0 / scale;
