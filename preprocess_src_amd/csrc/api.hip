@@ -171,23 +171,6 @@ long long push_target(const lbmibm_ctx *ctx, int ix, int iy, int iz, int q) {
     return (long long)tx + (long long)ctx->nx * (ty + (long long)ctx->ny * tz);
 }
 
-// Periodic image in the padded frame (lbm.cu:1350-1353, 1410-1411), or -1
-// for a wall node.
-inline long long padded_image(const lbmibm_ctx *ctx, int px, int py, int pz, bool &is_comp) {
-    auto w = [](int a, int n) { return a < 2 ? a + (n - 4) : (a > n - 3 ? a - (n - 4) : a); };
-    if (ctx->p.tube_radius > 0.0) {  // only z is periodic; outside the disc is wall
-        is_comp = false;
-        if (!tube_inside(ctx, px - 2, py - 2)) return -1;
-        is_comp = pz >= 2 && pz <= ctx->nzp - 3;
-        return (long long)(px - 2) + (long long)ctx->nx * ((py - 2) + (long long)ctx->ny * (w(pz, ctx->nzp) - 2));
-    }
-    const bool iny = py >= 2 && py <= ctx->nyp - 3;
-    is_comp = px >= 2 && px <= ctx->nxp - 3 && iny && pz >= 2 && pz <= ctx->nzp - 3;
-    if (!iny && !ctx->p.periodic_y) return -1;
-    const int ix = w(px, ctx->nxp) - 2, iy = w(py, ctx->nyp) - 2, iz = w(pz, ctx->nzp) - 2;
-    return (long long)ix + (long long)ctx->nx * (iy + (long long)ctx->ny * iz);
-}
-
 lbmibm_status sync_check(lbmibm_ctx *ctx) {
     LBMIBM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return LBMIBM_OK;

@@ -82,7 +82,7 @@ __device__ __forceinline__ int home_tile(const BinGeom &g, double x, double y, d
 // line's atomics one after another, which one atomic per wave and tile made
 // about 10 times as many.  Any order and any number of tiles is accepted (the
 // table has twice as many entries as a group has vertices).  On 64 cells of
-// 2562 vertices, per launch before and after: k_vol_center 22.0 -> 9.4 us,
+// 2562 vertices, per launch before and after: k_vol_center 22.0 -> 10.0 us,
 // k_bin_scatter 22.2 -> 6.4 us, k_bin_count 23.0 -> 5.4 us.
 constexpr int BIN_WG = 1024;  // vertices per work group of the binning kernels
 struct TileTable {
@@ -258,8 +258,10 @@ struct lbmibm_ctx {
     // FP32 values under a volume-of-fluid indicator, which is FP64: the
     // indicator's sweeps switch on the last bits of the velocity (a different
     // rounding of the spread force alone moves vf by 2e-6), so these runs
-    // keep FP32 products summed point by point, over tiles of TILE_XW nodes,
-    // and with them the results they always had.
+    // keep FP32 products summed point by point, over tiles of TILE_XW nodes: the
+    // two forms of the spreading as they always were, of which the timing at
+    // creation chooses one (their bits differ from each other's; those of the two
+    // interpolation forms do not).
     bool pointwise = false;
     int tile_x = lbmibm::TILE_X;  // nodes of a tile in x
     short4 *node0 = nullptr;                 // [Nv] first stencil node (x,z wrapped, y+3), bin order

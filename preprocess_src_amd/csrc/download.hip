@@ -169,7 +169,8 @@ static lbmibm_status staged(lbmibm_ctx *ctx, size_t n, size_t piece, size_t tota
     return LBMIBM_OK;
 }
 
-// Geometry of the padded rows.
+// Geometry of the padded rows; the periodic images in the halo as in lbm.cu:1350-1353,
+// 1410-1411.
 struct Frame {
     int nx, ny, nz, nxp, nyp, nzp;
     bool images, zero, py;         // periodic images / zeros in place of wall nodes / y periodic

@@ -662,8 +662,8 @@ __global__ __launch_bounds__(256) void k_spread_tiles(const SpreadRec<T> *__rest
 // issued them per vertex (about 12 cycles per wave and CU): a mesh of 2562
 // vertices on a radius of 4 has 13 vertices per cell, the uneven suspension of
 // 1024 cells 4.8.  Per launch, before and after: 64 cells of 2562 vertices
-// (FP32) 90 -> 31 us, that suspension 250 -> 194 us, 384 such cells in FP64
-// 144 -> 120 us; with 8x8x8 tiles, 16x8x8 before.  What bounds it now is the
+// (FP32) 90 -> 34 us, that suspension 250 -> 205 us, 384 such cells in FP64
+// 144 -> 122 us; with 8x8x8 tiles, 16x8x8 before.  What bounds it now is the
 // latency of its phases (loads, scan, sort, products) at the three work groups
 // that the box's LDS admits per CU.
 // The weights are formed in T, their products and sums in FP64.
@@ -984,8 +984,9 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
             __syncthreads();
         }
     } else {
-        // more vertices than the sort holds (thousands in a single lattice
-        // cell): their terms one by one
+        // more vertices than the sort holds: a stretch ends with a whole cell, so
+        // one of SB_CAP - SB_CHUNK vertices or more at its end may be too many.
+        // Their terms one by one
         const T w1 = (T)(1.0 / (64.0 * g.dx * g.dx * g.dx));
         for (int i = tid; i < cnt; i += WG_) {
             const int kc = key_of(node0[off + i]);
@@ -2374,7 +2375,9 @@ static bool spread_box_tables(const lbmibm_ctx *ctx, std::vector<int> &out) {
     const int n[3] = {ctx->nx, ctx->ny, ctx->nz}, nt[3] = {ctx->ntx, ctx->nty, ctx->ntz};
     const int tile[3] = {ctx->tile_x, TILE_Y, TILE_Z}, R[3] = {ctx->tile_x + 3, SB_Y, SB_Z};
     const bool wrap[3] = {true, ctx->p.periodic_y != 0, true};
-    if (n[0] < 5) return false;  // rows that a box of TILE_XW + 3 nodes meets more than SB_MAXC times
+    // boxes of TILE_XW + 3 nodes meet rows of four more than SB_MAXC times; with
+    // those of TILE_X + 3 such lattices stay without the form, which they never had
+    if (n[0] < 5) return false;
     out.assign((size_t)SB_MAXC * (n[0] + n[1] + n[2]), -1);
     size_t base = 0;
     for (int a = 0; a < 3; a++) {

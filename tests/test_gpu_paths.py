@@ -73,9 +73,9 @@ def _crowded(lx, ly, lz, levels, seed, lo, hi):
 
 
 # corners of the first stencil nodes (a vertex between nodes i and i + 1 starts
-# its stencil at i - 1): within two tiles (16 x 8 x 8 nodes) below the sort's capacity,
-# above it (several passes), in one lattice cell below and above it, and more
-# vertices than 16-bit indices hold; across the lower wall
+# its stencil at i - 1): within two tiles (8 x 8 x 8 nodes) below and above the share
+# of 800 vertices that a work group takes, in one lattice cell below and above the
+# sort's capacity, and more vertices than 16-bit indices hold; across the lower wall
 CROWDS = [([3, 3], (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)), ([4, 4], (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)),
           ([3], (5.1, 12.1, 12.1), (5.9, 12.9, 12.9)), ([4], (5.1, 12.1, 12.1), (5.9, 12.9, 12.9)),
           ([5, 3], (5.1, 12.1, 12.1), (6.9, 12.9, 12.9)), ([5] * 7, (2.0, 9.0, 9.0), (16.9, 16.9, 16.9)),
