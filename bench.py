@@ -243,7 +243,8 @@ def traffic_from_profile(precision):
 
 # kernel-table names -> kernel names in the rocprof summaries (FP32 workload)
 PROF_NAMES = {"k_lbm": "k_lbm<float, float, double, true, false, 1>", "k_spread_box": "k_spread_box<float>",
-              "k_spread_gather": "k_spread_gather<float>", "k_interp_tiles": "k_interp_tiles<float>",
+              "k_spread_gather": "k_spread_gather<float, 8>", "k_spread_combine": "k_spread_combine<float>",
+              "k_interp_tiles": "k_interp_tiles<float>",
               "k_bicg_res": "k_bicg_res<11>", "k_assemble": "k_assemble<float>",
               "k_bicg_onchip class 0": "k_bicg_onchip<float, 2, 512>",
               "k_bicg_onchip class 1": "k_bicg_onchip<float, 6, 512>", "k_vol_sums": "k_vol_sums",

@@ -2144,9 +2144,11 @@ template <typename T> lbmibm_status spread_launch(lbmibm_ctx *ctx, int form) {
                                          ctx->sb_maxextra, ctx->tile_ex, (ChunkBox *)ctx->sb_chunks));
             LBMIBM_LAUNCHED(ctx, "k_spread_box");
             if (ctx->sb_maxextra > 0) {
-                hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra, COMBINE_PARTS), dim3(COMBINE_WG), 0,
-                                   ctx->stream, (T *)ctx->sbox, (const ChunkBox *)ctx->sb_chunks, ctx->sb_extra,
-                                   ctx->tile_count, ctx->sb_maxextra);
+                LBMIBM_KT(ctx, ctx->stream, "k_spread_combine",
+                          hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra, COMBINE_PARTS),
+                                             dim3(COMBINE_WG), 0, ctx->stream, (T *)ctx->sbox,
+                                             (const ChunkBox *)ctx->sb_chunks, ctx->sb_extra, ctx->tile_count,
+                                             ctx->sb_maxextra));
                 LBMIBM_LAUNCHED(ctx, "k_spread_combine");
             }
         }
