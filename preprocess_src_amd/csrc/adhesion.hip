@@ -460,12 +460,14 @@ __global__ __launch_bounds__(AWG) void k_adh_resolve(AdhDev a, AdhRound q) {
 // MAXN = 16 (27 now, 12 of them here).  But a thousand losers are what one CU
 // takes in the time of a launch: all rounds in one group took 2.45 ms of a step
 // with 363 000 springs and 34.7 ms with 1.8 million (MAXN = 100), 0.50 and 2.2
-// in pairs of launches, 0.22 and 0.95 now.  ROUNDS_SPRINGS: with 8100 springs, of
-// which a third is near the wall, the group alone takes 0.09 ms, the pairs took
-// 0.25; below, the nine or ten launches that find nothing to do would cost 20 us of
-// every step.
+// in pairs of launches, 0.24 and 1.2 now.  ROUNDS_SPRINGS: with 8100 springs of 16
+// per knob, half of them near the wall, and MAXN = 100 the group alone takes 0.17 ms,
+// the pairs took 1.5; below, the launches that find nothing to do would cost 20 us
+// and more of every step.  Springs of one knob contend for the same receptors round
+// after round, so with more of them per knob (ROUNDS_PER_KNOB) the launches are made.
 constexpr int ROUNDS_GROUP = 1024;
-constexpr int ROUNDS_SPRINGS = 8192;  // springs up to which no other launches are made
+constexpr int ROUNDS_SPRINGS = 8192, ROUNDS_PER_KNOB = 16;  // springs up to which no other launches are made
+constexpr int ROUNDS_MANY = 65536;                          // and above which every round has one
 __global__ __launch_bounds__(1024) void k_adh_rounds(AdhDev a, AdhRound q, int which, int first, int most) {
     __shared__ int made;
     const int m = q.more[which];
@@ -495,10 +497,13 @@ __global__ __launch_bounds__(1024) void k_adh_rounds(AdhDev a, AdhRound q, int w
 // them.  A spring first learns how its bid of the round before ended, then makes
 // the next; receptors that somebody won in that round are told by the bids on them,
 // whether the winner has entered itself yet or not.  The `last` launch only
-// enters the winners, and lists the losers.  Eight launches: with four the
-// 1.8 million springs leave so many losers that a step takes 1 ms more, with six
-// 0.03; a launch for every round up to MAXN takes 0.25 ms more where MAXN is 100.
-constexpr int ROUND_GROUPS = 512, ROUND_LAUNCHES = 8;
+// enters the winners, and lists the losers.  Every round up to MAXN has its launch at
+// the set-up, where all springs lose at once, and for more than ROUNDS_MANY
+// springs (a launch that finds nothing to do costs 2.3 us); otherwise 4 rounds per
+// spring of a knob have one, at least 8, and k_adh_rounds takes what is left.  With 8
+// rounds always, 1.8 million springs at 400 per knob took 69 ms (10 in pairs of
+// launches, 3.0 now), and the set-up of those at 40 per knob 57 ms (9 and 7).
+constexpr int ROUND_GROUPS = 512;
 __global__ __launch_bounds__(AWG) void k_adh_round(AdhDev a, AdhRound q, int round, bool last, int most) {
     const int m = q.more[0];
     if (m <= most || (round > 1 && q.made[round - 1] == 0)) return;
@@ -573,14 +578,14 @@ lbmibm_status adh_bell(lbmibm_ctx *ctx, int init) {
                        ctx->adh_claim, (long long)a.nxw * a.nzw, q.more, q.made);
     hipLaunchKernelGGL(k_adh_propose, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, q);
     hipLaunchKernelGGL(k_adh_resolve, dim3(ablocks(nsp)), dim3(AWG), 0, st, a, q);
-    const bool few = nsp <= ROUNDS_SPRINGS;
+    const bool few = nsp <= ROUNDS_GROUP || (nsp <= ROUNDS_SPRINGS && a.ns <= ROUNDS_PER_KNOB);
     const int most = few ? INT_MAX : ROUNDS_GROUP;
     hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, 0, 1, most);
     if (!few) {
-        const int n = std::min(ROUND_LAUNCHES, a.maxn);
+        const int n = init || nsp > ROUNDS_MANY ? a.maxn : std::min(std::max(8LL, 4LL * a.ns), (long long)a.maxn);
         for (int r = 1; r <= n + 1; r++)
             hipLaunchKernelGGL(k_adh_round, dim3(ROUND_GROUPS), dim3(AWG), 0, st, a, q, r, r > n, most);
-        hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, 1, n + 1, INT_MAX);
+        if (n < a.maxn) hipLaunchKernelGGL(k_adh_rounds, dim3(1), dim3(1024), 0, st, a, q, 1, n + 1, INT_MAX);
     }
     LBMIBM_LAUNCHED(ctx, "k_adh_*");
     return LBMIBM_OK;

@@ -56,3 +56,39 @@ def test_lists_of_dense_receptors(density, maxn):
     assert np.allclose(gs["r_wall"], st["r_wall"], rtol=1e-14, atol=0)
     assert np.array_equal(gs["attach"], st["attach"])
     assert (st["id_wall"].reshape(-1, maxn)[:, -1] >= 0).any()  # full lists
+
+
+# two springs on each of 5124 knobs: eight launches, and what is left in one group
+CROWDED = [dict(receptor_density=4.0, max_neighwall=40), dict(receptor_density=1.0, max_neighwall=12, k_on0=3.0),
+           dict(receptor_density=16.0, max_neighwall=100, k_on0=3.0, k_off0=2.0)]
+
+
+@pytest.mark.parametrize("k", range(len(CROWDED)))
+def test_rounds_of_crowded_knobs(k):
+    from preprocess_src_amd import mesh
+    from tests.pairs import gpu_of, oracle_of
+    from tests.test_adhesion import ADH, LX, LZ
+    print(f"[crowded knobs] {CROWDED[k]}", flush=True)
+    y = -LY / 2 + 3.5
+    cells = mesh.assemble([4, 4], np.array([[-6.0, y, -0.4], [6.2, y, 0.3]]), np.repeat(np.eye(3)[None], 2, 0), 3.0,
+                          shape="sphere")
+    kw = dict(tau=0.9, p=5e-6, b=5e-3)
+    o = oracle_of(LX, LY, LZ, cells=cells, **kw)
+    g = gpu_of(LX, LY, LZ, "f64", cells=cells, **kw)
+    kn = np.ones(len(cells["x"]), np.uint8)
+    adh = dict(ADH, springs_per_knob=2, **CROWDED[k])
+    assert 8192 < 2 * kn.size <= 65536
+    g.adhesion_setup(adh, kn)
+    st = o.adhesion_setup(adh, kn)
+    nrec = o._adhs.nxw * o._adhs.nzw
+    o.volume_init()
+    g.volume_init()
+    assert (st["id_wall"].reshape(-1, adh["max_neighwall"])[:, 0] >= 0).sum() * 2 > 2048
+    for it in range(7):
+        gs = g.adhesion_state(nrec)
+        for name in ("id_wall", "attach", "is_attached"):
+            assert np.array_equal(gs[name], st[name]), (it, name)
+        if it < 6:
+            assert o.step(it + 1)[0] == 0
+            g.step(it + 1)
+    g.close()
