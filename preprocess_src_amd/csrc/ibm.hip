@@ -244,7 +244,8 @@ __global__ __launch_bounds__(BIN_WG) void k_bin_count(const double *__restrict__
 // per-tile load, largest first.  The tile kernels take their tiles in this
 // order, so the dispatcher starts the longest work groups first and fills the
 // tail with light ones (longest-processing-time-first scheduling); the order
-// within a key level is arbitrary and does not affect any result.
+// within a key level is arbitrary and does not affect any result.  The last level
+// holds nearly all tiles of a sparse lattice: a wave counts it with one atomic.
 __device__ void heavy_first_order(const int *load, int n, int *hist, int *order) {
     __shared__ int maxload;
     if (threadIdx.x == 0) maxload = 0;
@@ -256,7 +257,13 @@ __device__ void heavy_first_order(const int *load, int n, int *hist, int *order)
     __syncthreads();
     int shift = 0;
     while ((maxload >> shift) > 255) shift++;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) atomicAdd(&hist[255 - (load[i] >> shift)], 1);
+    const int lane = threadIdx.x & 63;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const int key = 255 - (load[i] >> shift);
+        const unsigned long long last = __ballot(key == 255);
+        if (key < 255) atomicAdd(&hist[key], 1);
+        else if (lane == __ffsll((long long)last) - 1) atomicAdd(&hist[255], __popcll(last));
+    }
     __syncthreads();
     if (threadIdx.x == 0) {  // exclusive scan of 256 bins
         int acc = 0;
@@ -267,18 +274,31 @@ __device__ void heavy_first_order(const int *load, int n, int *hist, int *order)
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) order[atomicAdd(&hist[255 - (load[i] >> shift)], 1)] = i;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const int key = 255 - (load[i] >> shift);
+        const unsigned long long last = __ballot(key == 255);
+        if (key < 255) {
+            order[atomicAdd(&hist[key], 1)] = i;
+        } else {
+            const int first = __ffsll((long long)last) - 1;
+            int at = 0;
+            if (lane == first) at = atomicAdd(&hist[255], __popcll(last));
+            order[__shfl(at, first) + __popcll(last & ((1ull << lane) - 1ull))] = i;
+        }
+    }
     __syncthreads();
 }
 
-// The heavy-first tile orders of the spreading (by candidate count: own bin
-// and the bins below on each axis) and of the interpolation (by own count).
+// The heavy-first tile orders of the spreading from source bins, if that form is
+// taken (by candidate count: own bin and the bins below on each axis), and of the
+// interpolation and the home boxes (by own count).
 // They only steer the dispatch order, and tile loads change slowly with the
 // cells, so they are refreshed on every TILE_ORDER_PERIOD-th binning (a call
 // counter on the device, so captured graphs refresh them too); any
 // permutation is a valid order, the initial one is the identity.
 constexpr int TILE_ORDER_PERIOD = 16;
 
+template <bool BINS>
 __device__ void tile_orders(const int *__restrict__ tile_count, int ntiles, const IbmGeom &g, const TileGeom &tg,
                             int *__restrict__ tile_cand, int *__restrict__ order_spread,
                             int *__restrict__ order_interp, int *__restrict__ calls) {
@@ -287,7 +307,7 @@ __device__ void tile_orders(const int *__restrict__ tile_count, int ntiles, cons
     if (threadIdx.x == 0) call = (*calls)++;
     __syncthreads();
     if (call % TILE_ORDER_PERIOD != 0) return;
-    for (int t = threadIdx.x; t < ntiles; t += 1024) {
+    for (int t = threadIdx.x; BINS && t < ntiles; t += 1024) {
         const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
         int sxs[4], sys[4], szs[4];
         const int nsx = source_tiles(tx, tx * tg.tx, g.nx, tg.tx, true, sxs);
@@ -300,7 +320,7 @@ __device__ void tile_orders(const int *__restrict__ tile_count, int ntiles, cons
         tile_cand[t] = c;
     }
     __syncthreads();
-    heavy_first_order(tile_cand, ntiles, sh, order_spread);
+    if (BINS) heavy_first_order(tile_cand, ntiles, sh, order_spread);
     heavy_first_order(tile_count, ntiles, sh, order_interp);
 }
 
@@ -308,12 +328,15 @@ __device__ void tile_orders(const int *__restrict__ tile_count, int ntiles, cons
 constexpr int SB_CHUNK = 800;
 __host__ __device__ __forceinline__ int spread_chunks(int cnt) { return (cnt + SB_CHUNK - 1) / SB_CHUNK; }
 
-// Exclusive scans over the tiles, in one work group, 1024 tiles per round: the
-// bins' offsets, and the extra chunks of the tiles that k_spread_box shares
+// Exclusive scans over the tiles, in one work group, 4096 tiles per round (four
+// consecutive ones per thread; one each took 79 us for the 65536 tiles of
+// 512x256x256 nodes, this 29; the orders that follow 550 us when they were due,
+// 80 now): the bins' offsets, and the extra chunks of the tiles that k_spread_box shares
 // out (listed in `extra`, (-1, 0) behind the last); and the maximum of the
 // per-block force maxima.  Both scans ride in one 64-bit wave scan, one barrier
 // a round.  The tile orders follow in the same launch (of their own they took
 // 5 us a step, nearly always to find that they are not due).
+template <bool BINS>
 __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile_count, int *__restrict__ tile_off,
                                                     int *__restrict__ tile_cur, int ntiles,
                                                     const float *__restrict__ blk_fmax, int nblk,
@@ -331,10 +354,22 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile
     if (lane == 0) wmax[wave] = fm;
     unsigned long long carry = 0ull;  // vertices in the low half, extra chunks in the high half
     int parity = 0;
-    for (int base = 0; base < ntiles; base += 1024, parity ^= 1) {
-        const int i = base + threadIdx.x;
-        const int cnt = i < ntiles ? tile_count[i] : 0, ex = max(spread_chunks(cnt) - 1, 0);
-        const unsigned long long own = (unsigned)cnt | ((unsigned long long)ex << 32);
+    constexpr int PER = 4;
+    for (int base = 0; base < ntiles; base += 1024 * PER, parity ^= 1) {
+        const int i = base + PER * (int)threadIdx.x;
+        const bool whole = i + PER <= ntiles;
+        int cnt[PER];
+        if (whole) {  // the arrays are aligned, i is a multiple of four
+            const int4 c = *(const int4 *)(tile_count + i);
+            cnt[0] = c.x; cnt[1] = c.y; cnt[2] = c.z; cnt[3] = c.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < PER; j++) cnt[j] = i + j < ntiles ? tile_count[i + j] : 0;
+        }
+        unsigned long long own = 0ull;
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            own += (unsigned)cnt[j] | ((unsigned long long)max(spread_chunks(cnt[j]) - 1, 0) << 32);
         unsigned long long incl = own;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -344,19 +379,35 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile
         if (lane == 63) wtot[parity][wave] = incl;
         __syncthreads();
         unsigned long long b = carry + incl - own;
-#pragma unroll
+#pragma unroll 4  // all 16 would take the registers of a whole CU, and wait for a free one
         for (int w = 0; w < 16; w++) {
             const unsigned long long t = wtot[parity][w];
             if (w < wave) b += t;
             carry += t;
         }
-        if (i < ntiles) {
-            tile_off[i] = (int)(unsigned)b;
-            tile_cur[i] = 0;
-            const int e0 = (int)(b >> 32);
-            tile_ex[i] = e0;
-            for (int c = 0; c < ex; c++)
-                if (e0 + c < maxextra) extra[e0 + c] = make_int2(i, c + 1);
+        int off[PER], ex[PER];
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            off[j] = (int)(unsigned)b;
+            ex[j] = (int)(b >> 32);
+            const int n = max(spread_chunks(cnt[j]) - 1, 0);
+#pragma unroll 1
+            for (int c = 0; c < n; c++)
+                if (ex[j] + c < maxextra) extra[ex[j] + c] = make_int2(i + j, c + 1);
+            b += (unsigned)cnt[j] | ((unsigned long long)n << 32);
+        }
+        if (whole) {
+            *(int4 *)(tile_off + i) = make_int4(off[0], off[1], off[2], off[3]);
+            *(int4 *)(tile_ex + i) = make_int4(ex[0], ex[1], ex[2], ex[3]);
+            *(int4 *)(tile_cur + i) = make_int4(0, 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int j = 0; j < PER; j++)
+                if (i + j < ntiles) {
+                    tile_off[i + j] = off[j];
+                    tile_ex[i + j] = ex[j];
+                    tile_cur[i + j] = 0;
+                }
         }
     }
     for (int e = (int)(carry >> 32) + (int)threadIdx.x; e < maxextra; e += 1024) extra[e] = make_int2(-1, 0);
@@ -365,7 +416,7 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const int *__restrict__ tile
         for (int w = 1; w < 16; w++) fm = fmaxf(fm, wmax[w]);
         *absmax = __float_as_uint(fm);
     }
-    tile_orders(tile_count, ntiles, g, tg, tile_cand, order_spread, order_interp, order_calls);
+    tile_orders<BINS>(tile_count, ntiles, g, tg, tile_cand, order_spread, order_interp, order_calls);
 }
 
 // Spreading data of a vertex, stored in bin order next to its first stencil
@@ -2085,7 +2136,7 @@ BinGeom bin_geom(const lbmibm_ctx *ctx) {
 lbmibm_status tile_offsets(lbmibm_ctx *ctx, hipStream_t stream, int nblk_fmax) {
     const IbmGeom g = geom_of(ctx);
     const TileGeom tg = tiles_of(ctx);
-    hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->tile_off, ctx->tile_cur,
+    hipLaunchKernelGGL((ctx->spread_form == 0 ? k_tile_scan<true> : k_tile_scan<false>), dim3(1), dim3(1024), 0, stream, ctx->tile_count, ctx->tile_off, ctx->tile_cur,
                        ctx->ntiles, ctx->blk_fmax, nblk_fmax, ctx->absmax, ctx->tile_ex, ctx->sb_extra,
                        ctx->sb_maxextra, g, tg, ctx->tile_cand, ctx->order_spread, ctx->order_interp,
                        ctx->order_calls);

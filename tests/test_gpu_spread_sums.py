@@ -133,3 +133,44 @@ def test_home_boxes_do_not_depend_on_the_order_of_the_binning(k, prec, monkeypat
         assert np.array_equal(F, first)
     g.close()
     assert np.abs(first).max() > 0.0
+
+
+@pytest.mark.parametrize("form", [0, 1])
+def test_more_tiles_than_the_scan_takes_at_once(form, monkeypatch):
+    """4913 tiles, 4096 at a time and four per thread, an odd number of them: full
+    tiles on both sides of the border and in the last rows, nearly all others empty."""
+    monkeypatch.setenv("LBMIBM_SPREAD_FORM", str(form))
+    shape = (135, 135, 129)
+    print(f"[many tiles] form={form}", flush=True)
+    from preprocess_src_amd import mesh
+    cells = mesh.assemble([4, 4, 4, 3], np.zeros((4, 3)), np.repeat(np.eye(3)[None], 4, 0), 3.0)
+    rng = np.random.default_rng(8)
+    n = cells["x"].size
+    at = rng.uniform(0.0, 1.0, (n, 3)) * 7.0
+    per = np.repeat(np.arange(4), np.diff(cells["voff"]))
+    # tiles 4095 and 4096 (x = 15 and 16, y = 2, z = 14), the last rows, anywhere
+    corner = np.array([[121.0, 17.0, 113.0], [129.0, 17.0, 113.0], [128.0, 128.0, 121.0]])
+    at[per < 3] += corner[per[per < 3]]
+    at[per == 3] = rng.uniform(0.0, 1.0, ((per == 3).sum(), 3)) * (np.array(shape) - 1.0)
+    forces = [1e-3 * rng.standard_normal(n) for _ in range(3)]
+    pos = [at[:, d] - (shape[d] - 1) / 2.0 for d in range(3)]
+    g = gpu_of(*shape, "f64", cells=cells)
+    g.set_cells_state(x=pos[0], y=pos[1], z=pos[2], fx=forces[0], fy=forces[1], fz=forces[2])
+    g.ibm_st1()
+    F = [f.reshape([v + 4 for v in shape[::-1]])[2:-2, 2:-2, 2:-2] for f in g.lattice_force()]
+    g.close()
+    first = np.floor(at)
+    t = np.pi / 2 * (at - first)
+    w = np.stack([1 - np.sin(t), 1 + np.cos(t), 1 + np.sin(t), 1 - np.cos(t)], 2) / 4.0
+    i = first.astype(int)[:, :, None] - 1 + np.arange(4)
+    want = np.zeros((3,) + shape[::-1])
+    for a in range(4):
+        for b in range(4):
+            for c in range(4):
+                ok = (i[:, 1, b] >= 0) & (i[:, 1, b] < shape[1])
+                q = w[:, 0, a] * w[:, 1, b] * w[:, 2, c] * ok
+                idx = (i[:, 2, c] % shape[2], np.clip(i[:, 1, b], 0, shape[1] - 1), i[:, 0, a] % shape[0])
+                for d in range(3):
+                    np.add.at(want[d], idx, q * forces[d])
+    for d in range(3):  # FP64 sums of at most a few thousand terms, as the other spreading tests
+        assert np.max(np.abs(F[d] - want[d])) < 1e-11 * np.max(np.abs(want[d]))
