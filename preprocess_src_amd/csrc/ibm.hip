@@ -734,15 +734,17 @@ template <typename T> constexpr int SB_SPAN = sizeof(T) == 4 ? 32 : 16;
 static_assert(SB_CAP > SB_CHUNK, "the sort takes a chunk and a spread about it");
 typedef double double_x4 __attribute__((ext_vector_type(4)));
 
-// The fixed-point sums of one chunk of a tile that is shared out, and their
-// scale: a power of two, or infinity where the chunk's forces are all 0 (and 0
+// The fixed-point sums of one chunk of a tile that is shared out.  Their scales
+// follow behind the boxes: a power of two, or infinity where the chunk's forces are all 0 (and 0
 // where one is infinite, which gives a tile without finite sums).  The boxes of the
 // extra chunks first, at the number of the chunk; behind them those of the
 // first chunks, at the number of the tile's first extra chunk.
 struct ChunkBox {
     long long v[3 * SB_N];
-    double scale;
 };
+__device__ __forceinline__ double *chunk_scales(ChunkBox *chunks, int maxextra) {
+    return (double *)(chunks + 2 * (size_t)maxextra);
+}
 
 template <typename T>
 __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_spread_box(const SpreadRec<T> *__restrict__ rec,
@@ -1061,7 +1063,8 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
     }
     const double inv_scale = 1.0 / scale;
     T *St = S + (size_t)tile * 3 * SB_N;
-    ChunkBox *box = chunks + (nch == 1 ? 0 : chunk > 0 ? (int)blockIdx.x : maxextra + ex0);
+    const int slot = chunk > 0 ? (int)blockIdx.x : maxextra + ex0;
+    ChunkBox *box = chunks + (nch == 1 ? 0 : slot);
     for (int k0 = tid; k0 < 3 * SB_N; k0 += 4 * WG_) {  // four reads, then four stores
         unsigned long long a[4];
 #pragma unroll
@@ -1074,7 +1077,7 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
             else St[k] = (T)FixedPoint<T>::real(a[j], inv_scale);
         }
     }
-    if (nch > 1 && tid == 0) box->scale = fmax > 0.0 ? scale : HUGE_VAL;
+    if (nch > 1 && tid == 0) chunk_scales(chunks, maxextra)[slot] = fmax > 0.0 ? scale : HUGE_VAL;
 }
 
 // Adds the chunks' boxes of each tile that was shared out into the tile's box:
@@ -1083,15 +1086,17 @@ __global__ __launch_bounds__(SPREAD_BOX_WG, sizeof(T) == 4 ? 6 : 4) void k_sprea
 // scales, which is the one that all of the tile's vertices in one work group would
 // have had, and rounded to T at the end; boxes rounded to FP32 and added in FP32
 // lost up to 2.8 times as much where the chunks' sums cancel.  That costs twice
-// the bytes: 64 cells 5.8 -> 7.1 us here and 33.4 -> 34.1 in k_spread_box, the
-// 1024-cell suspension 13.3 -> 18.6 and 198 -> 205.  The boxes are read once: past
-// the caches, or they would drive out those that the gather reads next (62 instead
-// of 55 us).  The gather adding the chunks itself took 64 instead of 44 us: the
+// the bytes: 64 cells 33.4 -> 34.1 us in k_spread_box (and 5.2 here), the 1024-cell
+// suspension 199 -> 206 (and 15.8 here).  What bounds this is the chain of loads: the
+// first two boxes' beside that of their number, then four boxes at a time; one
+// after another took 7.9 and 20.5, and 78 instead of 19 where 82000 vertices lie in a
+// few tiles.  The boxes are read once: past the caches, or they would drive out
+// those that the gather reads next (62 instead of 55 us).  The gather adding the chunks itself took 64 instead of 44 us: the
 // loop over them keeps its loads from being issued together.
 constexpr int COMBINE_WG = 256, COMBINE_PER = 4;  // threads and values of each; blockIdx.y: stretch of the box
 constexpr int COMBINE_PARTS = (3 * SB_N + COMBINE_WG * COMBINE_PER - 1) / (COMBINE_WG * COMBINE_PER);
 template <typename T>
-__global__ __launch_bounds__(COMBINE_WG) void k_spread_combine(T *__restrict__ S, const ChunkBox *__restrict__ chunks,
+__global__ __launch_bounds__(COMBINE_WG) void k_spread_combine(T *__restrict__ S, ChunkBox *__restrict__ chunks,
                                                          const int2 *__restrict__ extra,
                                                          const int *__restrict__ tile_count, int maxextra) {
     const int2 ex = extra[blockIdx.x];
@@ -1110,20 +1115,30 @@ __global__ __launch_bounds__(COMBINE_WG) void k_spread_combine(T *__restrict__ S
         sum[j] = 0;
     }
     const int nx = spread_chunks(tile_count[ex.x]) - 1;
-    double scale = fmin(first->scale, more[0].scale);  // the coarsest
-    for (int c = 1; c < nx; c++) scale = fmin(scale, more[c].scale);
+    const double *scales = chunk_scales(chunks, maxextra), *ms = scales + blockIdx.x;
+    const double s0 = scales[maxextra + blockIdx.x];
+    double scale = fmin(s0, ms[0]);  // the coarsest
+    for (int c = 1; c < nx; c++) scale = fmin(scale, ms[c]);
     const int e = ilogb(scale);
-    for (int c = 0; c <= nx; c++) {  // the next but one box's values while these are added
-        const double t = c == 0 ? first->scale : more[c - 1].scale;
+    auto add = [&](const long long (&w)[PER], double t) {
         // at most 62: a chunk without forces, at infinity, holds zeros
         const int sh = scale > 0.0 ? (int)min((long long)ilogb(t) - e, 62ll) : 0;
         const long long half = sh > 0 ? 1ll << (sh - 1) : 0;
 #pragma unroll
-        for (int j = 0; j < PER; j++) {
-            sum[j] += (v[j] + half) >> sh;
-            v[j] = next[j];
-            if (c + 1 < nx) next[j] = __builtin_nontemporal_load(&more[c + 1].v[k[j]]);
-        }
+        for (int j = 0; j < PER; j++) sum[j] += (w[j] + half) >> sh;
+    };
+    add(v, s0);
+    add(next, ms[0]);
+    constexpr int AHEAD = 4;  // boxes read at a time
+    for (int c0 = 1; c0 < nx; c0 += AHEAD) {
+        long long w[AHEAD][PER];
+#pragma unroll
+        for (int a = 0; a < AHEAD; a++)
+#pragma unroll
+            for (int j = 0; j < PER; j++) w[a][j] = __builtin_nontemporal_load(&more[min(c0 + a, nx - 1)].v[k[j]]);
+#pragma unroll
+        for (int a = 0; a < AHEAD; a++)
+            if (c0 + a < nx) add(w[a], ms[c0 + a]);
     }
     const double inv = 1.0 / scale;
     T *own = S + (size_t)ex.x * 3 * SB_N;
@@ -2198,7 +2213,7 @@ template <typename T> lbmibm_status spread_launch(lbmibm_ctx *ctx, int form) {
                 LBMIBM_KT(ctx, ctx->stream, "k_spread_combine",
                           hipLaunchKernelGGL(k_spread_combine<T>, dim3(ctx->sb_maxextra, COMBINE_PARTS),
                                              dim3(COMBINE_WG), 0, ctx->stream, (T *)ctx->sbox,
-                                             (const ChunkBox *)ctx->sb_chunks, ctx->sb_extra, ctx->tile_count,
+                                             (ChunkBox *)ctx->sb_chunks, ctx->sb_extra, ctx->tile_count,
                                              ctx->sb_maxextra));
                 LBMIBM_LAUNCHED(ctx, "k_spread_combine");
             }
@@ -2467,7 +2482,7 @@ static lbmibm_status spread_box_setup(lbmibm_ctx *ctx, bool *ok) {
     if (!ctx->sbox) {
         lbmibm_status s = dev_alloc(ctx, &ctx->sbox, (size_t)ctx->ntiles * 3 * (ctx->pointwise ? SP_N : SB_N) * ctx->szT);
         if (s == LBMIBM_OK && ctx->sb_maxextra > 0)
-            s = dev_alloc(ctx, &ctx->sb_chunks, 2 * (size_t)ctx->sb_maxextra * sizeof(ChunkBox));
+            s = dev_alloc(ctx, &ctx->sb_chunks, 2 * (size_t)ctx->sb_maxextra * (sizeof(ChunkBox) + sizeof(double)));
         if (s != LBMIBM_OK) return s;
     }
     *ok = true;
